@@ -64,7 +64,10 @@ enum pm_coeff_kind {
   PM_COEFF_CB = 1,
   /* as PM_COEFF_CB with cb[3] stored as FP16 holding Cb / cb_scale;
    * FP32 fields only */
-  PM_COEFF_CB_F16 = 2
+  PM_COEFF_CB_F16 = 2,
+  /* conductive, non-magnetic media (sigma_m = 0, mu_r = 1, so Da = 1 exactly
+   * and Db = db_const): ca[3] and cb[3] in field precision; yee scheme */
+  PM_COEFF_CACB = 3
 };
 
 /* Additive source term: field[c] += value for every cell c of the box, after
@@ -144,7 +147,7 @@ typedef struct pm_plan {
   const void* da[3];
   const void* db[3];
   double cb_scale;                /* PM_COEFF_CB_F16: Cb = cb_scale * cb[c] */
-  double db_const;                /* PM_COEFF_CB_F16: uniform Db */
+  double db_const;                /* every kind but PM_COEFF_FULL: uniform Db */
 
   /* CPML (yee only).  Thickness per face x-,x+,y-,y+,z-,z+ in cells.
    * Profiles per axis a (length n_a): *_e at half nodes (E-update terms),
@@ -187,9 +190,10 @@ typedef struct pm_plan {
    * (gating flags and the device copy of the ADE box table) */
   void* scratch;
 
-  /* Optional second buffer set for the fused step (yee; 3-D with padded
-   * row sy in {128, 256, 512}, or 2-D TM without dispersive boxes or full
-   * coefficient arrays).  With E2/H2 and
+  /* Optional second buffer set for the fused step (yee; 3-D with a padded
+   * row sy that is a multiple of 64 (with full coefficient arrays: 128, 256
+   * or 512), or 2-D TM without dispersive boxes and with Cb-only
+   * coefficients).  With E2/H2 and
    * psi_h2 (for every psi_h given) present, pm_run advances steps with one
    * fused H+E kernel that reads one set and writes the other; a run with an
    * odd step count does its first step in place, so every call returns with
@@ -284,8 +288,9 @@ int pm_dft_flush(pm_ctx* ctx, int64_t step_first, int32_t rows);
  * the unfused kernels, fuse = 2 asks for two steps per launch (temporal
  * blocking; ty must be 4 and vec 0; runs that sample monitors or add
  * sources with a per-cell profile, and the one to three steps of a run that
- * do not fill pairs of passes, take the one-step kernel).  Defaults: 1, 4,
- * 8, 0, 2.  Used by the autotuner. */
+ * do not fill pairs of passes, take the one-step kernel).  Until it is
+ * called, rows, planes and order follow rules on the grid's size and
+ * precision.  Used by the autotuner. */
 int pm_set_tuning(pm_ctx* ctx, int fuse, int ty, int kchunk, int vec, int order);
 
 /* Rows of the fused one-step kernel in workgroups of a whole padded row
@@ -293,8 +298,11 @@ int pm_set_tuning(pm_ctx* ctx, int fuse, int ty, int kchunk, int vec, int order)
  * recomputes H of the cell to its right; plans with Cb-only coefficients
  * whose middle cell lies outside the x CPML layers); 0 (default) = whole
  * rows when a launch shape fits them, else two segments (FP64 512-cell
- * rows).  The results do not depend on it.  pm_row_split_active: segments
- * the next fused step takes (0 when it is not fused).  Used by the
+ * rows), and segments of 64 cells for FP32 512-cell rows (with vec 0) and
+ * for rows of any other width or with Ca and Cb arrays, which take these
+ * whatever is asked for (ty 3 or 7, vec unused).  The results do not depend
+ * on it.  pm_row_split_active: segments the next fused step takes (0 when it
+ * is not fused).  Used by the
  * autotuner; no counterpart in the reference. */
 int pm_set_row_split(pm_ctx* ctx, int segments);
 int pm_row_split_active(pm_ctx* ctx);

@@ -20,7 +20,7 @@ PM_EX, PM_EY, PM_EZ, PM_HX, PM_HY, PM_HZ = range(6)
 COMP_ID = {"Ex": 0, "Ey": 1, "Ez": 2, "Hx": 3, "Hy": 4, "Hz": 5}
 SCHEME_COMPAT, SCHEME_YEE = 0, 1
 FP64, FP32 = 0, 1
-COEFF_FULL, COEFF_CB, COEFF_CB_F16 = 0, 1, 2
+COEFF_FULL, COEFF_CB, COEFF_CB_F16, COEFF_CACB = 0, 1, 2, 3
 RUN_SOURCES, RUN_SAMPLE, RUN_DFT, RUN_GRAPH, RUN_IO_ONLY = 1, 2, 4, 8, 16
 
 ERRORS = {

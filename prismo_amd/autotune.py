@@ -101,12 +101,16 @@ def tune(eng, steps: int = 6, warmup: int = 2, candidates: dict | None = None,
         return dict(best, fused=True, cached=True)
     cand = candidates or CANDIDATES
     splits = cand.get("xs", (1, 2))
+    # rows in segments of 64 cells (FP32 rows of 512 cells, every width
+    # without a whole-row shape): the automatic choice, tile heights 3 and 7
+    seg = [(1, 0, ty, kc, order, 0) for ty, kc, order in
+           product((3, 7), cand["kchunk"], cand["order"])]
     if getattr(eng, "is_2d", False):
         # the 2-D pass: rows per tile (kchunk) only
         shapes = [(1, 0, 2, kc, 2, 1) for kc in cand.get("rows_2d", CANDIDATES_2D)]
     else:
         shapes = [(1, vec, ty, kc, order, xs) for xs, vec, ty, kc, order in
-                  product(splits, cand["vec"], cand["ty"], cand["kchunk"], cand["order"])]
+                  product(splits, cand["vec"], cand["ty"], cand["kchunk"], cand["order"])] + seg
     if not getattr(eng, "is_2d", False) and (candidates is None or "two_step" in candidates):
         c2 = (candidates or {}).get("two_step", CANDIDATES2)
         shapes += [(2, 0, 4, kc, order, 1) for kc, order in product(c2["kchunk"], c2["order"])]
@@ -126,7 +130,7 @@ def tune(eng, steps: int = 6, warmup: int = 2, candidates: dict | None = None,
                     shape = eng.ctx.fused_shape()
                     rows = kc if getattr(eng, "is_2d", False) else ty
                     if shape is None or (vec and shape[0] != vec) or shape[2] != rows \
-                            or shape[3] != xs or (shape, kc, order) in seen:
+                            or (xs and shape[3] != xs) or (shape, kc, order) in seen:
                         continue
                     seen.add((shape, kc, order))
                 # whole pairs of passes (4 steps) keep the two-step path on

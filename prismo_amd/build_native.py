@@ -41,6 +41,8 @@ UNITS = {
     "geom.hip": ["-ffp-contract=off"],
     "fused_f32.hip": [],
     "fused_f64.hip": [],
+    "fused_seg_f32.hip": [],
+    "fused_seg_f64.hip": [],
     "tm2d.hip": [],
 }
 

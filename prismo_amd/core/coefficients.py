@@ -81,6 +81,11 @@ def _all_equal(a, v) -> bool:
     return bool(np.all(a == v))
 
 
+def is_nonmagnetic(mu_rel, sigma_m) -> bool:
+    """True when Da = 1 exactly and Db is one constant."""
+    return _all_equal(sigma_m, 0) and _all_equal(mu_rel, 1)
+
+
 def is_lossless_nonmagnetic(mu_rel, sigma_e, sigma_m) -> bool:
     """True when Ca = Da = 1 exactly and Db is one constant."""
     return _all_equal(sigma_e, 0) and _all_equal(sigma_m, 0) and _all_equal(mu_rel, 1)

@@ -16,7 +16,8 @@ from typing import Optional
 import numpy as np
 
 from .. import _native as N
-from .coefficients import cell_coefficients, component_average, is_lossless_nonmagnetic
+from .coefficients import (cell_coefficients, component_average, is_lossless_nonmagnetic,
+                           is_nonmagnetic)
 from .grid import COMPONENTS
 
 EPS0 = 8.854187817e-12
@@ -83,7 +84,7 @@ class StepEngine:
         self._bindings: dict = {}
         self.plan = N.pm_plan()
         self._fill_grid()
-        self._make_arena(cpml)
+        self._make_arena(cpml, ca=len(coeffs) == 7 and self._stores_ca(coeffs, coefficient_storage))
         self._fill_coefficients(coeffs, coefficient_storage)
         self._fill_cpml(cpml)
         self._fill_ade(list(ade))
@@ -105,14 +106,21 @@ class StepEngine:
         self._keep.append(t)
         return t
 
-    def _make_arena(self, cpml):
+    def _stores_ca(self, coeffs, storage) -> bool:
+        """Conductive, non-magnetic media in the textbook scheme: Ca and Cb
+        arrays (Da = 1 and Db is one constant)."""
+        return (storage in ("auto", "native") and self.scheme == "yee"
+                and is_nonmagnetic(coeffs[4], coeffs[6])
+                and not is_lossless_nonmagnetic(coeffs[4], coeffs[5], coeffs[6]))
+
+    def _make_arena(self, cpml, ca: bool = False):
         """One zeroed allocation for the coefficient, CPML memory and profile
         arrays, so they sit within a few hundred MB of each other: the fused
         kernel addresses them with 32-bit offsets from one base."""
         nx, ny, nz = self.grid.dimensions
         esz = 8 if self.precision == N.FP64 else 4
         field = nz * ny * self.sy * esz
-        total = 3 * field + 6 * (nx + ny + nz) * esz + 4096
+        total = (6 if ca else 3) * field + 6 * (nx + ny + nz) * esz + 4096
         if cpml is not None:
             cells = nx * ny * nz
             for a, n in enumerate((nx, ny, nz)):
@@ -199,7 +207,8 @@ class StepEngine:
                 raise ValueError("FP16 coefficients need lossless media, FP32 fields, 'yee'")
             kind = N.COEFF_CB_F16
         elif storage in ("auto", "native"):
-            kind = N.COEFF_CB if lossless else N.COEFF_FULL
+            kind = (N.COEFF_CB if lossless else
+                    N.COEFF_CACB if self._stores_ca(coeffs, storage) else N.COEFF_FULL)
         elif storage == "full":
             kind = N.COEFF_FULL
         else:
@@ -212,7 +221,7 @@ class StepEngine:
         if kind != N.COEFF_FULL:
             d0 = float(np.asarray(Db).flat[0])
             if not np.all(Db == d0):
-                raise ValueError("uniform Db expected for lossless non-magnetic media")
+                raise ValueError("uniform Db expected for non-magnetic media")
             p.db_const = d0
         self.cb_host = {}
         self.cb_dev = {}
@@ -220,6 +229,8 @@ class StepEngine:
         cb_dt = torch.float16 if kind == N.COEFF_CB_F16 else self.tdtype
         # the three Cb arrays back to back (the fused kernel's layout)
         cb_all = None if self.is_2d else self._carve((3, nz, ny, self.sy), cb_dt)
+        ca_all = (self._carve((3, nz, ny, self.sy), self.tdtype)
+                  if kind == N.COEFF_CACB and not self.is_2d else None)
         for a, c in enumerate(("Ex", "Ey", "Ez")):
             if c not in self.need_e:
                 continue
@@ -233,9 +244,9 @@ class StepEngine:
                 self.cb_host[c] = cb
                 self.cb_dev[c] = self._padded(cb, c, self.tdtype, dst)
             p.cb[a] = self.cb_dev[c].data_ptr()
-            if kind == N.COEFF_FULL:
-                p.ca[a] = self._padded(component_average(sl(Ca), c, self.is_2d), c,
-                                       self.tdtype).data_ptr()
+            if kind in (N.COEFF_FULL, N.COEFF_CACB):
+                p.ca[a] = self._padded(component_average(sl(Ca), c, self.is_2d), c, self.tdtype,
+                                       None if ca_all is None else ca_all[a]).data_ptr()
         if kind == N.COEFF_FULL:
             for a, c in enumerate(("Hx", "Hy", "Hz")):
                 if c not in self.need_h:
@@ -300,7 +311,7 @@ class StepEngine:
         """(Cb, Db) in FP64 at the cells of ``box`` ((i0, i1), (j0, j1),
         (k0, k1)) of E component ``comp`` and of the matching H points, read
         back from the device arrays (lossless media: Db is one constant)."""
-        if self.coeff_kind == N.COEFF_FULL:
+        if self.coeff_kind in (N.COEFF_FULL, N.COEFF_CACB):
             raise NotImplementedError("coefficients of lossy or magnetic media")
         (i0, i1), (j0, j1), (k0, k1) = box
         t = self.cb_dev[comp][k0:k1, j0:j1, i0:i1].permute(2, 1, 0).double().cpu().numpy()
@@ -349,8 +360,9 @@ class StepEngine:
                             side[a][q] = self._alloc(shape, self.tdtype).data_ptr()
 
     def _fill_fused(self, fused: bool):
-        """Second buffer set for the fused ping-pong step (3-D yee, one x-row
-        per wave64: pitch / 64 in {2, 4, 8}; 2-D TM yee: Ez, Hx, Hy)."""
+        """Second buffer set for the fused ping-pong step (3-D yee; with full
+        coefficient arrays only rows of 128, 256 or 512 cells; 2-D TM yee:
+        Ez, Hx, Hy)."""
         p = self.plan
         self.fused = False
         if not fused or self.scheme != "yee":
@@ -358,9 +370,14 @@ class StepEngine:
         if self.is_2d:
             self._fill_fused_2d()
             return
-        if self.sy not in (128, 256, 512):
+        if self.sy % 64 or (p.coeff_kind == N.COEFF_FULL and self.sy not in (128, 256, 512)):
             return
         nx, ny, nz = self.grid.dimensions
+        # the kernel addresses a field set with 32-bit offsets: a larger one
+        # would never be used
+        esz = 8 if self.precision == N.FP64 else 4
+        if self.sy not in (128, 256, 512) and 6 * nz * ny * self.sy * esz >= 1 << 32:
+            return
         # second field set: Ex Ey Ez Hx Hy Hz back to back at the stride of
         # the first set (ElectromagneticFields allocates it the same way)
         setb = self._alloc((6, nz, ny, self.sy), self.tdtype)
@@ -370,7 +387,9 @@ class StepEngine:
         for a in range(3):
             S = p.pml[2 * a] + p.pml[2 * a + 1]
             shape = {0: (nz, ny, S), 1: (nz, S, nx), 2: (S, ny, nx)}[a]
-            for src, dst in ((p.psi_h, p.psi_h2), (p.psi_e, p.psi_e2)):
+            # the second E-side memory serves two steps per launch only
+            for src, dst in (((p.psi_h, p.psi_h2), (p.psi_e, p.psi_e2))
+                             if self.sy in (128, 256) else ((p.psi_h, p.psi_h2),)):
                 if src[a][0] and src[a][1]:
                     pair = self._carve((2,) + shape, self.tdtype)
                     for q in range(2):
@@ -387,7 +406,7 @@ class StepEngine:
         Hy and second H-side CPML memory (Hy in the x slabs, Hx in the y
         slabs); lossy media and dispersive boxes keep the unfused kernels."""
         p = self.plan
-        if p.n_ade or p.coeff_kind == N.COEFF_FULL:
+        if p.n_ade or p.coeff_kind in (N.COEFF_FULL, N.COEFF_CACB):
             return
         nx, ny, _ = self.grid.dimensions
         setb = self._alloc((3, 1, ny, self.sy), self.tdtype)

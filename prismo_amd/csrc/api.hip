@@ -2,6 +2,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -31,7 +32,8 @@ struct pm_ctx {
   // tuning (0 auto, 1 whole rows, 2 two segments)
   bool split_ok = false;
   int tune_xs = 0;
-  bool kchunk_set = false;  // pm_set_tuning was called (the 2-D pass's rows)
+  bool kchunk_set = false;  // pm_set_tuning was called (else the rules below pick)
+  int n_cu = 256;           // compute units of the device
   // 2-D compat gate flags: the set the next H update fills (0 / 1) and the
   // set the E update of the current step reads
   int flag_set = 0, flag_set_e = 0;
@@ -212,7 +214,7 @@ int validate(pm_ctx* c, const pm_plan& p) {
     return fail(c, PM_EINVAL, "spacings and dt must be positive");
   if (p.precision != PM_FP64 && p.precision != PM_FP32)
     return fail(c, PM_EINVAL, "unknown precision %d", p.precision);
-  if (p.coeff_kind < PM_COEFF_FULL || p.coeff_kind > PM_COEFF_CB_F16)
+  if (p.coeff_kind < PM_COEFF_FULL || p.coeff_kind > PM_COEFF_CACB)
     return fail(c, PM_EINVAL, "unknown coeff_kind %d", p.coeff_kind);
   if (p.coeff_kind == PM_COEFF_CB_F16 && p.precision != PM_FP32)
     return fail(c, PM_ENOTSUP, "FP16 coefficients need FP32 fields");
@@ -224,6 +226,8 @@ int validate(pm_ctx* c, const pm_plan& p) {
       return fail(c, PM_ENOTSUP, "compat scheme is FP64 only");
     if (p.coeff_kind == PM_COEFF_CB_F16)
       return fail(c, PM_ENOTSUP, "compat scheme needs FP64 coefficients");
+    if (p.coeff_kind == PM_COEFF_CACB)
+      return fail(c, PM_ENOTSUP, "compat scheme takes full or Cb-only coefficients");
     for (int a = 0; a < 6; ++a)
       if (p.pml[a]) return fail(c, PM_ENOTSUP, "compat scheme has no CPML");
     if (p.n_ade) return fail(c, PM_ENOTSUP, "compat scheme has no ADE");
@@ -240,8 +244,9 @@ int validate(pm_ctx* c, const pm_plan& p) {
     if (needE[a] && !p.E[a]) return fail(c, PM_EINVAL, "E[%d] is NULL", a);
     if (needH[a] && !p.H[a]) return fail(c, PM_EINVAL, "H[%d] is NULL", a);
     if (needE[a] && !p.cb[a]) return fail(c, PM_EINVAL, "cb[%d] is NULL", a);
+    if ((p.coeff_kind == PM_COEFF_FULL || p.coeff_kind == PM_COEFF_CACB) && needE[a] && !p.ca[a])
+      return fail(c, PM_EINVAL, "ca[%d] is NULL", a);
     if (p.coeff_kind == PM_COEFF_FULL) {
-      if (needE[a] && !p.ca[a]) return fail(c, PM_EINVAL, "ca[%d] is NULL", a);
       if (needH[a] && (!p.da[a] || !p.db[a]))
         return fail(c, PM_EINVAL, "da/db[%d] is NULL", a);
     }
@@ -370,6 +375,63 @@ int do_e(pm_ctx* c) {
 // 11.5 us, the unfused H and E launches in 8.3 us.
 int rows2d(const pm_ctx* c) { return c->kchunk_set ? std::max(1, c->tune_kchunk) : 3; }
 
+// Rows the fused step takes in segments of 64 cells (fused_seg.h): those of
+// a width without whole-row or two-segment shapes, media with Ca and Cb
+// arrays, and, unless a split or a vector width is asked for, FP32 rows of
+// 512 cells (480 x 240 x 160 dispersive: 338 us a step in segments, 361 in two
+// halves, 425 whole; 500 x 60 x 40: 31.1, 33.0, over 37).  Whole rows of 128
+// and 256 cells are faster than their segments (256^3 FP32/FP16 Cb 224 and
+// 237 us, FP64 539 and 549; 128^3 37.3 and 42.6).
+bool seg_row(const pm_ctx* c) {
+  const pm_plan& p = c->plan;
+  if (p.ndim != 3 || p.sy % 64 || !seg_supported(p.coeff_kind, 7)) return false;
+  if (p.sy == 512 && p.precision == PM_FP32 && c->tune_xs == 0 && c->tune_vec == 0) return true;
+  return p.coeff_kind == PM_COEFF_CACB || (p.sy != 128 && p.sy != 256 && p.sy != 512);
+}
+// Rows per workgroup of the segments: FP64 holds 8 waves on a CU (about 190
+// VGPRs), and two workgroups of 4 waves cover each other's barriers where one
+// of 8 does not (180 x 140 x 120: 125 us a step, 131 with 7 rows); FP32 holds
+// 16, where 7 rows re-read fewer halo rows (301 x 187 x 149: 141 and 147).
+int seg_rows(const pm_ctx* c) {
+  if (c->kchunk_set) return c->tune_ty == 3 ? 3 : 7;
+  return c->plan.precision == PM_FP64 ? 3 : 7;
+}
+
+// Rows per workgroup of the whole-row shapes when none was asked for.
+int whole_rows(const pm_ctx* c) {
+  if (c->kchunk_set || c->plan.coeff_kind == PM_COEFF_FULL) return c->tune_ty;
+  return c->plan.precision == PM_FP64 ? 4 : 3;
+}
+
+// Planes per workgroup when none were asked for.  A workgroup of kc planes
+// steps kc + 1 of them (the H halo plane) after about two planes' worth of
+// start-up, so long chunks waste less; short ones fill the chip and shorten
+// the last wave of workgroups.  The rule counts rounds of workgroups over the
+// slots the registers leave (rounds under 3 in whole numbers, more of them
+// overlap) times planes per workgroup, over chunks of at most 12 planes (16 in
+// FP64), beyond which the caches lose the planes that neighbouring tiles share.
+// 64^3: 2 planes 9.9 us, 4 12.7, 8 19.6; 160 x 128 x 96: 12 planes 44.8,
+// 8 49.9, 16 52.9; 256^3: 10 planes 224, 12 226, 8 225, 16 227.
+int auto_planes(const pm_ctx* c, int w, int ty, int xs) {
+  const pm_plan& p = c->plan;
+  const bool f64 = p.precision == PM_FP64;
+  const int waves = w * (ty + 1);
+  const double slots = (double)c->n_cu * std::max(1, (f64 ? 8 : 16) / waves);
+  const double cols = (double)((p.ny + ty - 1) / ty) * xs;
+  int best = 1;
+  double best_cost = 0;
+  for (int kc = 1; kc <= std::min((int)p.nz, f64 ? 16 : 12); ++kc) {
+    const double r = cols * ((p.nz + kc - 1) / kc) / slots;
+    const double rounds = r < 3 ? std::ceil(r) : r + 0.5;
+    const double cost = rounds * (kc + 3);
+    if (kc == 1 || cost < best_cost) {
+      best = kc;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // Rows in xs segments (pm_set_row_split: 1 or 2; 0 = whole rows when a
 // shape fits them, else two segments).
 bool fused_shape(const pm_ctx* c, int* vec, int* w, int* ty, int* xs) {
@@ -384,6 +446,13 @@ bool fused_shape(const pm_ctx* c, int* vec, int* w, int* ty, int* xs) {
     return true;
   }
   const int prec = c->plan.precision, ck = c->plan.coeff_kind;
+  if (seg_row(c)) {
+    *vec = 1;
+    *w = 1;
+    *ty = seg_rows(c);
+    *xs = sy / 64;
+    return true;
+  }
   int opts[2] = {1, 2}, nopt = 2;
   if (c->tune_xs == 1 || c->tune_xs == 2) {
     opts[0] = c->tune_xs;
@@ -394,13 +463,18 @@ bool fused_shape(const pm_ctx* c, int* vec, int* w, int* ty, int* xs) {
     if (x == 2 && !c->split_ok) continue;
     const int rw = sy / x;  // cells per segment
     int prefer = c->tune_vec;
-    if (prefer <= 0) prefer = prec == PM_FP32 ? (rw >= 128 && x == 1 ? 2 : 1) : (rw <= 256 ? 1 : 2);
+    // one cell per lane where a workgroup of 16 waves then holds 3 rows
+    // (256^3 FP32: 226 us a step, 267 with two cells per lane and 4 rows)
+    if (prefer <= 0)
+      prefer = prec == PM_FP32 && (c->kchunk_set || ck == PM_COEFF_FULL)
+                   ? (rw >= 128 && x == 1 ? 2 : 1)
+                   : (rw <= 256 ? 1 : 2);
     const int vecs[4] = {prefer, 1, 2, 4};
     const int nv = c->tune_vec > 0 ? 1 : 4;
     for (int iv = 0; iv < nv; ++iv) {
       const int v = vecs[iv];
       if (rw % (64 * v)) continue;
-      for (int t : {c->tune_ty, 2}) {
+      for (int t : {whole_rows(c), 2}) {
         if (fused_supported(prec, ck, v, rw / (64 * v), t, x)) {
           *vec = v;
           *w = rw / (64 * v);
@@ -472,11 +546,18 @@ int do_fused(pm_ctx* c) {
   }
   int vec, w, ty, xs;
   fused_shape(c, &vec, &w, &ty, &xs);
-  const int r = p.precision == PM_FP32
-                    ? launch_yee_fused_f32(c->g, p.coeff_kind, fb, vec, w, ty,
-                                           c->tune_kchunk, c->tune_order, xs, c->stream)
-                    : launch_yee_fused_f64(c->g, p.coeff_kind, fb, vec, w, ty,
-                                           c->tune_kchunk, c->tune_order, xs, c->stream);
+  // tile order 3 unless tuned: neighbouring tiles on one XCD share halo rows
+  // in its L2 (301 x 187 x 149: 141 us, round-robin 147)
+  const int kc = c->kchunk_set ? c->tune_kchunk : auto_planes(c, w, ty, xs);
+  const int order = c->kchunk_set ? c->tune_order : 3;
+  const bool f32 = p.precision == PM_FP32;
+  int r;
+  if (seg_row(c))
+    r = f32 ? launch_yee_seg_f32(c->g, p.coeff_kind, fb, ty, kc, order, c->stream)
+            : launch_yee_seg_f64(c->g, p.coeff_kind, fb, ty, kc, order, c->stream);
+  else
+    r = f32 ? launch_yee_fused_f32(c->g, p.coeff_kind, fb, vec, w, ty, kc, order, xs, c->stream)
+            : launch_yee_fused_f64(c->g, p.coeff_kind, fb, vec, w, ty, kc, order, xs, c->stream);
   if (r != 0)
     return fail(c, PM_ENOTSUP, "fused step: no kernel for vec %d, w %d, ty %d, %d segments",
                 vec, w, ty, xs);
@@ -573,7 +654,8 @@ bool fused2d_eligible(const pm_plan& p) {
 bool fused_eligible(const pm_plan& p) {
   if (p.ndim == 2) return fused2d_eligible(p);
   if (p.scheme != PM_SCHEME_YEE || p.ndim != 3) return false;
-  if (p.sy != 128 && p.sy != 256 && p.sy != 512) return false;
+  if (p.sy % 64) return false;
+  if (p.coeff_kind == PM_COEFF_FULL && p.sy != 128 && p.sy != 256 && p.sy != 512) return false;
   if (p.nx > p.sy) return false;
   // the fused kernel addresses fields with 32-bit byte offsets
   const uint64_t esz = p.precision == PM_FP64 ? 8 : 4;
@@ -632,6 +714,11 @@ int pm_create(int device, void* stream, pm_ctx** out) {
   pm_ctx* c = new pm_ctx();
   c->device = device;
   c->stream = (hipStream_t)stream;
+  if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) !=
+          hipSuccess || c->n_cu < 1) {
+    (void)hipGetLastError();
+    c->n_cu = 256;
+  }
   // the two-step pass's second stream and its fork/join events; without
   // them the pass runs its two launches one after the other
   if (hipStreamCreateWithFlags(&c->s2, hipStreamNonBlocking) != hipSuccess ||

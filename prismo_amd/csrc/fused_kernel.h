@@ -89,6 +89,28 @@ __device__ __forceinline__ T lane_bcast(T v, int l) {
   }
 }
 
+// v moved across the wave's lanes by a DPP control (row_shl:n 0x100 + n: lane
+// l takes l + n of its 16; row_shr:n 0x110 + n: l - n; wave_shl:1 0x130 and
+// wave_shr:1 0x138: the same over all 64 lanes by one); lanes with no source
+// keep `fill`.  No LDS access and no SGPR.
+template <int CTRL>
+__device__ __forceinline__ int dpp32(int fill, int v) {
+  return __builtin_amdgcn_update_dpp(fill, v, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp(T fill, T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, dpp32<CTRL>(__builtin_bit_cast(int, fill),
+                                             __builtin_bit_cast(int, v)));
+  } else {
+    const unsigned long long f = __builtin_bit_cast(unsigned long long, fill);
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)dpp32<CTRL>((int)(unsigned)f, (int)(unsigned)u);
+    const unsigned hi = (unsigned)dpp32<CTRL>((int)(unsigned)(f >> 32), (int)(unsigned)(u >> 32));
+    return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);
+  }
+}
+
 // E-side CPML term, in place (E is computed on own cells only).
 template <typename T>
 __device__ __forceinline__ T fcpml_e(const KGrid& g, const KFz& z, T d, int a, int q, int p,
@@ -217,31 +239,38 @@ struct TileBox {
 template <typename T, int VEC, int W, int TY, int XS>
 struct FusedLds {
   static constexpr int RW = 64 * VEC * W;
-  T le[3][TY + 1][RW];     // E(n) of plane k
-  T lh[2][3][TY + 1][RW];  // H(n+1/2) of planes with parity 0 / 1
-  T xr[XS > 1 ? TY + 1 : 1];  // Ex(n) of plane k one cell right of the segment
+  // one wave per row takes its x neighbours from the neighbouring lanes, so
+  // Ey and Hy (which only x differences of other lanes read) stay out of LDS
+  static constexpr int NC = XS == 0 ? 2 : 3;
+  T le[NC][TY + 1][RW];     // E(n) of plane k: Ex [Ey] Ez
+  T lh[2][NC][TY + 1][RW];  // H(n+1/2) of planes with parity 0 / 1: Hx [Hy] Hz
+  T xr[XS != 1 ? TY + 1 : 1];  // Ex(n) of plane k one cell right of the segment
 };
 
 // One tile (TY rows x one z-chunk x one row segment of RW cells); b = the
 // workgroup's index within the launch segment of its kind (slab tiles or
 // interior tiles).
 //
-// Row segments (XS > 1: a padded row of XS * RW cells in XS workgroups).
+// Row segments (XS = 2: a padded row of 2 RW cells in two workgroups; XS = 0:
+// a row of any width in nseg workgroups of RW cells).
 // The H update of a segment's first cell takes E(n) of the cell to its left
 // from memory (E(n) is only read this step), and the E update of its last
 // cell takes H(n+1/2) of the cell to its right, which the last lane
 // recomputes from E(n), H(n-1/2) and the CPML memory of that cell with the
-// arithmetic the neighbouring segment uses for it (not stored).  Segment
-// boundaries lie outside the x CPML layers (the host checks).
+// arithmetic the neighbouring segment uses for it (not stored).  With XS = 2
+// the segment boundary lies outside the x CPML layers (the host checks); with
+// XS = 0 it may lie inside one, and the recomputed H takes that cell's x
+// CPML memory and profile as well.
 template <typename T, int CK, int VEC, int W, int TY, int XS, bool YZ, bool ADE>
 __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kchunk,
                                            int ntile_y, int nchunk, int nblocks, int order,
                                            const TileBox& bx, int b,
                                            FusedLds<T, VEC, W, TY, XS>& lds, const KAde* tab,
-                                           const T (*tcf)[12]) {
+                                           const T (*tcf)[12], int nseg = XS) {
   constexpr int RW = 64 * VEC * W;
   using ABits = std::conditional_t<(12 * VEC > 32), uint64_t, uint32_t>;
   static_assert(kMaxAde < 16, "box numbers are kept in 4 bits");
+  constexpr int CZ = XS == 0 ? 1 : 2;  // LDS slot of the z components
   auto& le = lds.le;
   auto& lh = lds.lh;
   const int per = (nblocks + 7) / 8;
@@ -260,8 +289,8 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
   }
   if (L >= nblocks) return;
   // consecutive tile numbers are the segments of one row tile
-  const int xs = XS > 1 ? L % XS : 0;
-  if constexpr (XS > 1) L /= XS;
+  const int xs = XS != 1 ? L % nseg : 0;
+  if constexpr (XS != 1) L /= nseg;
   int ty, kc;
   if constexpr (!YZ) {
     const int nty = bx.ty1 - bx.ty0, nkc = bx.kc1 - bx.kc0;
@@ -298,8 +327,8 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
   const int x0 = (tid % (64 * W)) * VEC;  // within the segment (LDS)
   const int gx0 = xs * RW + x0;             // within the row (memory)
   // this segment has a segment to its left / right
-  const bool seg_l = XS > 1 && xs > 0;
-  const bool seg_r = XS > 1 && xs + 1 < XS;
+  const bool seg_l = XS != 1 && xs > 0;
+  const bool seg_r = XS != 1 && xs + 1 < nseg;
   const bool lane_r = x0 == RW - VEC;
   const int j = ty * TY + w;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -394,15 +423,18 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
   // lane of every wave, loaded with the plane (lanes 0-1: Ey, Ez left of
   // the segment; 2-6: Ex, Ey, Ez, Hy, Hz right of it; 7: Ex right of it on
   // the row above the tile's first row; 8-9, slab tiles: the y and z H-side
-  // CPML memory right of it; other lanes repeat lane 2).  Scalar loads
+  // CPML memory right of it; 10-11, XS = 0: the x memory there; other lanes
+  // repeat lane 2).  Scalar loads
   // would cost no vector registers, but their counter is the one LDS
   // accesses use and they return out of order, so the first LDS wait of
   // every plane would wait for them.  A segment at the row's end reads
-  // column 0 or nx-1 (unused).  FP64 instances keep the scalar loads: at
-  // 168 VGPRs the lane-spread load's two registers per plane set cost them
-  // spills.
-  constexpr bool HL = XS > 1 && sizeof(T) == 4;
-  const int hlane = tid & 63;
+  // column 0 or nx-1 (unused).  FP64 instances with XS = 2 keep the scalar
+  // loads: at 168 VGPRs the lane-spread load's two registers per plane set
+  // cost them spills.
+  constexpr bool HL = XS == 0 || (XS == 2 && sizeof(T) == 4);
+  // slot of this lane: XS = 2 broadcasts (lane = slot); XS = 0 moves slots 0-1
+  // to lane 0 and slots 2-11, held by lanes 63-54, to lane 63
+  const int hlane = XS == 0 ? ((tid & 63) < 2 ? (tid & 63) : 65 - (tid & 63)) : (tid & 63);
   const char* hbase = z.bi;
   uint32_t hoff0 = 0, hstep = 0;
   if constexpr (HL) {
@@ -427,6 +459,13 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
       hbase = z.bc;
       hoff0 = z.phi[2] + z.ps[2] + (rcol0 + (uint32_t)nx * (uint32_t)jr) * esz;
       hstep = 0;
+    } else if (XS == 0 && (hlane == 10 || hlane == 11)) {
+      hbase = z.bc;
+      const uint32_t Sx = (uint32_t)(g.pml[0] + g.pml[1]);
+      const int sr = max(fslab((int)rcol0, nx, g.pml[0], g.pml[1]), 0);
+      hoff0 = z.phi[0] + (hlane == 11 ? z.ps[0] : 0u) +
+              fslab_off(g, 0, sr, (int)rcol0, jr, 0) * esz;
+      hstep = Sx * (uint32_t)ny * esz;
     } else {
       hoff0 = rowr * esz;
     }
@@ -493,7 +532,18 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
     return *(CT)(base + o);
   };
   T sr_exm = 0, hyh_p = 0, hzh_p = 0;
-  if constexpr (XS > 1) {
+  // x CPML slab position and H profile of that cell (XS = 0)
+  int sxr = -1;
+  T xbr = 1, xcr = 0, xikr = 1;
+  if constexpr (XS == 0) {
+    if (pml && seg_r && gxr < nx) sxr = fslab(gxr, nx, g.pml[0], g.pml[1]);
+    if (sxr >= 0) {
+      xbr = *zp<T>(z.bc, z.prof[0] + 3u * z.pn[0], gxr);
+      xcr = *zp<T>(z.bc, z.prof[0] + 4u * z.pn[0], gxr);
+      xikr = *zp<T>(z.bc, z.prof[0] + 5u * z.pn[0], gxr);
+    }
+  }
+  if constexpr (XS != 1) {
     if (row_ok && kb > 0) sr_exm = sld(z.bi, 0u, (uint32_t)jr * sy + rcol + (uint32_t)(kb - 1) * sz);
   }
 
@@ -554,7 +604,12 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
     //     column 0 or nx-1, unused)
     T sl_ey = 0, sl_ez = 0;
     T sr_ex = 0, sr_ey = 0, sr_ez = 0, sr_hy = 0, sr_hz = 0, sr_exu = 0, sr_q2 = 0, sr_q5 = 0;
-    if constexpr (HL) {
+    if constexpr (XS == 0) {
+      // valid in lane 0 (left) and lane 63 (right), the lanes that use them
+      sl_ey = seg_l ? cur.hl : (T)0;
+      sl_ez = seg_l ? dpp<0x101>((T)0, cur.hl) : (T)0;
+      sr_ex = cur.hl;
+    } else if constexpr (HL) {
       sl_ey = lane_bcast(cur.hl, 0);
       sl_ez = lane_bcast(cur.hl, 1);
       sr_ex = lane_bcast(cur.hl, 2);
@@ -567,7 +622,7 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
         sr_q2 = lane_bcast(cur.hl, 8);
         sr_q5 = lane_bcast(cur.hl, 9);
       }
-    } else if constexpr (XS > 1) {
+    } else if constexpr (XS != 1) {
       const uint32_t lo = (uint32_t)jr * sy + lcol + (uint32_t)k * sz;
       sl_ey = sld(z.bi, z.cs, lo);
       sl_ez = sld(z.bi, 2u * z.cs, lo);
@@ -592,6 +647,12 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
     fcb<T, CK, VEC>(z, 0, oq, cbx);
     fcb<T, CK, VEC>(z, 1, oq, cby);
     fcb<T, CK, VEC>(z, 2, oq, cbz);
+    T cax[VEC], cay[VEC], caz[VEC];
+    if constexpr (CK == PM_COEFF_CACB) {
+      fld(cax, zp<T>(z.bc, z.ca[0], oq));
+      fld(cay, zp<T>(z.bc, z.ca[1], oq));
+      fld(caz, zp<T>(z.bc, z.ca[2], oq));
+    }
     T qe[6][VEC];
     load_psi(z.pe, kq, qe);
     // z profiles of plane k (H side) and of the E plane (slab tiles only)
@@ -658,10 +719,10 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       le[0][w][x0 + e] = cur.ex[e];
-      le[1][w][x0 + e] = cur.ey[e];
-      le[2][w][x0 + e] = cur.ez[e];
+      if constexpr (XS != 0) le[1][w][x0 + e] = cur.ey[e];
+      le[CZ][w][x0 + e] = cur.ez[e];
     }
-    if constexpr (XS > 1) {
+    if constexpr (XS != 1) {
       if (lane_r) lds.xr[w] = sr_ex;
     }
     __syncthreads();
@@ -678,9 +739,15 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
         const int li = x0 + e, i = gx0 + e;
         const T ex = cur.ex[e], ey = cur.ey[e], ez = cur.ez[e];
         const T exj = w > 0 ? le[0][w - 1][li] : (first_row ? cur.exu[e] : (T)0);
-        const T ezj = w > 0 ? le[2][w - 1][li] : (first_row ? cur.ezu[e] : (T)0);
-        const T ezi = li > 0 ? le[2][w][li - 1] : (seg_l ? sl_ez : (T)0);
-        const T eyi = li > 0 ? le[1][w][li - 1] : (seg_l ? sl_ey : (T)0);
+        const T ezj = w > 0 ? le[CZ][w - 1][li] : (first_row ? cur.ezu[e] : (T)0);
+        T ezi, eyi;
+        if constexpr (XS == 0) {
+          ezi = dpp<0x138>(sl_ez, ez);
+          eyi = dpp<0x138>(sl_ey, ey);
+        } else {
+          ezi = li > 0 ? le[2][w][li - 1] : (seg_l ? sl_ez : (T)0);
+          eyi = li > 0 ? le[1][w][li - 1] : (seg_l ? sl_ey : (T)0);
+        }
         T c1 = (ez - ezj) * idy;  // Hx: dEz/dy - dEy/dz
         T c2 = (ey - eym[e]) * idz;
         T d1 = (ex - exm[e]) * idz;  // Hy: dEx/dz - dEz/dx
@@ -738,10 +805,44 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
       fzero(hz);
     }
     // (4b) row segments: H(n+1/2) of the cell right of the segment, with the
-    //      arithmetic of the H update above (that cell lies outside the x
-    //      CPML layers), kept in registers for the E update of the last cell
+    //      arithmetic of the H update above (with XS = 2 that cell lies outside
+    //      the x CPML layers), kept in registers for the E update of the last
+    //      cell
     T hyh = 0, hzh = 0;
-    if constexpr (XS > 1) {
+    if constexpr (XS == 0) {
+      // the whole wave computes, lane 63's result is used: no divergence
+      if (seg_r && row_ok) {
+        const T db = (T)g.db_const;
+        const T hl = cur.hl;
+        const T exj = w > 0 ? lds.xr[w - 1] : (first_row ? dpp<0x115>((T)0, hl) : (T)0);
+        T d1 = (hl - sr_exm) * idz;
+        T d2 = (dpp<0x112>((T)0, hl) - cur.ez[0]) * idx;
+        T f1 = (dpp<0x111>((T)0, hl) - cur.ey[0]) * idx;
+        T f2 = (hl - exj) * idy;
+        if (gxr < nx) {
+          if constexpr (YZ) {
+            if (sys >= 0) {
+              const T p0 = ybh * dpp<0x116>((T)0, hl) + ych * f2;
+              f2 = f2 * yikh + p0;
+            }
+            if (szs >= 0) {
+              const T p1 = zh[0] * dpp<0x117>((T)0, hl) + zh[1] * d1;
+              d1 = d1 * zh[2] + p1;
+            }
+          }
+          if (sxr >= 0) {
+            const T p0 = xbr * dpp<0x118>((T)0, hl) + xcr * d2;
+            const T p1 = xbr * dpp<0x119>((T)0, hl) + xcr * f1;
+            d2 = d2 * xikr + p0;
+            f1 = f1 * xikr + p1;
+          }
+        }
+        hyh = dpp<0x113>((T)0, hl) - db * (d1 - d2);
+        hzh = dpp<0x114>((T)0, hl) - db * (f1 - f2);
+        if (gxr >= nx || j >= ny - 1) hyh = 0;
+        if (gxr >= nx || k >= nz - 1) hzh = 0;
+      }
+    } else if constexpr (XS != 1) {
       if (seg_r && lane_r && row_ok) {
         const T db = (T)g.db_const;
         const T exj = w > 0 ? lds.xr[w - 1] : (first_row ? sr_exu : (T)0);
@@ -769,8 +870,8 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       lh[k & 1][0][w][x0 + e] = hx[e];
-      lh[k & 1][1][w][x0 + e] = hy[e];
-      lh[k & 1][2][w][x0 + e] = hz[e];
+      if constexpr (XS != 0) lh[k & 1][1][w][x0 + e] = hy[e];
+      lh[k & 1][CZ][w][x0 + e] = hz[e];
     }
     __syncthreads();
     // (6) E(n+1) on plane k-1
@@ -785,12 +886,21 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
       for (int e = 0; e < VEC; ++e) {
         const int li = x0 + e, i = gx0 + e;
         const int ir = li + 1 < RW ? li + 1 : li;
-        T hyx = lh[p][1][w][ir], hzx = lh[p][2][w][ir];
-        if (seg_r && li == RW - 1) {
-          hyx = hyh_p;
-          hzx = hzh_p;
+        T hyx, hzx;
+        if constexpr (XS == 0) {
+          // the last lane of the row's last segment: cells beyond the grid
+          // (zero) or, in a full row, a value no E cell uses
+          hyx = dpp<0x130>(hyh_p, hyp[e]);
+          hzx = dpp<0x130>(hzh_p, hzp[e]);
+        } else {
+          hyx = lh[p][1][w][ir];
+          hzx = lh[p][2][w][ir];
+          if (seg_r && li == RW - 1) {
+            hyx = hyh_p;
+            hzx = hzh_p;
+          }
         }
-        const T hxy = lh[p][0][w + 1][li], hzy = lh[p][2][w + 1][li];
+        const T hxy = lh[p][0][w + 1][li], hzy = lh[p][CZ][w + 1][li];
         T a1 = (hzy - hzp[e]) * idy;  // Ex: dHz/dy - dHy/dz
         T a2 = (hy[e] - hyp[e]) * idz;
         T b1 = (hx[e] - hxp[e]) * idz;  // Ey: dHx/dz - dHz/dx
@@ -832,6 +942,10 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
           vx = *zp<T>(z.bc, z.ca[0], o + e) * vx + fcbv<T, CK>(g, cbx[e]) * cx;
           vy = *zp<T>(z.bc, z.ca[1], o + e) * vy + fcbv<T, CK>(g, cby[e]) * cy;
           vz = *zp<T>(z.bc, z.ca[2], o + e) * vz + fcbv<T, CK>(g, cbz[e]) * cz;
+        } else if constexpr (CK == PM_COEFF_CACB) {
+          vx = cax[e] * vx + cbx[e] * cx;
+          vy = cay[e] * vy + cby[e] * cy;
+          vz = caz[e] * vz + cbz[e] * cz;
         } else {
           vx = vx + fcbv<T, CK>(g, cbx[e]) * cx;
           vy = vy + fcbv<T, CK>(g, cby[e]) * cy;
@@ -878,7 +992,7 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
       hyp[e] = hy[e];
       hzp[e] = hz[e];
     }
-    if constexpr (XS > 1) {
+    if constexpr (XS != 1) {
       sr_exm = sr_ex;
       hyh_p = hyh;
       hzh_p = hzh;
@@ -906,7 +1020,9 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
     for (int e = 0; e < VEC; ++e) {
       const int li = x0 + e, i = gx0 + e;
       const int ir = li + 1 < RW ? li + 1 : li;
-      const T hyx = (seg_r && li == RW - 1) ? hyh_p : lh[p][1][w][ir];
+      T hyx;
+      if constexpr (XS == 0) hyx = dpp<0x130>(hyh_p, hyp[e]);
+      else hyx = (seg_r && li == RW - 1) ? hyh_p : lh[p][1][w][ir];
       T c1 = (hyx - hyp[e]) * idx;
       T c2 = (lh[p][0][w + 1][li] - hxp[e]) * idy;
       const bool ezok = i < nx - 1 && j < ny - 1;
@@ -916,7 +1032,7 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
       }
       const T cz = c1 - c2;
       T vz;
-      if constexpr (CK == PM_COEFF_FULL)
+      if constexpr (CK == PM_COEFF_FULL || CK == PM_COEFF_CACB)
         vz = *zp<T>(z.bc, z.ca[2], o + e) * ezm[e] + fcbv<T, CK>(g, cbz[e]) * cz;
       else
         vz = ezm[e] + fcbv<T, CK>(g, cbz[e]) * cz;
@@ -930,6 +1046,26 @@ __device__ __forceinline__ void fused_tile(const KGrid& g, const KFz& z, int kch
     fst(zpw<T>(z.bo, (uint32_t)(1) * z.cs, o), zero);
     fst(zpw<T>(z.bo, (uint32_t)(2) * z.cs, o), oz);
   }
+}
+
+// Dispersive instances: the box table copied to LDS once per workgroup, and
+// the nine update coefficients of each box in the field type.
+template <typename T>
+__device__ __forceinline__ void stage_ade(const KGrid& g, KAde* ade_tab, T (*ade_cf)[12]) {
+  static_assert(sizeof(KAde) % 4 == 0, "KAde is copied as 32-bit words");
+  const int n = g.n_ade * (int)(sizeof(KAde) / 4);
+  const gptr<const uint32_t> src = (gptr<const uint32_t>)g.ade;
+  uint32_t* dst = (uint32_t*)ade_tab;
+  for (int t = threadIdx.x; t < n; t += blockDim.x) dst[t] = src[t];
+  __syncthreads();
+  if ((int)threadIdx.x < g.n_ade * 9) {
+    const int bq = threadIdx.x / 9, q = threadIdx.x % 9;
+    const KAde& a = ade_tab[bq];
+    const double v = q == 0 ? a.ke : q == 1 ? a.kp : q == 2 ? a.kq : q == 3 ? a.ks
+                   : q == 4 ? a.a0 : q == 5 ? a.a1 : q == 6 ? a.a2 : q == 7 ? a.a3 : a.a4;
+    ade_cf[bq][q] = (T)v;
+  }
+  __syncthreads();
 }
 
 // One launch for all tiles: workgroups [0, seg) take the CPML slab tiles
@@ -951,22 +1087,7 @@ __global__ __launch_bounds__(64 * W * (TY + 1)) void k_yee_fused(const KGrid g, 
   // and the nine update coefficients of each box in the field type (the
   // E update then reads them without a conversion)
   __shared__ T ade_cf[ADE ? kMaxAde : 1][12];
-  if constexpr (ADE) {
-    static_assert(sizeof(KAde) % 4 == 0, "KAde is copied as 32-bit words");
-    const int n = g.n_ade * (int)(sizeof(KAde) / 4);
-    const gptr<const uint32_t> src = (gptr<const uint32_t>)g.ade;
-    uint32_t* dst = (uint32_t*)ade_tab;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) dst[t] = src[t];
-    __syncthreads();
-    if ((int)threadIdx.x < g.n_ade * 9) {
-      const int bq = threadIdx.x / 9, q = threadIdx.x % 9;
-      const KAde& a = ade_tab[bq];
-      const double v = q == 0 ? a.ke : q == 1 ? a.kp : q == 2 ? a.kq : q == 3 ? a.ks
-                     : q == 4 ? a.a0 : q == 5 ? a.a1 : q == 6 ? a.a2 : q == 7 ? a.a3 : a.a4;
-      ade_cf[bq][q] = (T)v;
-    }
-    __syncthreads();
-  }
+  if constexpr (ADE) stage_ade<T>(g, ade_tab, ade_cf);
   const int b = blockIdx.x;
   if (b < seg)
     fused_tile<T, CK, VEC, W, TY, XS, true, ADE>(g, z, kchunk, ntile_y, nchunk, n_out, order,
@@ -981,25 +1102,33 @@ constexpr bool fused_fits() {
   return 64 * W * (TY + 1) <= 1024 && (size_t)9 * (TY + 1) * 64 * VEC * W * sizeof(T) <= 65536;
 }
 
+// Interior box of tiles of TY rows and kchunk planes: a tile computes H on
+// rows j0 .. j0+TY and E on rows j0 .. j0+TY-1, planes kb .. ke (H) and
+// kb .. ke-1 (E).
+inline TileBox interior_tiles(const KGrid& g, int TY, int kchunk) {
+  const int ntile_y = (g.ny + TY - 1) / TY;
+  const int nchunk = (g.nz + kchunk - 1) / kchunk;
+  TileBox bx{0, ntile_y, 0, nchunk};
+  if (g.has_pml) {
+    const int ylo = g.pml[2], yhi = g.ny - g.pml[3];  // rows [ylo, yhi) are inside
+    const int zlo = g.pml[4], zhi = g.nz - g.pml[5];
+    bx.ty0 = (ylo + TY - 1) / TY;
+    bx.ty1 = std::max(bx.ty0, (yhi - 1 - TY) / TY + 1);
+    if ((bx.ty1 - 1) * TY + TY > yhi - 1) bx.ty1 = bx.ty0;
+    bx.kc0 = (zlo + kchunk - 1) / kchunk;
+    bx.kc1 = std::max(bx.kc0, (zhi - 1) / kchunk);
+    if (bx.kc1 > bx.kc0 && (bx.kc1 - 1) * kchunk + kchunk > zhi - 1) bx.kc1 = bx.kc0;
+    if (bx.ty1 <= bx.ty0 || bx.kc1 <= bx.kc0) bx = TileBox{0, 0, 0, 0};
+  }
+  return bx;
+}
+
 template <typename T, int CK, int VEC, int W, int TY, int XS>
 int launch_fused_one(const KGrid& g, const KFz& z, int kchunk, int order, hipStream_t s) {
   if constexpr (fused_fits<T, VEC, W, TY>()) {
     const int ntile_y = (g.ny + TY - 1) / TY;
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
-    // interior box: a tile computes H on rows j0 .. j0+TY and E on rows
-    // j0 .. j0+TY-1, planes kb .. ke (H) and kb .. ke-1 (E)
-    TileBox bx{0, ntile_y, 0, nchunk};
-    if (g.has_pml) {
-      const int ylo = g.pml[2], yhi = g.ny - g.pml[3];  // rows [ylo, yhi) are inside
-      const int zlo = g.pml[4], zhi = g.nz - g.pml[5];
-      bx.ty0 = (ylo + TY - 1) / TY;
-      bx.ty1 = std::max(bx.ty0, (yhi - 1 - TY) / TY + 1);
-      if ((bx.ty1 - 1) * TY + TY > yhi - 1) bx.ty1 = bx.ty0;
-      bx.kc0 = (zlo + kchunk - 1) / kchunk;
-      bx.kc1 = std::max(bx.kc0, (zhi - 1) / kchunk);
-      if (bx.kc1 > bx.kc0 && (bx.kc1 - 1) * kchunk + kchunk > zhi - 1) bx.kc1 = bx.kc0;
-      if (bx.ty1 <= bx.ty0 || bx.kc1 <= bx.kc0) bx = TileBox{0, 0, 0, 0};
-    }
+    const TileBox bx = interior_tiles(g, TY, kchunk);
     // XS workgroups (row segments) per tile
     const int n_in = (bx.ty1 - bx.ty0) * (bx.kc1 - bx.kc0) * XS;
     const int n_out = ntile_y * nchunk * XS - n_in;

@@ -199,6 +199,13 @@ int launch_yee_fused_f32(const KGrid& g, int ck, const FusedBufs& fb, int vec, i
 int launch_yee_fused_f64(const KGrid& g, int ck, const FusedBufs& fb, int vec, int w, int ty,
                          int kchunk, int order, int xs, hipStream_t s);
 bool fused_supported(int precision, int ck, int vec, int w, int ty, int xs);
+// The same step in row segments of 64 cells, for rows of any width
+// (fused_seg.h): ty 3 or 7 rows per workgroup.
+int launch_yee_seg_f32(const KGrid& g, int ck, const FusedBufs& fb, int ty, int kchunk, int order,
+                       hipStream_t s);
+int launch_yee_seg_f64(const KGrid& g, int ck, const FusedBufs& fb, int ty, int kchunk, int order,
+                       hipStream_t s);
+bool seg_supported(int ck, int ty);
 // Two Yee steps per launch (fused2_kernel.h), FP32 fields, Cb in FP32 or
 // FP16, no dispersive boxes; the sources of the first step (table row
 // src_row, n_src entries of the device table src) are added inside.

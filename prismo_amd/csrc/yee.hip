@@ -97,7 +97,7 @@ __device__ __forceinline__ void e_apply(const KGrid& g, int c, int64_t off, int 
     return;
   }
   const T cb = load_cb<T, CK>(g, c, off);
-  if constexpr (CK == PM_COEFF_FULL) {
+  if constexpr (CK == PM_COEFF_FULL || CK == PM_COEFF_CACB) {
     F[off] = ((const T*)g.ca[c])[off] * e + cb * curl;
   } else {
     F[off] = e + cb * curl;
@@ -236,11 +236,19 @@ __global__ __launch_bounds__(kBX* kBY) void k_yee_e(const KGrid g, int kchunk) {
   }
 }
 
-static int kchunk_for(int nz) { return nz >= 64 ? 16 : (nz >= 8 ? 4 : 1); }
+// Planes per block: long chunks carry the neighbouring plane in registers,
+// but a small grid needs short ones to fill the chip (64^3 FP32, 16 planes:
+// 64 blocks, 36 + 39 us for H and E).
+static int kchunk_for(const KGrid& g) {
+  const int cols = ((g.nx + kBX - 1) / kBX) * ((g.ny + kBY - 1) / kBY);
+  int kc = g.nz >= 64 ? 16 : (g.nz >= 8 ? 4 : 1);
+  while (kc > 1 && cols * ((g.nz + kc - 1) / kc) < 1024) kc /= 2;
+  return kc;
+}
 
 template <typename T, int CK>
 static void launch_h_t(const KGrid& g, hipStream_t s) {
-  const int kc = g.ndim == 3 ? kchunk_for(g.nz) : 1;
+  const int kc = g.ndim == 3 ? kchunk_for(g) : 1;
   dim3 grid((g.nx + kBX - 1) / kBX, (g.ny + kBY - 1) / kBY, (g.nz + kc - 1) / kc);
   dim3 block(kBX, kBY);
   if (g.ndim == 3)
@@ -251,7 +259,7 @@ static void launch_h_t(const KGrid& g, hipStream_t s) {
 
 template <typename T, int CK>
 static void launch_e_t(const KGrid& g, hipStream_t s) {
-  const int kc = g.ndim == 3 ? kchunk_for(g.nz) : 1;
+  const int kc = g.ndim == 3 ? kchunk_for(g) : 1;
   dim3 grid((g.nx + kBX - 1) / kBX, (g.ny + kBY - 1) / kBY, (g.nz + kc - 1) / kc);
   dim3 block(kBX, kBY);
   if (g.ndim == 3)
@@ -263,20 +271,21 @@ static void launch_e_t(const KGrid& g, hipStream_t s) {
 void launch_yee_h(const KGrid& g, int precision, int ck, hipStream_t s) {
   if (precision == PM_FP64) {
     if (ck == PM_COEFF_FULL) launch_h_t<double, PM_COEFF_FULL>(g, s);
-    else launch_h_t<double, PM_COEFF_CB>(g, s);
+    else launch_h_t<double, PM_COEFF_CB>(g, s);  // Db is one constant: no other kind differs
   } else {
     if (ck == PM_COEFF_FULL) launch_h_t<float, PM_COEFF_FULL>(g, s);
-    else if (ck == PM_COEFF_CB) launch_h_t<float, PM_COEFF_CB>(g, s);
-    else launch_h_t<float, PM_COEFF_CB_F16>(g, s);
+    else launch_h_t<float, PM_COEFF_CB>(g, s);
   }
 }
 
 void launch_yee_e(const KGrid& g, int precision, int ck, hipStream_t s) {
   if (precision == PM_FP64) {
     if (ck == PM_COEFF_FULL) launch_e_t<double, PM_COEFF_FULL>(g, s);
+    else if (ck == PM_COEFF_CACB) launch_e_t<double, PM_COEFF_CACB>(g, s);
     else launch_e_t<double, PM_COEFF_CB>(g, s);
   } else {
     if (ck == PM_COEFF_FULL) launch_e_t<float, PM_COEFF_FULL>(g, s);
+    else if (ck == PM_COEFF_CACB) launch_e_t<float, PM_COEFF_CACB>(g, s);
     else if (ck == PM_COEFF_CB) launch_e_t<float, PM_COEFF_CB>(g, s);
     else launch_e_t<float, PM_COEFF_CB_F16>(g, s);
   }

@@ -143,7 +143,7 @@ class ModeSource(Source):
         from ..modes.yee import yee_modes
 
         eng = self._sim.solver.updater.engine_for(self._sim.fields)
-        if eng.coeff_kind == N.COEFF_FULL:
+        if eng.coeff_kind in (N.COEFF_FULL, N.COEFF_CACB):
             raise NotImplementedError("mode sources in lossy or magnetic media")
         a = _AX[self.axis]
         b, c = _CYC[a]

@@ -65,6 +65,52 @@ int pm_mlp_mse_batched(void* stream, int32_t batch, int32_t M, int32_t N, const 
 int pm_mlp_adam(void* stream, int64_t n, float* p, const float* g, float* m, float* v,
                 float lr, float beta1, float beta2, float eps, float weight_decay, int32_t t);
 
+/* Whole networks: layers 1 <= L <= 12 of widths sizes[0] (input) ..
+ * sizes[L] (output), each 1 .. 512; GELU after every layer but the last.  A
+ * member's parameters are flat: all weights ([out][in] row-major, layer by
+ * layer), then all biases.  Members (1 <= batch <= 65535) lie at multiples of
+ * the given strides (elements).  The sums of every product are those of
+ * pm_mlp_gemm.
+ *
+ * The kernels read the weights as BF16 in their operand order: `packed`, a
+ * zero-filled buffer of pm_mlp_net_packed elements per member (with train != 0
+ * also the transposes the backward pass reads; 0: the network is not taken),
+ * 16-byte aligned with a stride that is a multiple of 8. */
+int64_t pm_mlp_net_packed(int32_t layers, const int32_t* sizes, int32_t train);
+int pm_mlp_net_pack(void* stream, int32_t batch, int32_t layers, const int32_t* sizes,
+                    const float* P, int64_t stride_p, uint16_t* packed, int64_t stride_packed,
+                    int32_t train);
+
+/* Y[m][:] of every member for rows X[m][:] (stride_x 0: the members share X).
+ * acts / zs (both or neither): activations and pre-activations of the hidden
+ * layers, layer k as (M, sizes[k+1]) after the layers before it. */
+int pm_mlp_net_forward(void* stream, int32_t batch, int32_t M, int32_t layers,
+                       const int32_t* sizes, const float* P, int64_t stride_p,
+                       const uint16_t* packed, int64_t stride_packed, const float* X,
+                       int64_t stride_x, float* Y, int64_t stride_y, float* acts, float* zs,
+                       int64_t stride_a);
+
+/* One pass over `rows` training rows in minibatches of batch_rows (the last
+ * one shorter): per minibatch s the mean squared error's gradient (weights w
+ * per output column, NULL = 1) in G and one Adam step t0 + s + 1 with rate
+ * lr[s] (a host array) and decay weight_decay on the weights.  Row r of member
+ * q is row idx[q * stride_idx + r] of X and T (shared by the members).  packed
+ * (train != 0) holds P's weights and is kept up to date; work:
+ * batch * pm_mlp_net_work(.., batch_rows) elements; loss[s * batch + q], zeroed
+ * by the caller. */
+int64_t pm_mlp_net_work(int32_t layers, const int32_t* sizes, int32_t rows);
+int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t* sizes, float* P,
+                     float* G, float* m, float* v, int64_t stride_p, uint16_t* packed,
+                     int64_t stride_packed, const float* X, const float* T, const int64_t* idx,
+                     int64_t stride_idx, const float* w, int32_t rows, int32_t batch_rows,
+                     float* work, const float* lr, float beta1, float beta2, float eps,
+                     float weight_decay, int32_t t0, float* loss);
+
+/* Mean and standard deviation (divisor members - 1) over the members of n
+ * values at S[q * stride]. */
+int pm_mlp_net_stats(void* stream, int32_t members, int64_t n, const float* S, int64_t stride,
+                     float* mean, float* std);
+
 #ifdef __cplusplus
 }
 #endif

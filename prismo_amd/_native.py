@@ -160,6 +160,15 @@ MLP_SIGNATURES = {
                              i64, vp, i64, i64, vp, i64, vp, i64], C.c_int),
     "pm_mlp_colsum_batched": ([vp, i32, i32, i32, vp, i64, i64, vp, i64], C.c_int),
     "pm_mlp_mse_batched": ([vp, i32, i32, i32, vp, vp, i64, vp, vp, vp], C.c_int),
+    "pm_mlp_net_packed": ([i32, vp, i32], i64),
+    "pm_mlp_net_work": ([i32, vp, i32], i64),
+    "pm_mlp_net_pack": ([vp, i32, i32, vp, vp, i64, vp, i64, i32], C.c_int),
+    "pm_mlp_net_forward": ([vp, i32, i32, i32, vp, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp,
+                            i64], C.c_int),
+    "pm_mlp_net_train": ([vp, i32, i32, vp, vp, vp, vp, vp, i64, vp, i64, vp, vp, vp, i64, vp,
+                          i32, i32, vp, vp, C.c_float, C.c_float, C.c_float, C.c_float, i32, vp],
+                         C.c_int),
+    "pm_mlp_net_stats": ([vp, i32, i64, vp, i64, vp, vp], C.c_int),
 }
 
 BATCH_SIGNATURES = {

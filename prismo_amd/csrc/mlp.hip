@@ -55,26 +55,23 @@ struct GemmBatch {
   int64_t a, b, c, bias, z;
 };
 
-__global__ __launch_bounds__(256) void k_gemm(int mode, int M, int N, int K,
-                                              const float* __restrict__ A, int64_t lam,
-                                              int64_t lak, const float* __restrict__ B,
-                                              int64_t lbk, int64_t lbn, float* __restrict__ C,
-                                              int64_t ldc, const float* __restrict__ bias,
-                                              float* __restrict__ Z, GemmBatch bs) {
-  {
-    const int64_t q = blockIdx.z;
-    A += q * bs.a;
-    B += q * bs.b;
-    C += q * bs.c;
-    if (bias) bias += q * bs.bias;
-    if (Z) Z += q * bs.z;
-  }
-  __shared__ unsigned short sa[kBM][kBK + kPad];
-  __shared__ unsigned short sb[kBN][kBK + kPad];
+struct GemmLds {
+  unsigned short a[kBM][kBK + kPad];
+  unsigned short b[kBN][kBK + kPad];
+};
+
+// The 64 x 64 block of C at (m0, n0), by the 256 threads of a workgroup.
+__device__ __forceinline__ void gemm_tile(int mode, int M, int N, int K,
+                                          const float* __restrict__ A, int64_t lam, int64_t lak,
+                                          const float* __restrict__ B, int64_t lbk, int64_t lbn,
+                                          float* __restrict__ C, int64_t ldc,
+                                          const float* __restrict__ bias, float* __restrict__ Z,
+                                          int m0, int n0, GemmLds& lds) {
+  auto& sa = lds.a;
+  auto& sb = lds.b;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
   const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;
   const int li = lane & 15, lq = lane >> 4;
   f32x4 acc[2][2];
@@ -183,14 +180,24 @@ __global__ __launch_bounds__(256) void k_gemm(int mode, int M, int N, int K,
       }
 }
 
+__global__ __launch_bounds__(256) void k_gemm(int mode, int M, int N, int K,
+                                              const float* __restrict__ A, int64_t lam,
+                                              int64_t lak, const float* __restrict__ B,
+                                              int64_t lbk, int64_t lbn, float* __restrict__ C,
+                                              int64_t ldc, const float* __restrict__ bias,
+                                              float* __restrict__ Z, GemmBatch bs) {
+  __shared__ GemmLds lds;
+  const int64_t q = blockIdx.z;
+  gemm_tile(mode, M, N, K, A + q * bs.a, lam, lak, B + q * bs.b, lbk, lbn, C + q * bs.c, ldc,
+            bias ? bias + q * bs.bias : nullptr, Z ? Z + q * bs.z : nullptr, blockIdx.y * kBM,
+            blockIdx.x * kBN, lds);
+}
+
 // one workgroup per 64 columns; 4 waves split the rows, then combine in LDS
-__global__ __launch_bounds__(256) void k_colsum(int M, int N, const float* __restrict__ A,
-                                                int64_t lda, float* __restrict__ out,
-                                                int64_t sa, int64_t so) {
-  __shared__ float part[4][64];
-  A += (int64_t)blockIdx.y * sa;  // problem of a batch
-  out += (int64_t)blockIdx.y * so;
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63);
+__device__ __forceinline__ void colsum_tile(int M, int N, const float* __restrict__ A,
+                                            int64_t lda, float* __restrict__ out, int c0,
+                                            float (&part)[4][64]) {
+  const int c = c0 + (threadIdx.x & 63);
   const int w = threadIdx.x >> 6;
   float s = 0.0f;
   if (c < N)
@@ -200,6 +207,14 @@ __global__ __launch_bounds__(256) void k_colsum(int M, int N, const float* __res
   if (w == 0 && c < N)
     out[c] = (part[0][threadIdx.x] + part[1][threadIdx.x]) +
              (part[2][threadIdx.x] + part[3][threadIdx.x]);
+}
+
+__global__ __launch_bounds__(256) void k_colsum(int M, int N, const float* __restrict__ A,
+                                                int64_t lda, float* __restrict__ out,
+                                                int64_t sa, int64_t so) {
+  __shared__ float part[4][64];
+  const int64_t q = blockIdx.y;  // problem of a batch
+  colsum_tile(M, N, A + q * sa, lda, out + q * so, blockIdx.x * 64, part);
 }
 
 __global__ __launch_bounds__(256) void k_mse(int M, int N, const float* __restrict__ Y,
@@ -249,6 +264,435 @@ __global__ __launch_bounds__(256) void k_adam(int64_t n, float* __restrict__ p,
     const float mh = mi / c1, vh = vi / c2;
     p[e] -= lr * (mh / (sqrtf(vh) + eps) + wd * p[e]);
   }
+}
+
+// ------------------------------------------------------- whole networks
+// A layer-by-layer pass moves every activation through memory between
+// launches of 64 x 64 tiles: on 65 536 rows of a 4 x 256 network 86 us a
+// layer, on a training batch of 256 rows 24 us a launch with 64 workgroups
+// (a sixteenth of the chip) waiting for memory.  Here a workgroup takes BM
+// rows through all layers, the activations staying in LDS as the BF16 values
+// the next product would round them to anyway (the same products in the same
+// order: the sums are bitwise those of gemm_tile).  What it reads per layer is
+// the weights alone, packed as BF16 in operand order (one 16-byte load per
+// lane, tile and K-step, no guard), from L2.
+//
+// 8 waves as WR x WC; a wave owns RT row tiles and NT column tiles of 16,
+// column tiles interleaved over the waves (tile t WC + wc).
+
+constexpr int kNetL = 12;      // layers
+constexpr int kNetWidth = 512; // widest layer
+
+// A network of L layers of widths n[0] .. n[L], parameters flat per member:
+// all weights (row-major [out][in]), then all biases.
+struct NetDesc {
+  int L;
+  int n[kNetL + 1];
+  int64_t woff[kNetL], boff[kNetL];  // in the member's flat parameters
+  int64_t poff[kNetL], qoff[kNetL];  // packed weights, packed transposed weights
+  int64_t aoff[kNetL];               // rows times this: hidden layer k's values
+  int64_t goff[kNetL];               // rows times this: layer k's output gradient
+  int64_t nW, nP;                    // weights, parameters
+  int64_t nfwd, npack;               // packed elements without / with the transposes
+  int64_t nhid, ngrad;               // values per row over hidden / all layers
+  int kp;                            // LDS row: widest padded operand + 8
+};
+
+__host__ __device__ constexpr int up32(int n) { return (n + 31) & ~31; }
+__host__ __device__ constexpr int up16(int n) { return (n + 15) & ~15; }
+
+// Operand order: tile of 16 columns (n) x 32 k: lane l holds column l % 16,
+// k = 8 (l / 16) .. + 7.
+__device__ __forceinline__ int64_t pack_at(int n, int k, int K) {
+  const int kt = up32(K) / 32;
+  const int lane = (n & 15) + 16 * ((k >> 3) & 3);
+  return (((int64_t)(n >> 4) * kt + (k >> 5)) * 64 + lane) * 8 + (k & 7);
+}
+
+// The packed copies of parameter e (a weight); transposed ones where the
+// backward pass takes them (not of the first layer).
+__device__ __forceinline__ void pack_weight(const NetDesc& d, unsigned short* pk, int64_t e,
+                                            float v, bool trans) {
+  int k = 0;
+  while (k + 1 < d.L && e >= d.woff[k + 1]) ++k;
+  const int fi = d.n[k];
+  const int r = (int)(e - d.woff[k]);
+  const int o = r / fi, i = r - o * fi;
+  const unsigned short b = to_bf16(v);
+  pk[d.poff[k] + pack_at(o, i, fi)] = b;
+  if (trans && k > 0) pk[d.qoff[k] + pack_at(i, o, d.n[k + 1])] = b;
+}
+
+__global__ __launch_bounds__(256) void k_net_pack(const NetDesc d, const float* __restrict__ P,
+                                                  int64_t ps, unsigned short* __restrict__ pk,
+                                                  int64_t ks, int trans) {
+  const int64_t q = blockIdx.y;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < d.nW;
+       e += (int64_t)gridDim.x * 256)
+    pack_weight(d, pk + q * ks, e, P[q * ps + e], trans != 0);
+}
+
+extern __shared__ unsigned short net_lds[];
+
+// acc += A B over K (padded to 32) for this wave's tiles; A from LDS rows,
+// B from the packed weights, the next K-step's loads in flight.
+template <int RT, int NT, int WC>
+__device__ __forceinline__ void net_gemm(const unsigned short* sA, int kp, int row0, int wc,
+                                         int ntiles, int K, const unsigned short* __restrict__ pk,
+                                         f32x4 (&acc)[RT][NT]) {
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int kt = up32(K) / 32;
+  bf16x8 bn[NT];
+  const unsigned short* bp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    // tiles past the layer's width repeat the last one (unused)
+    const int nt = min(t * WC + wc, ntiles - 1);
+    bp[t] = pk + ((int64_t)nt * kt * 64 + lane) * 8;
+    bn[t] = *(const bf16x8*)bp[t];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][t] = f32x4{0, 0, 0, 0};
+  }
+  const unsigned short* ap = sA + (row0 + li) * kp + 8 * lq;
+  for (int s = 0; s < kt; ++s) {
+    bf16x8 bv[NT], av[RT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      bv[t] = bn[t];
+      bp[t] += s + 1 < kt ? 512 : 0;
+      bn[t] = *(const bf16x8*)bp[t];
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) av[r] = *(const bf16x8*)(ap + 16 * r * kp + 32 * s);
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[r], bv[t], acc[r][t], 0, 0, 0);
+  }
+}
+
+// Rows m0 .. of src (row stride ld, through idx when given) into LDS as BF16,
+// zero beyond the rows and beyond column n up to a multiple of 32; copy keeps
+// the gathered values.
+__device__ __forceinline__ void net_stage(unsigned short* sA, int kp, int bm, int m0, int M,
+                                          int n, const float* __restrict__ src, int64_t ld,
+                                          const int64_t* __restrict__ idx,
+                                          float* __restrict__ copy) {
+  const int np = up32(n);
+  for (int f = threadIdx.x; f < bm * np; f += blockDim.x) {
+    const int r = f / np, c = f - r * np;
+    float v = 0.0f;
+    if (m0 + r < M && c < n) {
+      const int64_t row = idx ? idx[m0 + r] : m0 + r;
+      v = src[row * ld + c];
+      if (copy) copy[(int64_t)(m0 + r) * n + c] = v;
+    }
+    sA[r * kp + c] = to_bf16(v);
+  }
+}
+
+// Y = network(X) for rows of every member (blockIdx.y); hidden activations and
+// pre-activations kept in acts / zs (member stride as_, layer k at M aoff[k])
+// when given.
+template <int RT, int NT, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC) void k_net_forward(
+    const NetDesc d, int M, const float* __restrict__ P, int64_t ps,
+    const unsigned short* __restrict__ pk, int64_t ks, const float* __restrict__ X, int64_t xs,
+    float* __restrict__ Y, int64_t ys, float* __restrict__ acts, float* __restrict__ zs,
+    int64_t as_) {
+  constexpr int BM = 16 * RT * WR;
+  unsigned short* sA = net_lds;
+  const int64_t q = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wv / WC, wc = wv % WC;
+  const int m0 = blockIdx.x * BM, row0 = wr * 16 * RT;
+  const float* Pq = P + q * ps;
+  net_stage(sA, d.kp, BM, m0, M, d.n[0], X + q * xs, d.n[0], nullptr, nullptr);
+  __syncthreads();
+  for (int k = 0; k < d.L; ++k) {
+    const int K = d.n[k], N = d.n[k + 1];
+    f32x4 acc[RT][NT];
+    net_gemm<RT, NT, WC>(sA, d.kp, row0, wc, up16(N) / 16, K, pk + q * ks + d.poff[k], acc);
+    const bool last = k + 1 == d.L;
+    __syncthreads();  // every wave has read its operands: the rows are replaced
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = 16 * (t * WC + wc) + li;
+      if (16 * (t * WC + wc) >= up32(N)) continue;
+      const float bias = n < N ? Pq[d.boff[k] + n] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = row0 + 16 * r + 4 * lq + e;
+          const int m = m0 + row;
+          const float z = acc[r][t][e] + bias;
+          if (last) {
+            if (n < N && m < M) Y[q * ys + (int64_t)m * N + n] = z;
+            continue;
+          }
+          const float a = n < N ? gelu(z) : 0.0f;
+          sA[row * d.kp + n] = to_bf16(a);
+          if (zs && n < N && m < M) {
+            const int64_t o = q * as_ + (int64_t)M * d.aoff[k] + (int64_t)m * N + n;
+            zs[o] = z;
+            acts[o] = a;
+          }
+        }
+    }
+    __syncthreads();
+  }
+}
+
+// One training batch of every member (blockIdx.y), 16 rows per workgroup:
+// forward, the weighted squared error's gradient and loss, and the gradient
+// carried back to the first hidden layer.  Rows are gathered through idx;
+// acts (the gathered inputs, then the hidden activations), pre-activations and
+// output gradients of every layer go to the workspace for k_net_grads.
+template <int NT>
+__global__ __launch_bounds__(512) void k_net_train(
+    const NetDesc d, int B, const float* __restrict__ P, int64_t ps,
+    const unsigned short* __restrict__ pk, int64_t ks, const float* __restrict__ X,
+    const float* __restrict__ T, const int64_t* __restrict__ idx, int64_t is,
+    const float* __restrict__ w, float* __restrict__ x0, float* __restrict__ acts,
+    float* __restrict__ zs, float* __restrict__ G, float* __restrict__ loss) {
+  constexpr int WC = 8;
+  unsigned short* sA = net_lds;
+  __shared__ float red[8];
+  const int64_t q = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int wc = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = blockIdx.x * 16;
+  const float* Pq = P + q * ps;
+  const unsigned short* pq = pk + q * ks;
+  idx += q * is;
+  x0 += q * (int64_t)B * d.n[0];
+  acts += q * (int64_t)B * d.nhid;
+  zs += q * (int64_t)B * d.nhid;
+  G += q * (int64_t)B * d.ngrad;
+  net_stage(sA, d.kp, 16, m0, B, d.n[0], X, d.n[0], idx, x0);
+  __syncthreads();
+  const int NL = d.n[d.L];
+  const float scale = 1.0f / (float)((int64_t)B * NL);
+  float s = 0.0f;
+  for (int k = 0; k < d.L; ++k) {
+    const int K = d.n[k], N = d.n[k + 1];
+    f32x4 acc[1][NT];
+    net_gemm<1, NT, WC>(sA, d.kp, 0, wc, up16(N) / 16, K, pq + d.poff[k], acc);
+    const bool last = k + 1 == d.L;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = 16 * (t * WC + wc) + li;
+      if (16 * (t * WC + wc) >= up32(N)) continue;
+      const float bias = n < N ? Pq[d.boff[k] + n] : 0.0f;
+      const float wt = last && w && n < N ? w[n] : 1.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 4 * lq + e, m = m0 + row;
+        const bool ok = n < N && m < B;
+        const float z = acc[0][t][e] + bias;
+        float v = 0.0f;
+        if (last) {
+          if (ok) {
+            const float dd = z - T[idx[m] * NL + n];
+            s += wt * dd * dd;
+            v = 2.0f * wt * dd * scale;
+            G[(int64_t)B * d.goff[k] + (int64_t)m * N + n] = v;
+          }
+        } else if (n < N) {
+          v = gelu(z);
+          if (ok) {
+            const int64_t o = (int64_t)B * d.aoff[k] + (int64_t)m * N + n;
+            zs[o] = z;
+            acts[o] = v;
+          }
+        }
+        sA[row * d.kp + n] = to_bf16(v);
+      }
+    }
+    __syncthreads();
+  }
+  // back through the layers: G_{k-1} = (G_k W_k) gelu'(z_{k-1})
+  for (int k = d.L - 1; k > 0; --k) {
+    const int K = d.n[k + 1], N = d.n[k];
+    f32x4 acc[1][NT];
+    net_gemm<1, NT, WC>(sA, d.kp, 0, wc, up16(N) / 16, K, pq + d.qoff[k], acc);
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = 16 * (t * WC + wc) + li;
+      if (16 * (t * WC + wc) >= up32(N)) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 4 * lq + e, m = m0 + row;
+        float v = 0.0f;
+        if (n < N && m < B) {
+          // this thread wrote the pre-activation in the forward pass
+          v = acc[0][t][e] * dgelu(zs[(int64_t)B * d.aoff[k - 1] + (int64_t)m * N + n]);
+          G[(int64_t)B * d.goff[k - 1] + (int64_t)m * N + n] = v;
+        }
+        sA[row * d.kp + n] = to_bf16(v);
+      }
+    }
+    __syncthreads();
+  }
+  for (int h = 32; h >= 1; h >>= 1) s += __shfl_xor(s, h);
+  if (lane == 0) red[wc] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float a = 0.0f;
+    for (int i = 0; i < 8; ++i) a += red[i];
+    atomicAdd(loss + q, a * scale);
+  }
+}
+
+// Weight gradients (64 x 64 tiles of G_k^T a_k) and bias gradients (column
+// sums) of all layers, one launch.
+__global__ __launch_bounds__(256) void k_net_grads(const NetDesc d, int B,
+                                                   const float* __restrict__ x0,
+                                                   const float* __restrict__ acts,
+                                                   const float* __restrict__ G,
+                                                   float* __restrict__ gP, int64_t ps) {
+  __shared__ GemmLds lds;
+  __shared__ float part[4][64];
+  const int64_t q = blockIdx.y;
+  G += q * (int64_t)B * d.ngrad;
+  gP += q * ps;
+  int b = blockIdx.x;
+  for (int k = 0; k < d.L; ++k) {
+    const int fi = d.n[k], fo = d.n[k + 1];
+    const int gx = (fi + kBN - 1) / kBN, gy = (fo + kBM - 1) / kBM;
+    const float* g = G + (int64_t)B * d.goff[k];
+    if (b < gx * gy) {
+      const float* a = k == 0 ? x0 + q * (int64_t)B * fi
+                              : acts + q * (int64_t)B * d.nhid + (int64_t)B * d.aoff[k - 1];
+      gemm_tile(PM_MLP_PLAIN, fo, fi, B, g, 1, fo, a, fi, 1, gP + d.woff[k], fi, nullptr, nullptr,
+                (b / gx) * kBM, (b % gx) * kBN, lds);
+      return;
+    }
+    b -= gx * gy;
+    if (b < gy) {
+      colsum_tile(B, fo, g, fo, gP + d.boff[k], b * 64, part);
+      return;
+    }
+    b -= gy;
+  }
+}
+
+// k_adam's update on every member's parameters (decay on the weights only),
+// with the packed copies of the new weights.
+__global__ __launch_bounds__(256) void k_net_adam(const NetDesc d, float* __restrict__ p,
+                                                  const float* __restrict__ g,
+                                                  float* __restrict__ m, float* __restrict__ v,
+                                                  int64_t ps, unsigned short* __restrict__ pk,
+                                                  int64_t ks, float lr, float b1, float b2,
+                                                  float eps, float wd, float c1, float c2) {
+  const int64_t q = blockIdx.y;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < d.nP;
+       e += (int64_t)gridDim.x * 256) {
+    const int64_t o = q * ps + e;
+    const float gi = g[o];
+    const float mi = b1 * m[o] + (1.0f - b1) * gi;
+    const float vi = b2 * v[o] + (1.0f - b2) * gi * gi;
+    m[o] = mi;
+    v[o] = vi;
+    const float mh = mi / c1, vh = vi / c2;
+    const float pe = p[o];
+    const float pn = pe - lr * (mh / (sqrtf(vh) + eps) + (e < d.nW ? wd : 0.0f) * pe);
+    p[o] = pn;
+    if (e < d.nW) pack_weight(d, pk + q * ks, e, pn, true);
+  }
+}
+
+// Mean and standard deviation (divisor nm - 1) over the members' values.
+__global__ __launch_bounds__(256) void k_net_stats(int nm, int64_t n, const float* __restrict__ S,
+                                                   int64_t ss, float* __restrict__ mean,
+                                                   float* __restrict__ sd) {
+  for (int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; e < n;
+       e += (int64_t)gridDim.x * 1024) {
+    const int c = (int)min((int64_t)4, n - e);
+    float a[4] = {0, 0, 0, 0}, v[4] = {0, 0, 0, 0};
+    for (int q = 0; q < nm; ++q)
+      for (int i = 0; i < c; ++i) a[i] += S[q * ss + e + i];
+    for (int i = 0; i < 4; ++i) a[i] /= (float)nm;
+    for (int q = 0; q < nm; ++q)
+      for (int i = 0; i < c; ++i) {
+        const float t = S[q * ss + e + i] - a[i];
+        v[i] += t * t;
+      }
+    for (int i = 0; i < c; ++i) {
+      mean[e + i] = a[i];
+      sd[e + i] = sqrtf(v[i] / (float)(nm - 1));
+    }
+  }
+}
+
+// The network's layout, or false when the whole-network kernels do not take it.
+bool net_desc(int L, const int32_t* n, NetDesc* out) {
+  if (L < 1 || L > kNetL || !n) return false;
+  NetDesc d{};
+  d.L = L;
+  for (int k = 0; k <= L; ++k) {
+    if (n[k] < 1 || n[k] > kNetWidth) return false;
+    d.n[k] = n[k];
+    d.kp = std::max(d.kp, up32(n[k]) + 8);
+  }
+  int64_t w = 0, pk = 0, a = 0, g = 0;
+  for (int k = 0; k < L; ++k) {
+    d.woff[k] = w;
+    w += (int64_t)n[k] * n[k + 1];
+    d.poff[k] = pk;
+    pk += (int64_t)up16(n[k + 1]) * up32(n[k]);
+    d.aoff[k] = a;
+    if (k + 1 < L) a += n[k + 1];
+    d.goff[k] = g;
+    g += n[k + 1];
+  }
+  d.nfwd = pk;
+  for (int k = 1; k < L; ++k) {
+    d.qoff[k] = pk;
+    pk += (int64_t)up16(n[k]) * up32(n[k + 1]);
+  }
+  d.npack = pk;
+  d.nW = w;
+  for (int k = 0; k < L; ++k) {
+    d.boff[k] = w;
+    w += n[k + 1];
+  }
+  d.nP = w;
+  d.nhid = a;
+  d.ngrad = g;
+  *out = d;
+  return true;
+}
+
+// Column tiles per wave for the widest layer output over wc waves.
+int net_nt(const NetDesc& d, int wc, bool back) {
+  int most = 0;
+  for (int k = back ? 0 : 1; k <= d.L; ++k) most = std::max(most, up32(d.n[k]) / 16);
+  return (most + wc - 1) / wc;
+}
+
+// The packed weights are read 16 bytes at a time.
+bool packed_ok(const uint16_t* p, int64_t stride) {
+  return p && (uintptr_t)p % 16 == 0 && stride % 8 == 0;
+}
+
+template <typename F>
+int net_launch(F* fn, dim3 grid, dim3 block, size_t lds, hipStream_t s, void** args) {
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute((const void*)fn,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  const hipError_t e = hipLaunchKernel((const void*)fn, grid, block, args, lds, s);
+  return e == hipSuccess ? 0 : (int)e;
 }
 
 int status() {
@@ -325,6 +769,120 @@ int pm_mlp_adam(void* stream, int64_t n, float* p, const float* g, float* m, flo
   const int blocks = (int)std::min<int64_t>((n + 255) / 256, 2048);
   hipLaunchKernelGGL(k_adam, dim3(blocks), dim3(256), 0, (hipStream_t)stream, n, p, g, m, v,
                      lr, beta1, beta2, eps, weight_decay, c1, c2);
+  return status();
+}
+
+int64_t pm_mlp_net_packed(int32_t layers, const int32_t* sizes, int32_t train) {
+  NetDesc d;
+  if (!net_desc(layers, sizes, &d)) return 0;
+  return train ? d.npack : d.nfwd;
+}
+
+int64_t pm_mlp_net_work(int32_t layers, const int32_t* sizes, int32_t rows) {
+  NetDesc d;
+  if (!net_desc(layers, sizes, &d) || rows < 1) return 0;
+  return (int64_t)rows * (d.n[0] + 2 * d.nhid + d.ngrad);
+}
+
+int pm_mlp_net_pack(void* stream, int32_t batch, int32_t layers, const int32_t* sizes,
+                    const float* P, int64_t stride_p, uint16_t* packed, int64_t stride_packed,
+                    int32_t train) {
+  NetDesc d;
+  if (!net_desc(layers, sizes, &d) || !P || !packed_ok(packed, stride_packed) || batch < 1 ||
+      batch > 65535)
+    return PM_EINVAL;
+  const int blocks = (int)std::min<int64_t>((d.nW + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_net_pack, dim3(blocks, batch), dim3(256), 0, (hipStream_t)stream, d, P,
+                     stride_p, packed, stride_packed, train);
+  return status();
+}
+
+int pm_mlp_net_forward(void* stream, int32_t batch, int32_t M, int32_t layers,
+                       const int32_t* sizes, const float* P, int64_t stride_p,
+                       const uint16_t* packed, int64_t stride_packed, const float* X,
+                       int64_t stride_x, float* Y, int64_t stride_y, float* acts, float* zs,
+                       int64_t stride_a) {
+  NetDesc d;
+  if (!net_desc(layers, sizes, &d) || !P || !packed_ok(packed, stride_packed) || !X || !Y ||
+      batch < 1 || batch > 65535 || M < 0 || (acts == nullptr) != (zs == nullptr))
+    return PM_EINVAL;
+  if (M == 0) return 0;
+  void* args[] = {&d, &M, &P, &stride_p, &packed, &stride_packed, &X, &stride_x, &Y, &stride_y,
+                  &acts, &zs, &stride_a};
+  hipStream_t s = (hipStream_t)stream;
+  // 128 rows per workgroup (64 when a layer is wider than 256, for the
+  // registers) read the weights once for all of them; when those are too few
+  // workgroups for 256 CUs, 16 rows
+  const int wide = net_nt(d, 4, false) > 4 ? 64 : 128;
+  const bool big = (int64_t)batch * ((M + wide - 1) / wide) >= 256;
+  const int bm = big ? wide : 16;
+  const dim3 grid((M + bm - 1) / bm, batch), block(512);
+  const size_t lds = (size_t)bm * d.kp * sizeof(unsigned short);
+  if (big) {
+    const int nt = net_nt(d, 4, false);
+    if (nt <= 1) return net_launch(k_net_forward<4, 1, 2, 4>, grid, block, lds, s, args);
+    if (nt <= 2) return net_launch(k_net_forward<4, 2, 2, 4>, grid, block, lds, s, args);
+    if (nt <= 4) return net_launch(k_net_forward<4, 4, 2, 4>, grid, block, lds, s, args);
+    return net_launch(k_net_forward<2, 8, 2, 4>, grid, block, lds, s, args);
+  }
+  const int nt = net_nt(d, 8, false);
+  if (nt <= 1) return net_launch(k_net_forward<1, 1, 1, 8>, grid, block, lds, s, args);
+  if (nt <= 2) return net_launch(k_net_forward<1, 2, 1, 8>, grid, block, lds, s, args);
+  return net_launch(k_net_forward<1, 4, 1, 8>, grid, block, lds, s, args);
+}
+
+int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t* sizes, float* P,
+                     float* G, float* m, float* v, int64_t stride_p, uint16_t* packed,
+                     int64_t stride_packed, const float* X, const float* T, const int64_t* idx,
+                     int64_t stride_idx, const float* w, int32_t rows, int32_t batch_rows,
+                     float* work, const float* lr, float beta1, float beta2, float eps,
+                     float weight_decay, int32_t t0, float* loss) {
+  NetDesc d;
+  if (!net_desc(layers, sizes, &d) || !P || !G || !m || !v ||
+      !packed_ok(packed, stride_packed) || !X || !T || !idx || !work || !lr || !loss || batch < 1 || batch > 65535 || rows < 1 || batch_rows < 1 || t0 < 0)
+    return PM_EINVAL;
+  hipStream_t s = (hipStream_t)stream;
+  const size_t lds = (size_t)16 * d.kp * sizeof(unsigned short);
+  const int nt = net_nt(d, 8, true);
+  int jobs = 0;
+  for (int k = 0; k < d.L; ++k)
+    jobs += ((d.n[k + 1] + kBM - 1) / kBM) * ((d.n[k] + kBN - 1) / kBN + 1);
+  const int ablocks = (int)std::min<int64_t>((d.nP + 255) / 256, 1024);
+  int step = 0;
+  for (int32_t i0 = 0; i0 < rows; i0 += batch_rows, ++step) {
+    int B = std::min(batch_rows, rows - i0);
+    float* x0 = work;
+    float* acts = x0 + (int64_t)batch * B * d.n[0];
+    float* zs = acts + (int64_t)batch * B * d.nhid;
+    float* gr = zs + (int64_t)batch * B * d.nhid;
+    const int64_t* ix = idx + i0;
+    float* ls = loss + (int64_t)step * batch;
+    void* args[] = {&d, &B, &P, &stride_p, &packed, &stride_packed, &X, &T, &ix, &stride_idx, &w,
+                    &x0, &acts, &zs, &gr, &ls};
+    const dim3 grid((B + 15) / 16, batch);
+    int r = nt <= 1   ? net_launch(k_net_train<1>, grid, dim3(512), lds, s, args)
+            : nt <= 2 ? net_launch(k_net_train<2>, grid, dim3(512), lds, s, args)
+                      : net_launch(k_net_train<4>, grid, dim3(512), lds, s, args);
+    if (r) return r;
+    hipLaunchKernelGGL(k_net_grads, dim3(jobs, batch), dim3(256), 0, s, d, B, x0, acts, gr, G,
+                       stride_p);
+    const int32_t t = t0 + step + 1;
+    const float c1 = 1.0f - powf(beta1, (float)t), c2 = 1.0f - powf(beta2, (float)t);
+    hipLaunchKernelGGL(k_net_adam, dim3(ablocks, batch), dim3(256), 0, s, d, P, G, m, v, stride_p,
+                       packed, stride_packed, lr[step], beta1, beta2, eps, weight_decay, c1, c2);
+    r = status();
+    if (r) return r;
+  }
+  return 0;
+}
+
+int pm_mlp_net_stats(void* stream, int32_t members, int64_t n, const float* S, int64_t stride,
+                     float* mean, float* std) {
+  if (members < 1 || n < 0 || !S || !mean || !std) return PM_EINVAL;
+  if (n == 0) return 0;
+  const int blocks = (int)std::min<int64_t>((n + 1023) / 1024, 8192);
+  hipLaunchKernelGGL(k_net_stats, dim3(blocks), dim3(256), 0, (hipStream_t)stream, members, n, S,
+                     stride, mean, std);
   return status();
 }
 

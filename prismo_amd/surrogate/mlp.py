@@ -1,18 +1,20 @@
 """Spectral surrogate: an MLP trained and evaluated by the project's own
 BF16 MFMA kernels (include/pmmlp.h), with FP32 master weights.
 
-Layers: ``n_in -> hidden x depth (GELU) -> n_out``.  Forward: one GEMM per
-layer with the bias and GELU fused into its epilogue (the pre-activations
-are kept for the backward pass).  Backward: per layer one GEMM for the
-weight gradient (dY^T A over the batch), one column sum for the bias
-gradient and one GEMM for the input gradient with the GELU derivative fused
-into its epilogue.  Loss: weighted MSE.  Optimiser: Adam (decoupled weight
-decay) on the FP32 masters; the GEMMs round operands to BF16 as they stage
-them.  ``SurrogateEnsemble`` trains several members from different seeds;
+Layers: ``n_in -> hidden x depth (GELU) -> n_out``.  Networks of up to 12
+layers and 512 units a layer run whole: the forward pass is one launch (a
+workgroup takes its rows through all layers), a training minibatch three
+(forward with loss and backward, all weight and bias gradients, Adam).  Wider
+or deeper ones, and ``backward`` on its own, take one GEMM per layer with the
+bias and GELU (or its derivative) fused into its epilogue.  Loss: weighted
+MSE.  Optimiser: Adam (decoupled weight decay) on the FP32 masters; products
+round their operands to BF16 and sum in FP32.  ``SurrogateEnsemble`` trains several members from different seeds;
 their spread is the predictive uncertainty.
 """
 
 from __future__ import annotations
+
+import ctypes as C
 
 import numpy as np
 
@@ -80,6 +82,30 @@ class SpectralMLP:
         if rc != 0:
             raise N.NativeError(f"{what} failed ({rc})")
 
+    def _net(self):
+        """(layers, widths) for the whole-network kernels, or None when they
+        do not take this network or its parameters are not the views of the
+        flat buffer it was built with."""
+        if self.lib.pm_mlp_net_packed(len(self.shapes), self._widths(), 0) == 0:
+            return None
+        base = self._flat.data_ptr()
+        ow, ob = base, base + 4 * self._nW
+        for (fo, fi), W, b in zip(self.shapes, self.W, self.b):
+            if W.data_ptr() != ow or b.data_ptr() != ob or W.shape != (fo, fi) \
+                    or not W.is_contiguous() or b.shape != (fo,) or not b.is_contiguous():
+                return None
+            ow += 4 * fo * fi
+            ob += 4 * fo
+        return len(self.shapes), self._widths()
+
+    def _widths(self):
+        return (C.c_int32 * len(self.sizes))(*self.sizes)
+
+    def _rows_ok(self, t, width) -> bool:
+        torch = _torch()
+        return (t.dim() == 2 and t.shape[0] > 0 and t.shape[1] == width
+                and t.dtype == torch.float32 and t.device == self.device)
+
     def _gemm(self, mode, M, Nn, K, A, lam, lak, B, lbk, lbn, C, ldc, bias=None, Z=None):
         rc = self.lib.pm_mlp_gemm(self._stream(), mode, M, Nn, K, A.data_ptr(), lam, lak,
                                   B.data_ptr(), lbk, lbn, C.data_ptr(), ldc,
@@ -97,6 +123,9 @@ class SpectralMLP:
         torch = _torch()
         X = X.contiguous()
         M = X.shape[0]
+        net = self._net() if self._rows_ok(X, self.sizes[0]) else None
+        if net is not None:
+            return self._net_forward(net, X, keep)
         acts, zs = [X], []
         a = X
         L = len(self.W)
@@ -115,6 +144,35 @@ class SpectralMLP:
             acts.append(out)
             a = out
         return (a, (acts, zs)) if keep else a
+
+    def _net_forward(self, net, X, keep):
+        torch = _torch()
+        L, widths = net
+        M = X.shape[0]
+        pk = torch.zeros(self.lib.pm_mlp_net_packed(L, widths, 0), dtype=torch.int16,
+                         device=self.device)
+        st = self._stream()
+        self._check(self.lib.pm_mlp_net_pack(st, 1, L, widths, self._flat.data_ptr(), 0,
+                                             pk.data_ptr(), 0, 0), "pm_mlp_net_pack")
+        Y = torch.empty((M, self.sizes[-1]), dtype=torch.float32, device=self.device)
+        hid = self.sizes[1:-1]
+        buf = None
+        if keep:
+            buf = torch.empty((2, M * sum(hid)), dtype=torch.float32, device=self.device)
+        both = keep and bool(hid)
+        self._check(self.lib.pm_mlp_net_forward(
+            st, 1, M, L, widths, self._flat.data_ptr(), 0, pk.data_ptr(), 0, X.data_ptr(), 0,
+            Y.data_ptr(), 0, buf[0].data_ptr() if both else None,
+            buf[1].data_ptr() if both else None, 0), "pm_mlp_net_forward")
+        if not keep:
+            return Y
+        acts, zs = [X], []
+        o = 0
+        for h in hid:
+            acts.append(buf[0][o:o + M * h].view(M, h))
+            zs.append(buf[1][o:o + M * h].view(M, h))
+            o += M * h
+        return Y, (acts + [Y], zs)
 
     def backward(self, cache, dY):
         """Gradients [(dW, db)] of sum(dY * Y), as views of the network's
@@ -198,6 +256,13 @@ class SpectralMLP:
     def _fit_epochs(self, X, T, epochs, batch, lr, w, rng, lr_final, wd, hist):
         torch = _torch()
         M = X.shape[0]
+        run = _net_trainer([self], self._flat, self._gflat, X, T, batch, w)
+        if run is not None:
+            if self._adam is None:
+                self._adam = (torch.zeros_like(self._flat), torch.zeros_like(self._flat))
+            h, self.t = run(self._stream(), self._adam, [rng], epochs, lr, lr_final, wd, self.t)
+            hist.extend(h[0])
+            return
         steps = epochs * ((M + batch - 1) // batch)
         s = 0
         for ep in range(epochs):
@@ -218,14 +283,69 @@ class SpectralMLP:
             hist.append(float(tot.item()) / nb)
 
 
+def _net_trainer(members, P, G, X, T, batch, w):
+    """Training of ``members`` in lockstep by the whole-network kernels, their
+    parameters and gradients the rows of ``P`` and ``G``: a function
+    ``(stream, (m, v), rngs, epochs, lr, lr_final, wd, t) -> (loss history
+    per member, t)``, or None when the kernels do not take this training."""
+    torch = _torch()
+    m0, nm = members[0], len(members)
+    net = m0._net()
+    Pn = P.numel() // nm
+    if net is None or batch < 1 or not (m0._rows_ok(X, m0.sizes[0])
+                                        and m0._rows_ok(T, m0.sizes[-1])
+                                        and T.shape[0] == X.shape[0]):
+        return None
+    if w is not None and (w.dtype != torch.float32 or w.shape != (m0.sizes[-1],)
+                          or not w.is_contiguous() or w.device != m0.device):
+        return None
+    for k, m in enumerate(members):
+        if m._net() is None or m._flat.data_ptr() != P.data_ptr() + 4 * k * Pn \
+                or m._gflat.data_ptr() != G.data_ptr() + 4 * k * Pn:
+            return None
+    L, widths = net
+    lib, dev, M = m0.lib, m0.device, X.shape[0]
+    X, T = X.contiguous(), T.contiguous()
+
+    def run(stream, moments, rngs, epochs, lr, lr_final, wd, t):
+        mA, vA = moments
+        nb = (M + batch - 1) // batch
+        elems = lib.pm_mlp_net_packed(L, widths, 1)
+        pk = torch.zeros((nm, elems), dtype=torch.int16, device=dev)
+        m0._check(lib.pm_mlp_net_pack(stream, nm, L, widths, P.data_ptr(), Pn, pk.data_ptr(),
+                                      elems, 1), "pm_mlp_net_pack")
+        work = torch.empty(nm * lib.pm_mlp_net_work(L, widths, min(batch, M)),
+                           dtype=torch.float32, device=dev)
+        steps, s = epochs * nb, 0
+        hist = [[] for _ in range(nm)]
+        for _ in range(epochs):
+            perm = torch.from_numpy(np.stack([r.permutation(M) for r in rngs])).to(dev)
+            loss = torch.zeros((nb, nm), dtype=torch.float32, device=dev)
+            rates = np.array([lr_final + 0.5 * (lr - lr_final)
+                              * (1 + np.cos(np.pi * (s + i) / max(1, steps)))
+                              for i in range(nb)], dtype=np.float32)
+            m0._check(lib.pm_mlp_net_train(
+                stream, nm, L, widths, P.data_ptr(), G.data_ptr(), mA.data_ptr(), vA.data_ptr(),
+                Pn, pk.data_ptr(), elems, X.data_ptr(), T.data_ptr(), perm.data_ptr(), M,
+                w.data_ptr() if w is not None else None, M, batch, work.data_ptr(),
+                rates.ctypes.data, 0.9, 0.999, 1e-8, wd, t, loss.data_ptr()), "pm_mlp_net_train")
+            s += nb
+            t += nb
+            h = loss.double().sum(0).cpu().numpy()
+            for q in range(nm):
+                hist[q].append(float(h[q]) / nb)
+        return hist, t
+
+    return run
+
+
 class SurrogateEnsemble:
     """Members trained from different seeds on the same data; prediction =
     member mean, uncertainty = member standard deviation.
 
     The members' parameters live in one (members, P) buffer (each member's
     ``SpectralMLP`` views its row), and ``fit`` trains them in lockstep:
-    every GEMM, column sum and loss of a step is one batched launch over the
-    members and Adam one launch over the buffer.  Each member sees what its
+    every launch of a step works on all members.  Each member sees what its
     own ``fit(seed=k)`` would (same initial weights, same minibatch order):
     the parameters come out the same."""
 
@@ -261,6 +381,12 @@ class SurrogateEnsemble:
         steps = epochs * ((M + batch - 1) // batch)
         if self._adam is None:
             self._adam = (torch.zeros_like(self.P), torch.zeros_like(self.P))
+        run = _net_trainer(self.members, self.P, self.G, X, T, batch, w)
+        if run is not None:
+            hist, self.t = run(st, self._adam, rngs, epochs, lr, lr_final, wd, self.t)
+            for m in self.members:
+                m.t = self.t
+            return hist
         mA, vA = self._adam
         P0, G0 = self.P.data_ptr(), self.G.data_ptr()
         f4 = 4  # bytes per element
@@ -339,9 +465,35 @@ class SurrogateEnsemble:
 
     def predict(self, X, chunk: int = 16384):
         torch = _torch()
+        m0, nm, Pn = self.members[0], len(self.members), self.P.shape[1]
+        if m0._rows_ok(X, m0.sizes[0]) and all(
+                m._net() is not None and m._flat.data_ptr() == self.P.data_ptr() + 4 * k * Pn
+                for k, m in enumerate(self.members)):
+            return self._net_predict(X.contiguous())
         outs = []
         for m in self.members:
             parts = [m.forward(X[i:i + chunk]) for i in range(0, X.shape[0], chunk)]
             outs.append(torch.cat(parts))
         S = torch.stack(outs)
         return S.mean(0), S.std(0)
+
+    def _net_predict(self, X):
+        """All members' outputs in one launch, then their mean and spread."""
+        torch = _torch()
+        m0, nm, Pn = self.members[0], len(self.members), self.P.shape[1]
+        L, widths = m0._net()
+        M, no = X.shape[0], m0.sizes[-1]
+        st = m0._stream()
+        elems = self.lib.pm_mlp_net_packed(L, widths, 0)
+        pk = torch.zeros((nm, elems), dtype=torch.int16, device=self.device)
+        self._check(self.lib.pm_mlp_net_pack(st, nm, L, widths, self.P.data_ptr(), Pn,
+                                             pk.data_ptr(), elems, 0), "pm_mlp_net_pack")
+        S = torch.empty((nm, M, no), dtype=torch.float32, device=self.device)
+        self._check(self.lib.pm_mlp_net_forward(
+            st, nm, M, L, widths, self.P.data_ptr(), Pn, pk.data_ptr(), elems, X.data_ptr(), 0,
+            S.data_ptr(), M * no, None, None, 0), "pm_mlp_net_forward")
+        out = torch.empty((2, M, no), dtype=torch.float32, device=self.device)
+        self._check(self.lib.pm_mlp_net_stats(st, nm, M * no, S.data_ptr(), M * no,
+                                              out[0].data_ptr(), out[1].data_ptr()),
+                    "pm_mlp_net_stats")
+        return out[0], out[1]

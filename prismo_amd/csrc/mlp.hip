@@ -26,6 +26,7 @@ namespace pm {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBM = 64, kBN = 64, kBK = 128, kPad = 8;
@@ -39,8 +40,27 @@ __device__ __forceinline__ unsigned short to_bf16(float x) {
   return (unsigned short)(u >> 16);
 }
 
+// gelu(z) = z Phi(z) = max(z, 0) - t Q(t), t = |z|, with the normal tail
+// Q(t) = exp(-t^2 / 2) R(t) and R = erfcx(t / sqrt 2) / 2 a polynomial in
+// u = 1 / (1 + p t) (the form of Abramowitz & Stegun 7.1.26; p and the seven
+// coefficients fitted here to R in least squares reweighted towards the
+// largest error, 3e-9 in t Q).  One exp2 and one reciprocal without a branch,
+// where erff takes both of its branches on a mixed wave: screening 65 536
+// rows spent a third of its time there.  RMS error over z ~ N(0, 2) 3.7e-8,
+// 4.9e-8 for z (1 + erff(z / sqrt 2)) / 2.  NaN stays NaN, +inf stays +inf
+// (t is held to 16), -inf gives NaN as that product does.
 __device__ __forceinline__ float gelu(float z) {
-  return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f));
+  const float t = fabsf(fminf(z, 16.0f));
+  const float u = __builtin_amdgcn_rcpf(fmaf(0.33f, t, 1.0f));
+  float r = 0.0445816509797629f;
+  r = fmaf(r, u, -0.21599956951883484f);
+  r = fmaf(r, u, 0.3222291694117826f);
+  r = fmaf(r, u, -0.0799483629557832f);
+  r = fmaf(r, u, 0.17562644735107985f);
+  r = fmaf(r, u, 0.12110024391227908f);
+  r = fmaf(r, u, 0.13241042378950282f);
+  const float q = r * u * __builtin_amdgcn_exp2f(t * t * -0.72134752044448170f);
+  return fmaf(-t, q, z < 0.0f ? 0.0f : z);
 }
 
 // d gelu / dz = Phi(z) + z phi(z)
@@ -295,6 +315,10 @@ struct NetDesc {
   int64_t nW, nP;                    // weights, parameters
   int64_t nfwd, npack;               // packed elements without / with the transposes
   int64_t nhid, ngrad;               // values per row over hidden / all layers
+  // training workspace, widths padded to 16: pre-activations (zpad values a
+  // row, layer k from zpo[k]), inputs, gradients
+  int64_t zpad, apad, gpad;
+  int64_t zpo[kNetL], apo[kNetL], gpo[kNetL];
   int kp;                            // LDS row: widest padded operand + 8
 };
 
@@ -334,52 +358,107 @@ __global__ __launch_bounds__(256) void k_net_pack(const NetDesc d, const float* 
 
 extern __shared__ unsigned short net_lds[];
 
-// acc += A B over K (padded to 32) for this wave's tiles; A from LDS rows,
-// B from the packed weights, the next K-step's loads in flight.
-template <int RT, int NT, int WC>
-__device__ __forceinline__ void net_gemm(const unsigned short* sA, int kp, int row0, int wc,
-                                         int ntiles, int K, const unsigned short* __restrict__ pk,
-                                         f32x4 (&acc)[RT][NT]) {
-  const int lane = threadIdx.x & 63;
-  const int li = lane & 15, lq = lane >> 4;
-  const int kt = up32(K) / 32;
-  bf16x8 bn[NT];
-  const unsigned short* bp[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
+__device__ __forceinline__ bf16x4 to_bf16x4(f32x4 v) { return __builtin_convertvector(v, bf16x4); }
+
+// The wave's weight tiles of PD K-steps, in flight ahead of the products that
+// take them: a K-step's loads wait for L2 or the Infinity Cache (the weights
+// were just written by other XCDs), 1 to 2 us against 0.1 us of MFMA.
+template <int NT, int WC, int PD>
+struct NetTiles {
+  bf16x8 b[PD][NT];
+  __device__ __forceinline__ static bf16x8 at(const unsigned short* pk, int wc, int t, int ntiles,
+                                              int kt, int s) {
     // tiles past the layer's width repeat the last one (unused)
     const int nt = min(t * WC + wc, ntiles - 1);
-    bp[t] = pk + ((int64_t)nt * kt * 64 + lane) * 8;
-    bn[t] = *(const bf16x8*)bp[t];
+    const unsigned short* base = pk + ((int64_t)nt * kt + s) * 512;  // uniform
+    return *(const bf16x8*)(base + 8 * (threadIdx.x & 63));
+  }
+  __device__ __forceinline__ void fill(const unsigned short* pk, int wc, int N, int K) {
+    const int kt = up32(K) / 32, ntiles = up16(N) / 16;
+#pragma unroll
+    for (int p = 0; p < PD; ++p)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b[p][t] = at(pk, wc, t, ntiles, kt, min(p, kt - 1));
+  }
+};
+
+// acc = W A over K (padded to 32) for this wave's tiles: weights from the packed
+// buffer (first K-steps already in w), activations from LDS rows.  The weights
+// are the row operand, so a lane holds 4 consecutive columns (16 tile + 4 lq + e)
+// of one activation row (row0 + 16 r + li): one 8-byte LDS store and one 16-byte
+// memory store where the other order takes four of each.
+template <int RT, int NT, int WC, int PD>
+__device__ __forceinline__ void net_gemm(const unsigned short* sA, int kp, int row0, int wc, int N,
+                                         int K, const unsigned short* __restrict__ pk,
+                                         NetTiles<NT, WC, PD>& w, f32x4 (&acc)[RT][NT]) {
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int kt = up32(K) / 32, ntiles = up16(N) / 16;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][t] = f32x4{0, 0, 0, 0};
-  }
   const unsigned short* ap = sA + (row0 + li) * kp + 8 * lq;
-  for (int s = 0; s < kt; ++s) {
-    bf16x8 bv[NT], av[RT];
+  for (int s0 = 0; s0 < kt; s0 += PD) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      bv[t] = bn[t];
-      bp[t] += s + 1 < kt ? 512 : 0;
-      bn[t] = *(const bf16x8*)bp[t];
+    for (int p = 0; p < PD; ++p) {
+      const int s = s0 + p;
+      if (s < kt) {
+        bf16x8 wv[NT], av[RT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          wv[t] = w.b[p][t];
+          // this slot's next K-step, or, when the layer fits the slots, the
+          // matrix the slots serve next
+          if (s + PD < kt) w.b[p][t] = w.at(pk, wc, t, ntiles, kt, s + PD);
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) av[r] = *(const bf16x8*)(ap + 16 * r * kp + 32 * s);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t], av[r], acc[r][t], 0, 0, 0);
+      }
     }
-#pragma unroll
-    for (int r = 0; r < RT; ++r) av[r] = *(const bf16x8*)(ap + 16 * r * kp + 32 * s);
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[r], bv[t], acc[r][t], 0, 0, 0);
   }
 }
 
+// Values n .. n+3 of a row of N (beyond N the last one: the caller does not use
+// them).
+__device__ __forceinline__ f32x4 load4(const float* p, int n, int N) {
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = p[min(n + e, N - 1)];
+  return v;
+}
+
+// All biases of a member into LDS behind the activation rows: read from memory
+// in the epilogue they would wait for the next layer's weights, issued before
+// them (vector loads return in order).
+__device__ __forceinline__ float* net_biases(unsigned short* sA, int rows, const NetDesc& d,
+                                             const float* __restrict__ Pq) {
+  float* sb = (float*)(sA + rows * d.kp);
+  for (int f = threadIdx.x; f < (int)d.ngrad; f += blockDim.x) sb[f] = Pq[d.nW + f];
+  return sb;
+}
+
+// The same stored; vec: rows are 16-byte aligned.
+__device__ __forceinline__ void store4(float* p, int n, int N, bool vec, f32x4 v) {
+  if (vec) {
+    if (n < N) *(f32x4*)(p + n) = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n + e < N) p[n + e] = v[e];
+}
+
 // Rows m0 .. of src (row stride ld, through idx when given) into LDS as BF16,
-// zero beyond the rows and beyond column n up to a multiple of 32; copy keeps
-// the gathered values.
+// zero beyond the rows and beyond column n up to a multiple of 32.
 __device__ __forceinline__ void net_stage(unsigned short* sA, int kp, int bm, int m0, int M,
                                           int n, const float* __restrict__ src, int64_t ld,
-                                          const int64_t* __restrict__ idx,
-                                          float* __restrict__ copy) {
+                                          const int64_t* __restrict__ idx) {
   const int np = up32(n);
   for (int f = threadIdx.x; f < bm * np; f += blockDim.x) {
     const int r = f / np, c = f - r * np;
@@ -387,7 +466,6 @@ __device__ __forceinline__ void net_stage(unsigned short* sA, int kp, int bm, in
     if (m0 + r < M && c < n) {
       const int64_t row = idx ? idx[m0 + r] : m0 + r;
       v = src[row * ld + c];
-      if (copy) copy[(int64_t)(m0 + r) * n + c] = v;
     }
     sA[r * kp + c] = to_bf16(v);
   }
@@ -396,8 +474,11 @@ __device__ __forceinline__ void net_stage(unsigned short* sA, int kp, int bm, in
 // Y = network(X) for rows of every member (blockIdx.y); hidden activations and
 // pre-activations kept in acts / zs (member stride as_, layer k at M aoff[k])
 // when given.
-template <int RT, int NT, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC) void k_net_forward(
+//
+// Two workgroups of the tall shape share a CU (128 VGPRs): one's products run
+// beside the other's epilogue.
+template <int RT, int NT, int WR, int WC, int PD>
+__global__ __launch_bounds__(64 * WR * WC, RT == 4 && NT == 4 ? 4 : 1) void k_net_forward(
     const NetDesc d, int M, const float* __restrict__ P, int64_t ps,
     const unsigned short* __restrict__ pk, int64_t ks, const float* __restrict__ X, int64_t xs,
     float* __restrict__ Y, int64_t ys, float* __restrict__ acts, float* __restrict__ zs,
@@ -411,55 +492,103 @@ __global__ __launch_bounds__(64 * WR * WC) void k_net_forward(
   const int wr = wv / WC, wc = wv % WC;
   const int m0 = blockIdx.x * BM, row0 = wr * 16 * RT;
   const float* Pq = P + q * ps;
-  net_stage(sA, d.kp, BM, m0, M, d.n[0], X + q * xs, d.n[0], nullptr, nullptr);
+  const unsigned short* pq = pk + q * ks;
+  Y += q * ys;
+  const bool yvec = d.n[d.L] % 4 == 0 && ((uintptr_t)Y & 15) == 0;
+  NetTiles<NT, WC, PD> w;
+  w.fill(pq + d.poff[0], wc, d.n[1], d.n[0]);
+  net_stage(sA, d.kp, BM, m0, M, d.n[0], X + q * xs, d.n[0], nullptr);
+  const float* sb = net_biases(sA, BM, d, Pq);
   __syncthreads();
   for (int k = 0; k < d.L; ++k) {
     const int K = d.n[k], N = d.n[k + 1];
     f32x4 acc[RT][NT];
-    net_gemm<RT, NT, WC>(sA, d.kp, row0, wc, up16(N) / 16, K, pk + q * ks + d.poff[k], acc);
+    net_gemm<RT, NT, WC, PD>(sA, d.kp, row0, wc, N, K, pq + d.poff[k], w, acc);
     const bool last = k + 1 == d.L;
+    // the next layer's first weights come in during the epilogue
+    if (!last) w.fill(pq + d.poff[k + 1], wc, d.n[k + 2], N);
     __syncthreads();  // every wave has read its operands: the rows are replaced
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int n = 16 * (t * WC + wc) + li;
+      const int n = 16 * (t * WC + wc) + 4 * lq;
       if (16 * (t * WC + wc) >= up32(N)) continue;
-      const float bias = n < N ? Pq[d.boff[k] + n] : 0.0f;
+      const f32x4 bias = load4(sb + d.goff[k], n, N);
 #pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = row0 + 16 * r + 4 * lq + e;
-          const int m = m0 + row;
-          const float z = acc[r][t][e] + bias;
-          if (last) {
-            if (n < N && m < M) Y[q * ys + (int64_t)m * N + n] = z;
-            continue;
-          }
-          const float a = n < N ? gelu(z) : 0.0f;
-          sA[row * d.kp + n] = to_bf16(a);
-          if (zs && n < N && m < M) {
-            const int64_t o = q * as_ + (int64_t)M * d.aoff[k] + (int64_t)m * N + n;
-            zs[o] = z;
-            acts[o] = a;
-          }
+      for (int r = 0; r < RT; ++r) {
+        const int row = row0 + 16 * r + li, m = m0 + row;
+        const f32x4 z = acc[r][t] + bias;
+        if (last) {
+          if (m < M) store4(Y + (int64_t)m * N, n, N, yvec, z);
+          continue;
         }
+        f32x4 a;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = n + e < N ? gelu(z[e]) : 0.0f;
+        *(bf16x4*)(sA + row * d.kp + n) = to_bf16x4(a);
+        if (zs && m < M) {
+          const int64_t o = q * as_ + (int64_t)M * d.aoff[k] + (int64_t)m * N;
+          store4(zs + o, n, N, false, z);
+          store4(acts + o, n, N, false, a);
+        }
+      }
     }
     __syncthreads();
   }
 }
 
-// One training batch of every member (blockIdx.y), 16 rows per workgroup:
+// Workspace of one training minibatch (rows padded to B32, a multiple of 32):
+// pre-activations (row stride up16), the layers' inputs and output gradients as
+// BF16 in the operand order of the weight gradients (K = row), and each
+// 16-row block's column sums of the gradients.
+struct NetWork {
+  float* zs;
+  unsigned short* a;
+  unsigned short* g;
+  float* part;
+};
+
+__host__ __device__ inline int64_t net_work_floats(const NetDesc& d, int B32) {
+  return B32 * (d.zpad + d.apad / 2 + d.gpad / 2) + (B32 / 16) * d.ngrad;
+}
+
+__device__ __forceinline__ NetWork net_work(const NetDesc& d, float* work, int64_t q, int B32) {
+  float* p = work + q * ((net_work_floats(d, B32) + 3) & ~3ll);
+  NetWork w;
+  w.zs = p;
+  p += B32 * d.zpad;
+  w.a = (unsigned short*)p;
+  p += B32 * (d.apad / 2);
+  w.g = (unsigned short*)p;
+  p += B32 * (d.gpad / 2);
+  w.part = p;
+  return w;
+}
+
+// The 16 LDS rows (block m0) of width N as operand tiles with K = row.
+__device__ __forceinline__ void net_rows_out(const unsigned short* sA, int kp, int N, int m0,
+                                             int B32, unsigned short* __restrict__ dst) {
+  const int kt = B32 / 32;
+  for (int f = threadIdx.x; f < 2 * up16(N); f += blockDim.x) {
+    const int n = f >> 1, h = f & 1;
+    typedef unsigned short us8 __attribute__((ext_vector_type(8)));
+    us8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = sA[(8 * h + e) * kp + n];
+    const int lane = (n & 15) + 16 * (((m0 >> 3) & 3) + h);
+    *(us8*)(dst + (((int64_t)(n >> 4) * kt + (m0 >> 5)) * 64 + lane) * 8) = v;
+  }
+}
+
+// One training minibatch of every member (blockIdx.y), 16 rows per workgroup:
 // forward, the weighted squared error's gradient and loss, and the gradient
-// carried back to the first hidden layer.  Rows are gathered through idx;
-// acts (the gathered inputs, then the hidden activations), pre-activations and
-// output gradients of every layer go to the workspace for k_net_grads.
-template <int NT>
+// carried back to the first hidden layer.  Rows are gathered through idx; rows
+// from B to B32 have zero gradients.
+template <int NT, int PD>
 __global__ __launch_bounds__(512) void k_net_train(
-    const NetDesc d, int B, const float* __restrict__ P, int64_t ps,
+    const NetDesc d, int B, int B32, const float* __restrict__ P, int64_t ps,
     const unsigned short* __restrict__ pk, int64_t ks, const float* __restrict__ X,
     const float* __restrict__ T, const int64_t* __restrict__ idx, int64_t is,
-    const float* __restrict__ w, float* __restrict__ x0, float* __restrict__ acts,
-    float* __restrict__ zs, float* __restrict__ G, float* __restrict__ loss) {
+    const float* __restrict__ wcol, float* __restrict__ work, float* __restrict__ loss) {
   constexpr int WC = 8;
   unsigned short* sA = net_lds;
   __shared__ float red[8];
@@ -467,80 +596,103 @@ __global__ __launch_bounds__(512) void k_net_train(
   const int lane = threadIdx.x & 63;
   const int li = lane & 15, lq = lane >> 4;
   const int wc = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m0 = blockIdx.x * 16;
+  const int m0 = blockIdx.x * 16, m = m0 + li;
   const float* Pq = P + q * ps;
   const unsigned short* pq = pk + q * ks;
   idx += q * is;
-  x0 += q * (int64_t)B * d.n[0];
-  acts += q * (int64_t)B * d.nhid;
-  zs += q * (int64_t)B * d.nhid;
-  G += q * (int64_t)B * d.ngrad;
-  net_stage(sA, d.kp, 16, m0, B, d.n[0], X, d.n[0], idx, x0);
+  const NetWork W = net_work(d, work, q, B32);
+  float* part = W.part + (int64_t)blockIdx.x * d.ngrad;
+  NetTiles<NT, WC, PD> w;
+  w.fill(pq + d.poff[0], wc, d.n[1], d.n[0]);
+  net_stage(sA, d.kp, 16, m0, B, d.n[0], X, d.n[0], idx);
+  const float* sb = net_biases(sA, 16, d, Pq);
+  const int64_t trow = m < B ? idx[m] : 0;
   __syncthreads();
+  net_rows_out(sA, d.kp, d.n[0], m0, B32, W.a + (int64_t)B32 * d.apo[0]);
   const int NL = d.n[d.L];
   const float scale = 1.0f / (float)((int64_t)B * NL);
   float s = 0.0f;
+  // column sums over the block's rows (the 16 lanes of a quarter wave)
+  auto rows16 = [&](f32x4 v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 1; h < 16; h *= 2)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], h);
+    return v;
+  };
   for (int k = 0; k < d.L; ++k) {
     const int K = d.n[k], N = d.n[k + 1];
     f32x4 acc[1][NT];
-    net_gemm<1, NT, WC>(sA, d.kp, 0, wc, up16(N) / 16, K, pq + d.poff[k], acc);
+    net_gemm<1, NT, WC, PD>(sA, d.kp, 0, wc, N, K, pq + d.poff[k], w, acc);
     const bool last = k + 1 == d.L;
+    // targets ahead of the weights that the backward pass starts with
+    f32x4 y[NT], wt[NT];
+    if (last) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int n = min(16 * (t * WC + wc) + 4 * lq, N - 1);
+        y[t] = load4(T + trow * NL, n, N);
+        wt[t] = wcol ? load4(wcol, n, N) : f32x4{1, 1, 1, 1};
+      }
+    }
+    if (!last) w.fill(pq + d.poff[k + 1], wc, d.n[k + 2], N);
+    else if (k > 0) w.fill(pq + d.qoff[k], wc, d.n[k], N);
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int n = 16 * (t * WC + wc) + li;
+      const int n = 16 * (t * WC + wc) + 4 * lq;
       if (16 * (t * WC + wc) >= up32(N)) continue;
-      const float bias = n < N ? Pq[d.boff[k] + n] : 0.0f;
-      const float wt = last && w && n < N ? w[n] : 1.0f;
+      const f32x4 z = acc[0][t] + load4(sb + d.goff[k], n, N);
+      f32x4 v = {0, 0, 0, 0};
+      if (last) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = 4 * lq + e, m = m0 + row;
-        const bool ok = n < N && m < B;
-        const float z = acc[0][t][e] + bias;
-        float v = 0.0f;
-        if (last) {
-          if (ok) {
-            const float dd = z - T[idx[m] * NL + n];
-            s += wt * dd * dd;
-            v = 2.0f * wt * dd * scale;
-            G[(int64_t)B * d.goff[k] + (int64_t)m * N + n] = v;
-          }
-        } else if (n < N) {
-          v = gelu(z);
-          if (ok) {
-            const int64_t o = (int64_t)B * d.aoff[k] + (int64_t)m * N + n;
-            zs[o] = z;
-            acts[o] = v;
-          }
+        for (int e = 0; e < 4; ++e) {
+          if (n + e >= N || m >= B) continue;
+          const float dd = z[e] - y[t][e];
+          s += wt[t][e] * dd * dd;
+          v[e] = 2.0f * wt[t][e] * dd * scale;
         }
-        sA[row * d.kp + n] = to_bf16(v);
+        const f32x4 sum = rows16(v);
+        if (li == 0) store4(part + d.goff[k], n, N, false, sum);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = n + e < N ? gelu(z[e]) : 0.0f;
+        if (n < up16(N))
+          *(f32x4*)(W.zs + B32 * d.zpo[k] + (int64_t)m * up16(N) + n) = z;
       }
+      *(bf16x4*)(sA + li * d.kp + n) = to_bf16x4(v);
     }
     __syncthreads();
+    net_rows_out(sA, d.kp, N, m0, B32,
+                 last ? W.g + (int64_t)B32 * d.gpo[k] : W.a + (int64_t)B32 * d.apo[k + 1]);
   }
   // back through the layers: G_{k-1} = (G_k W_k) gelu'(z_{k-1})
   for (int k = d.L - 1; k > 0; --k) {
     const int K = d.n[k + 1], N = d.n[k];
-    f32x4 acc[1][NT];
-    net_gemm<1, NT, WC>(sA, d.kp, 0, wc, up16(N) / 16, K, pq + d.qoff[k], acc);
+    f32x4 acc[1][NT], z[NT];
+    // this thread stored these pre-activations in the forward pass
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = min(16 * (t * WC + wc) + 4 * lq, up16(N) - 4);
+      z[t] = *(const f32x4*)(W.zs + B32 * d.zpo[k - 1] + (int64_t)m * up16(N) + n);
+    }
+    net_gemm<1, NT, WC, PD>(sA, d.kp, 0, wc, N, K, pq + d.qoff[k], w, acc);
+    if (k > 1) w.fill(pq + d.qoff[k - 1], wc, d.n[k - 1], N);
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int n = 16 * (t * WC + wc) + li;
+      const int n = 16 * (t * WC + wc) + 4 * lq;
       if (16 * (t * WC + wc) >= up32(N)) continue;
+      f32x4 v = {0, 0, 0, 0};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = 4 * lq + e, m = m0 + row;
-        float v = 0.0f;
-        if (n < N && m < B) {
-          // this thread wrote the pre-activation in the forward pass
-          v = acc[0][t][e] * dgelu(zs[(int64_t)B * d.aoff[k - 1] + (int64_t)m * N + n]);
-          G[(int64_t)B * d.goff[k - 1] + (int64_t)m * N + n] = v;
-        }
-        sA[row * d.kp + n] = to_bf16(v);
-      }
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N && m < B) v[e] = acc[0][t][e] * dgelu(z[t][e]);
+      const f32x4 sum = rows16(v);
+      if (li == 0) store4(part + d.goff[k - 1], n, N, false, sum);
+      *(bf16x4*)(sA + li * d.kp + n) = to_bf16x4(v);
     }
     __syncthreads();
+    net_rows_out(sA, d.kp, N, m0, B32, W.g + (int64_t)B32 * d.gpo[k - 1]);
   }
   for (int h = 32; h >= 1; h >>= 1) s += __shfl_xor(s, h);
   if (lane == 0) red[wc] = s;
@@ -552,84 +704,177 @@ __global__ __launch_bounds__(512) void k_net_train(
   }
 }
 
-// Weight gradients (64 x 64 tiles of G_k^T a_k) and bias gradients (column
-// sums) of all layers, one launch.
-__global__ __launch_bounds__(256) void k_net_grads(const NetDesc d, int B,
-                                                   const float* __restrict__ x0,
-                                                   const float* __restrict__ acts,
-                                                   const float* __restrict__ G,
-                                                   float* __restrict__ gP, int64_t ps) {
-  __shared__ GemmLds lds;
-  __shared__ float part[4][64];
+struct AdamArgs {
+  float lr, b1, b2, eps, wd, c1, c2;
+};
+
+// k_adam's update of one parameter.
+__device__ __forceinline__ float adam_one(const AdamArgs& h, float g, float wd, float p, float& m,
+                                          float& v) {
+  m = h.b1 * m + (1.0f - h.b1) * g;
+  v = h.b2 * v + (1.0f - h.b2) * g * g;
+  const float mh = m / h.c1, vh = v / h.c2;
+  return p - h.lr * (mh / (sqrtf(vh) + h.eps) + wd * p);
+}
+
+// Weight gradients G_k^T a_k (64 x 64 tiles, operands straight from the
+// workspace, no LDS), bias gradients (the blocks' column sums added up) and
+// Adam on the parameters they belong to, with the packed copies of the new
+// weights: one launch for all layers and members, the gradients and moments
+// of a tile in registers throughout.
+__global__ __launch_bounds__(256) void k_net_update(const NetDesc d, int B32,
+                                                    float* __restrict__ work,
+                                                    float* __restrict__ P, float* __restrict__ G,
+                                                    float* __restrict__ mm,
+                                                    float* __restrict__ vv, int64_t ps,
+                                                    unsigned short* __restrict__ pk, int64_t ks,
+                                                    AdamArgs h) {
   const int64_t q = blockIdx.y;
-  G += q * (int64_t)B * d.ngrad;
-  gP += q * ps;
+  const NetWork W = net_work(d, work, q, B32);
+  P += q * ps;
+  G += q * ps;
+  mm += q * ps;
+  vv += q * ps;
+  pk += q * ks;
   int b = blockIdx.x;
-  for (int k = 0; k < d.L; ++k) {
-    const int fi = d.n[k], fo = d.n[k + 1];
-    const int gx = (fi + kBN - 1) / kBN, gy = (fo + kBM - 1) / kBM;
-    const float* g = G + (int64_t)B * d.goff[k];
-    if (b < gx * gy) {
-      const float* a = k == 0 ? x0 + q * (int64_t)B * fi
-                              : acts + q * (int64_t)B * d.nhid + (int64_t)B * d.aoff[k - 1];
-      gemm_tile(PM_MLP_PLAIN, fo, fi, B, g, 1, fo, a, fi, 1, gP + d.woff[k], fi, nullptr, nullptr,
-                (b / gx) * kBM, (b % gx) * kBN, lds);
-      return;
-    }
-    b -= gx * gy;
-    if (b < gy) {
-      colsum_tile(B, fo, g, fo, gP + d.boff[k], b * 64, part);
-      return;
-    }
-    b -= gy;
+  int k = 0, gx = 0;
+  for (; k < d.L; ++k) {
+    gx = (d.n[k] + 63) / 64;
+    const int jobs = gx * ((d.n[k + 1] + 63) / 64) + 1;
+    if (b < jobs) break;
+    b -= jobs;
   }
+  if (k >= d.L) return;
+  const int fi = d.n[k], fo = d.n[k + 1];
+  if (b == 0) {
+    for (int n = threadIdx.x; n < fo; n += 256) {
+      float s = 0.0f;
+      for (int i = 0; i < B32 / 16; ++i) s += W.part[(int64_t)i * d.ngrad + d.goff[k] + n];
+      const int64_t o = d.boff[k] + n;
+      float m = mm[o], v = vv[o];
+      G[o] = s;
+      P[o] = adam_one(h, s, 0.0f, P[o], m, v);
+      mm[o] = m;
+      vv[o] = v;
+    }
+    return;
+  }
+  b -= 1;
+  constexpr int PD = 8;  // a minibatch of 256 rows is all in flight at once
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o0 = (b / gx) * 64 + (wv >> 1) * 32, i0 = (b % gx) * 64 + (wv & 1) * 32;
+  if (o0 >= fo || i0 >= fi) return;
+  const int kt = B32 / 32;
+  const unsigned short* ga = W.g + (int64_t)B32 * d.gpo[k] + 8 * lane;
+  const unsigned short* aa = W.a + (int64_t)B32 * d.apo[k] + 8 * lane;
+  // tiles past the layer repeat its last one (unused)
+  int64_t go[2], ao[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    go[t] = (int64_t)min(o0 / 16 + t, up16(fo) / 16 - 1) * kt * 512;
+    ao[t] = (int64_t)min(i0 / 16 + t, up16(fi) / 16 - 1) * kt * 512;
+  }
+  bf16x8 gv[PD][2], av[PD][2];
+#pragma unroll
+  for (int p = 0; p < PD; ++p)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      gv[p][t] = *(const bf16x8*)(ga + go[t] + min(p, kt - 1) * 512);
+      av[p][t] = *(const bf16x8*)(aa + ao[t] + min(p, kt - 1) * 512);
+    }
+  // the tile's parameters and moments, behind the operands (loads return in
+  // order); lane: rows o = 4 lq + e, column i = li of each 16 x 16 tile
+  f32x4 acc[2][2], pv[2][2], mv[2][2], vm[2][2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      acc[r][c] = f32x4{0, 0, 0, 0};
+      const int i = min(i0 + 16 * c + li, fi - 1), ob = o0 + 16 * r + 4 * lq;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t o = d.woff[k] + (int64_t)min(ob + e, fo - 1) * fi + i;
+        pv[r][c][e] = P[o];
+        mv[r][c][e] = mm[o];
+        vm[r][c][e] = vv[o];
+      }
+    }
+  for (int s0 = 0; s0 < kt; s0 += PD) {
+#pragma unroll
+    for (int p = 0; p < PD; ++p) {
+      const int s = s0 + p;
+      if (s < kt) {
+        const bf16x8 g0 = gv[p][0], g1 = gv[p][1], a0 = av[p][0], a1 = av[p][1];
+        if (s + PD < kt) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            gv[p][t] = *(const bf16x8*)(ga + go[t] + (s + PD) * 512);
+            av[p][t] = *(const bf16x8*)(aa + ao[t] + (s + PD) * 512);
+          }
+        }
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g0, a0, acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g0, a1, acc[0][1], 0, 0, 0);
+        acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g1, a0, acc[1][0], 0, 0, 0);
+        acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g1, a1, acc[1][1], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int i = i0 + 16 * c + li, ob = o0 + 16 * r + 4 * lq;
+      if (i >= fi) continue;
+      float pn[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float m = mv[r][c][e], v = vm[r][c][e];
+        pn[e] = adam_one(h, acc[r][c][e], h.wd, pv[r][c][e], m, v);
+        if (ob + e >= fo) continue;
+        const int64_t o = d.woff[k] + (int64_t)(ob + e) * fi + i;
+        G[o] = acc[r][c][e];
+        P[o] = pn[e];
+        mm[o] = m;
+        vv[o] = v;
+        pk[d.poff[k] + pack_at(ob + e, i, fi)] = to_bf16(pn[e]);
+      }
+      if (k > 0) {
+        unsigned short* qp = pk + d.qoff[k] + pack_at(i, ob, fo);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (ob + e < fo) qp[e] = to_bf16(pn[e]);
+      }
+    }
 }
 
-// k_adam's update on every member's parameters (decay on the weights only),
-// with the packed copies of the new weights.
-__global__ __launch_bounds__(256) void k_net_adam(const NetDesc d, float* __restrict__ p,
-                                                  const float* __restrict__ g,
-                                                  float* __restrict__ m, float* __restrict__ v,
-                                                  int64_t ps, unsigned short* __restrict__ pk,
-                                                  int64_t ks, float lr, float b1, float b2,
-                                                  float eps, float wd, float c1, float c2) {
-  const int64_t q = blockIdx.y;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < d.nP;
-       e += (int64_t)gridDim.x * 256) {
-    const int64_t o = q * ps + e;
-    const float gi = g[o];
-    const float mi = b1 * m[o] + (1.0f - b1) * gi;
-    const float vi = b2 * v[o] + (1.0f - b2) * gi * gi;
-    m[o] = mi;
-    v[o] = vi;
-    const float mh = mi / c1, vh = vi / c2;
-    const float pe = p[o];
-    const float pn = pe - lr * (mh / (sqrtf(vh) + eps) + (e < d.nW ? wd : 0.0f) * pe);
-    p[o] = pn;
-    if (e < d.nW) pack_weight(d, pk + q * ks, e, pn, true);
-  }
-}
-
-// Mean and standard deviation (divisor nm - 1) over the members' values.
+// Mean and standard deviation (divisor nm - 1) over the members' values, four
+// per thread; vec: every row of S and both outputs are 16-byte aligned.
 __global__ __launch_bounds__(256) void k_net_stats(int nm, int64_t n, const float* __restrict__ S,
                                                    int64_t ss, float* __restrict__ mean,
-                                                   float* __restrict__ sd) {
+                                                   float* __restrict__ sd, int vec) {
   for (int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; e < n;
        e += (int64_t)gridDim.x * 1024) {
     const int c = (int)min((int64_t)4, n - e);
-    float a[4] = {0, 0, 0, 0}, v[4] = {0, 0, 0, 0};
-    for (int q = 0; q < nm; ++q)
-      for (int i = 0; i < c; ++i) a[i] += S[q * ss + e + i];
-    for (int i = 0; i < 4; ++i) a[i] /= (float)nm;
-    for (int q = 0; q < nm; ++q)
-      for (int i = 0; i < c; ++i) {
-        const float t = S[q * ss + e + i] - a[i];
-        v[i] += t * t;
-      }
-    for (int i = 0; i < c; ++i) {
-      mean[e + i] = a[i];
-      sd[e + i] = sqrtf(v[i] / (float)(nm - 1));
+    auto get = [&](int q) __attribute__((always_inline)) {
+      const float* p = S + q * ss + e;
+      if (vec && c == 4) return *(const f32x4*)p;
+      return load4(p, 0, c);
+    };
+    f32x4 a = {0, 0, 0, 0}, v = {0, 0, 0, 0};
+    for (int q = 0; q < nm; ++q) a += get(q);
+    a /= (float)nm;
+    for (int q = 0; q < nm; ++q) {
+      const f32x4 t = get(q) - a;
+      v += t * t;
     }
+    v /= (float)(nm - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = sqrtf(v[i]);
+    const bool w = vec && c == 4;
+    store4(mean + e, 0, c, w, a);
+    store4(sd + e, 0, c, w, v);
   }
 }
 
@@ -653,6 +898,12 @@ bool net_desc(int L, const int32_t* n, NetDesc* out) {
     if (k + 1 < L) a += n[k + 1];
     d.goff[k] = g;
     g += n[k + 1];
+    d.apo[k] = d.apad;
+    d.apad += up16(n[k]);
+    d.gpo[k] = d.gpad;
+    d.gpad += up16(n[k + 1]);
+    d.zpo[k] = d.zpad;
+    if (k + 1 < L) d.zpad += up16(n[k + 1]);
   }
   d.nfwd = pk;
   for (int k = 1; k < L; ++k) {
@@ -781,7 +1032,7 @@ int64_t pm_mlp_net_packed(int32_t layers, const int32_t* sizes, int32_t train) {
 int64_t pm_mlp_net_work(int32_t layers, const int32_t* sizes, int32_t rows) {
   NetDesc d;
   if (!net_desc(layers, sizes, &d) || rows < 1) return 0;
-  return (int64_t)rows * (d.n[0] + 2 * d.nhid + d.ngrad);
+  return (net_work_floats(d, up32(rows)) + 3) & ~3ll;
 }
 
 int pm_mlp_net_pack(void* stream, int32_t batch, int32_t layers, const int32_t* sizes,
@@ -817,18 +1068,18 @@ int pm_mlp_net_forward(void* stream, int32_t batch, int32_t M, int32_t layers,
   const bool big = (int64_t)batch * ((M + wide - 1) / wide) >= 256;
   const int bm = big ? wide : 16;
   const dim3 grid((M + bm - 1) / bm, batch), block(512);
-  const size_t lds = (size_t)bm * d.kp * sizeof(unsigned short);
+  const size_t lds = (size_t)bm * d.kp * sizeof(unsigned short) + d.ngrad * sizeof(float);
   if (big) {
     const int nt = net_nt(d, 4, false);
-    if (nt <= 1) return net_launch(k_net_forward<4, 1, 2, 4>, grid, block, lds, s, args);
-    if (nt <= 2) return net_launch(k_net_forward<4, 2, 2, 4>, grid, block, lds, s, args);
-    if (nt <= 4) return net_launch(k_net_forward<4, 4, 2, 4>, grid, block, lds, s, args);
-    return net_launch(k_net_forward<2, 8, 2, 4>, grid, block, lds, s, args);
+    if (nt <= 1) return net_launch(k_net_forward<4, 1, 2, 4, 4>, grid, block, lds, s, args);
+    if (nt <= 2) return net_launch(k_net_forward<4, 2, 2, 4, 2>, grid, block, lds, s, args);
+    if (nt <= 4) return net_launch(k_net_forward<4, 4, 2, 4, 1>, grid, block, lds, s, args);
+    return net_launch(k_net_forward<2, 8, 2, 4, 1>, grid, block, lds, s, args);
   }
   const int nt = net_nt(d, 8, false);
-  if (nt <= 1) return net_launch(k_net_forward<1, 1, 1, 8>, grid, block, lds, s, args);
-  if (nt <= 2) return net_launch(k_net_forward<1, 2, 1, 8>, grid, block, lds, s, args);
-  return net_launch(k_net_forward<1, 4, 1, 8>, grid, block, lds, s, args);
+  if (nt <= 1) return net_launch(k_net_forward<1, 1, 1, 8, 8>, grid, block, lds, s, args);
+  if (nt <= 2) return net_launch(k_net_forward<1, 2, 1, 8, 8>, grid, block, lds, s, args);
+  return net_launch(k_net_forward<1, 4, 1, 8, 4>, grid, block, lds, s, args);
 }
 
 int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t* sizes, float* P,
@@ -842,34 +1093,28 @@ int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t*
       !packed_ok(packed, stride_packed) || !X || !T || !idx || !work || !lr || !loss || batch < 1 || batch > 65535 || rows < 1 || batch_rows < 1 || t0 < 0)
     return PM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
-  const size_t lds = (size_t)16 * d.kp * sizeof(unsigned short);
+  const size_t lds = (size_t)16 * d.kp * sizeof(unsigned short) + d.ngrad * sizeof(float);
   const int nt = net_nt(d, 8, true);
   int jobs = 0;
   for (int k = 0; k < d.L; ++k)
-    jobs += ((d.n[k + 1] + kBM - 1) / kBM) * ((d.n[k] + kBN - 1) / kBN + 1);
-  const int ablocks = (int)std::min<int64_t>((d.nP + 255) / 256, 1024);
+    jobs += ((d.n[k + 1] + 63) / 64) * ((d.n[k] + 63) / 64) + 1;
   int step = 0;
   for (int32_t i0 = 0; i0 < rows; i0 += batch_rows, ++step) {
-    int B = std::min(batch_rows, rows - i0);
-    float* x0 = work;
-    float* acts = x0 + (int64_t)batch * B * d.n[0];
-    float* zs = acts + (int64_t)batch * B * d.nhid;
-    float* gr = zs + (int64_t)batch * B * d.nhid;
+    int B = std::min(batch_rows, rows - i0), B32 = up32(B);
     const int64_t* ix = idx + i0;
     float* ls = loss + (int64_t)step * batch;
-    void* args[] = {&d, &B, &P, &stride_p, &packed, &stride_packed, &X, &T, &ix, &stride_idx, &w,
-                    &x0, &acts, &zs, &gr, &ls};
-    const dim3 grid((B + 15) / 16, batch);
-    int r = nt <= 1   ? net_launch(k_net_train<1>, grid, dim3(512), lds, s, args)
-            : nt <= 2 ? net_launch(k_net_train<2>, grid, dim3(512), lds, s, args)
-                      : net_launch(k_net_train<4>, grid, dim3(512), lds, s, args);
+    void* args[] = {&d, &B, &B32, &P, &stride_p, &packed, &stride_packed, &X, &T, &ix,
+                    &stride_idx, &w, &work, &ls};
+    const dim3 grid(B32 / 16, batch);
+    int r = nt <= 1   ? net_launch(k_net_train<1, 8>, grid, dim3(512), lds, s, args)
+            : nt <= 2 ? net_launch(k_net_train<2, 8>, grid, dim3(512), lds, s, args)
+                      : net_launch(k_net_train<4, 4>, grid, dim3(512), lds, s, args);
     if (r) return r;
-    hipLaunchKernelGGL(k_net_grads, dim3(jobs, batch), dim3(256), 0, s, d, B, x0, acts, gr, G,
-                       stride_p);
     const int32_t t = t0 + step + 1;
-    const float c1 = 1.0f - powf(beta1, (float)t), c2 = 1.0f - powf(beta2, (float)t);
-    hipLaunchKernelGGL(k_net_adam, dim3(ablocks, batch), dim3(256), 0, s, d, P, G, m, v, stride_p,
-                       packed, stride_packed, lr[step], beta1, beta2, eps, weight_decay, c1, c2);
+    const AdamArgs h{lr[step], beta1, beta2, eps, weight_decay,
+                     1.0f - powf(beta1, (float)t), 1.0f - powf(beta2, (float)t)};
+    hipLaunchKernelGGL(k_net_update, dim3(jobs, batch), dim3(256), 0, s, d, B32, work, P, G, m, v,
+                       stride_p, packed, stride_packed, h);
     r = status();
     if (r) return r;
   }
@@ -881,8 +1126,9 @@ int pm_mlp_net_stats(void* stream, int32_t members, int64_t n, const float* S, i
   if (members < 1 || n < 0 || !S || !mean || !std) return PM_EINVAL;
   if (n == 0) return 0;
   const int blocks = (int)std::min<int64_t>((n + 1023) / 1024, 8192);
+  const int vec = (((uintptr_t)S | (uintptr_t)mean | (uintptr_t)std) & 15) == 0 && stride % 4 == 0;
   hipLaunchKernelGGL(k_net_stats, dim3(blocks), dim3(256), 0, (hipStream_t)stream, members, n, S,
-                     stride, mean, std);
+                     stride, mean, std, vec);
   return status();
 }
 

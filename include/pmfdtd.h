@@ -192,8 +192,8 @@ typedef struct pm_plan {
 
   /* Optional second buffer set for the fused step (yee; 3-D with a padded
    * row sy that is a multiple of 64 (with full coefficient arrays: 128, 256
-   * or 512), or 2-D TM without dispersive boxes and with Cb-only
-   * coefficients).  With E2/H2 and
+   * or 512), or 2-D TM without dispersive boxes and with Cb-only or, with
+   * psi_e2, Ca and Cb coefficients).  With E2/H2 and
    * psi_h2 (for every psi_h given) present, pm_run advances steps with one
    * fused H+E kernel that reads one set and writes the other; a run with an
    * odd step count does its first step in place, so every call returns with
@@ -202,7 +202,8 @@ typedef struct pm_plan {
   void* H2[3];
   void* psi_h2[3][2];
   /* Optional: a second E-side CPML memory set (same layout as psi_e).  With
-   * it (for every psi_e given), FP32 plans with Cb in FP32 or FP16, no
+   * it (for every psi_e given), 2-D TM plans advance up to 8 steps per launch,
+   * sources and samples inside, and 3-D FP32 plans with Cb in FP32 or FP16, no
    * dispersive boxes, padded rows of 128 or 256 cells and at most 64 x CPML
    * layers can advance two steps per launch (pm_set_tuning fuse = 2). */
   void* psi_e2[3][2];
@@ -288,8 +289,10 @@ int pm_dft_flush(pm_ctx* ctx, int64_t step_first, int32_t rows);
  * the unfused kernels, fuse = 2 asks for two steps per launch (temporal
  * blocking; ty must be 4 and vec 0; runs that sample monitors or add
  * sources with a per-cell profile, and the one to three steps of a run that
- * do not fill pairs of passes, take the one-step kernel).  Until it is
- * called, rows, planes and order follow rules on the grid's size and
+ * do not fill pairs of passes, take the one-step kernel).  2-D plans with a
+ * second psi_e set take up to 8 steps per launch with fuse = 2 (ty, kchunk,
+ * vec and order unused) and until this is called; fuse = 1 with the rows per
+ * tile selects their one-pass step.  Until it is called, rows, planes and order follow rules on the grid's size and
  * precision.  Used by the autotuner. */
 int pm_set_tuning(pm_ctx* ctx, int fuse, int ty, int kchunk, int vec, int order);
 
@@ -313,7 +316,8 @@ int pm_row_split_active(pm_ctx* ctx);
 int pm_fused_shape(pm_ctx* ctx, int32_t* out);
 
 /* Steps per fused launch pm_run will use with the current plan and tuning
- * for a run without monitor sampling: 0 (unfused kernels), 1 or 2. */
+ * for a run without monitor sampling: 0 (unfused kernels), 1 or 2 (2-D plans:
+ * 2 when several were asked for with fuse = 2, 1 until then). */
 int pm_fused_active(pm_ctx* ctx);
 
 /* Block until all work on the context's stream has finished. */
@@ -322,7 +326,7 @@ int pm_sync(pm_ctx* ctx);
 /* Average kernel time (ms) since timing was enabled, measured with HIP
  * events on the context stream around every launch of kernel class `which`
  * (0 = H update, 1 = E update, 2 = whole step, 3 = fused H+E step,
- * 4 = spectral flush of one sample block, 5 = two-step launch, 6 = one graph
+ * 4 = spectral flush of one sample block, 5 = launch of two (2-D: up to eight) steps, 6 = one graph
  * replay of a PM_RUN_GRAPH block, timed on the second stream); enabled (and reset) by
  * pm_set_timing.  enable = 0 turns timing off; enable = s >= 1 times the
  * kernels of every s-th step of pm_run (steps whose index is a multiple of

@@ -44,6 +44,7 @@ UNITS = {
     "fused_seg_f32.hip": [],
     "fused_seg_f64.hip": [],
     "tm2d.hip": [],
+    "tm2d_multi.hip": [],
 }
 
 

@@ -403,10 +403,12 @@ class StepEngine:
 
     def _fill_fused_2d(self):
         """2-D TM (the yee scheme steps Ez, Hx, Hy in 2-D): a second Ez, Hx,
-        Hy and second H-side CPML memory (Hy in the x slabs, Hx in the y
-        slabs); lossy media and dispersive boxes keep the unfused kernels."""
+        Hy and a second CPML memory (Hy and Ez terms in the x slabs, Hx and
+        Ez terms in the y slabs); launches of several steps write both,
+        one-pass launches the fields and the H-side memory.  Magnetic media
+        and dispersive boxes keep the unfused kernels."""
         p = self.plan
-        if p.n_ade or p.coeff_kind in (N.COEFF_FULL, N.COEFF_CACB):
+        if p.n_ade or p.coeff_kind == N.COEFF_FULL:
             return
         nx, ny, _ = self.grid.dimensions
         setb = self._alloc((3, 1, ny, self.sy), self.tdtype)
@@ -419,6 +421,8 @@ class StepEngine:
             for q in range(2):
                 if p.psi_h[a][q]:
                     p.psi_h2[a][q] = self._alloc(shape, self.tdtype).data_ptr()
+                if p.psi_e[a][q]:
+                    p.psi_e2[a][q] = self._alloc(shape, self.tdtype).data_ptr()
         self.fused = True
 
     def _fill_ade(self, regions):

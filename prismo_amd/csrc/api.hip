@@ -32,6 +32,8 @@ struct pm_ctx {
   // tuning (0 auto, 1 whole rows, 2 two segments)
   bool split_ok = false;
   int tune_xs = 0;
+  // 2-D: several steps per launch (needs the second E-side CPML memory)
+  bool multi2d_ok = false;
   bool kchunk_set = false;  // pm_set_tuning was called (else the rules below pick)
   int n_cu = 256;           // compute units of the device
   // 2-D compat gate flags: the set the next H update fills (0 / 1) and the
@@ -589,6 +591,36 @@ FusedBufs fused2_bufs(const pm_ctx* c) {
   return fb;
 }
 
+// m steps of a 2-D run in one launch from the current sets into the others
+// (fields and both halves' CPML memory), with their sources and samples; with
+// clock, n counts from the step it holds.
+int do_multi2d(pm_ctx* c, int64_t n, int m, bool src, bool smp, const int64_t* clock) {
+  Span sp(c, 5);
+  const pm_plan& p = c->plan;
+  const bool a_in = c->parity == 0, e_in = c->pe_parity == 0;
+  Tm2dBufs b{};
+  b.Ei = a_in ? p.E[2] : p.E2[2];
+  b.Eo = a_in ? p.E2[2] : p.E[2];
+  for (int q = 0; q < 2; ++q) {
+    b.Hi[q] = a_in ? p.H[q] : p.H2[q];
+    b.Ho[q] = a_in ? p.H2[q] : p.H[q];
+    // x layers: Hy and Ez terms (axis 0: first, second array), y layers: Hx
+    // and Ez terms (axis 1: second, first array)
+    const int h = q == 0 ? 0 : 1, e = q == 0 ? 1 : 0;
+    b.psh_in[q] = a_in ? p.psi_h[q][h] : p.psi_h2[q][h];
+    b.psh_out[q] = a_in ? p.psi_h2[q][h] : p.psi_h[q][h];
+    b.pse_in[q] = e_in ? p.psi_e[q][e] : p.psi_e2[q][e];
+    b.pse_out[q] = e_in ? p.psi_e2[q][e] : p.psi_e[q][e];
+  }
+  if (launch_tm2d_multi(c->g, p.precision, p.coeff_kind, b, src ? &c->aux : nullptr,
+                        smp ? &c->aux : nullptr, n, clock, m, c->n_cu, c->stream))
+    return fail(c, PM_ENOTSUP, "several 2-D steps per launch: plan not supported");
+  c->parity ^= 1;
+  c->pe_parity ^= 1;
+  set_psi_e(c);
+  return launch_status(c, "2-D steps launch");
+}
+
 // Two steps (n, n+1) in one launch from the current sets into the others,
 // with the sources of step n added inside the kernel.
 int do_fused2(pm_ctx* c, int64_t n, bool src) {
@@ -649,6 +681,26 @@ bool fused2d_eligible(const pm_plan& p) {
     for (int q = 0; q < 2; ++q)
       if (p.psi_h[a][q] && !p.psi_h2[a][q]) return false;
   return true;
+}
+
+// Several 2-D steps per launch (tm2d_multi.hip): no dispersive boxes, one Db,
+// second sets of everything a step writes.
+bool multi2d_eligible(const pm_plan& p) {
+  if (p.scheme != PM_SCHEME_YEE || p.ndim != 2 || p.n_ade || p.coeff_kind == PM_COEFF_FULL)
+    return false;
+  if (!p.E2[2] || !p.H2[0] || !p.H2[1]) return false;
+  if ((uint64_t)p.sy * (uint64_t)p.ny >= (1ull << 31)) return false;
+  for (int a = 0; a < 2; ++a)
+    for (int q = 0; q < 2; ++q)
+      if ((p.psi_h[a][q] && !p.psi_h2[a][q]) || (p.psi_e[a][q] && !p.psi_e2[a][q])) return false;
+  return true;
+}
+
+// Runs of this context take several steps per launch: by default where the
+// plan allows it, or asked for with fuse 2; a tuned one-pass step (fuse 1 with
+// its rows per tile) and fuse 0 do not.
+bool use_multi2d(const pm_ctx* c) {
+  return c->multi2d_ok && (c->fuse == 2 || (c->fuse == 1 && !c->kchunk_set));
 }
 
 bool fused_eligible(const pm_plan& p) {
@@ -935,6 +987,7 @@ int pm_configure(pm_ctx* c, const pm_plan* plan) {
   c->parity = 0;
   c->pe_parity = 0;
   set_psi_e(c);
+  c->multi2d_ok = multi2d_eligible(p);
   c->fused2_ok = fused2_eligible(c);
   c->src_kind0 = true;
   for (int s = 0; s < x.n_src; ++s)
@@ -1066,6 +1119,52 @@ int eager_step(pm_ctx* c, int64_t n, bool in_place, bool fused, bool src, bool s
   return 0;
 }
 
+// Steps of the next launch of a 2-D run at step n with `left` to go: a launch
+// does not cross the end of a sample block.
+int multi2d_len(const pm_ctx* c, int64_t n, int64_t left, bool smp) {
+  int64_t m = std::min<int64_t>(tm2d_multi_steps(), left);
+  if (smp) m = std::min<int64_t>(m, c->plan.sample_T - n % c->plan.sample_T);
+  return (int)m;
+}
+
+// nsteps 2-D steps, several per launch, in an even number of launches, so the
+// state ends in the set it started from: where the count is odd the first
+// launch is cut in two, or, if it holds one step, that step is taken in place.
+// With clock (a captured block starting at a multiple of sample_T): n counts
+// from the step it holds, no bookkeeping of samples.
+int run_multi2d(pm_ctx* c, int64_t step0, int32_t nsteps, bool src, bool smp, bool dft,
+                const int64_t* clock) {
+  int64_t launches = 0;
+  for (int64_t s = 0; s < nsteps; ++launches) s += multi2d_len(c, step0 + s, nsteps - s, smp);
+  bool odd = (launches & 1) != 0;
+  int cut = 0;  // the second part of a launch cut in two
+  int r;
+  for (int32_t s = 0; s < nsteps;) {
+    const int64_t n = step0 + s;
+    c->span_on = !clock && c->timing && n % c->timing_stride == 0;
+    int m = cut ? cut : multi2d_len(c, n, nsteps - s, smp);
+    cut = 0;
+    if (odd) {
+      odd = false;
+      if (m == 1 && clock) return fail(c, PM_EINVAL, "odd one-step block in a captured run");
+      if (m == 1) {
+        if ((r = eager_step(c, n, true, true, src, smp, dft))) return r;
+        ++s;
+        continue;
+      }
+      m -= 1;
+      cut = 1;
+    }
+    if (smp && !clock && (r = sample_pre(c, n, dft))) return r;
+    if ((r = do_multi2d(c, n, m, src, smp, clock))) return r;
+    if (smp && !clock)
+      for (int k = 0; k < m; ++k)
+        if ((r = sample_post(c, n + k, dft))) return r;
+    s += m;
+  }
+  return 0;
+}
+
 // Capture one block of G steps that starts in buffer set `par` into graph
 // slot `slot`, on the second stream: per step the fields, the sources (table row from the step
 // clock, which holds the block's first step) and the samples (row k of X);
@@ -1076,7 +1175,7 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
   const pm_plan& p = c->plan;
   int64_t* clk = step_clock(c);
   hipStream_t s0 = c->stream;
-  const int par0 = c->parity;
+  const int par0 = c->parity, pe0 = c->pe_parity;
   const bool span0 = c->span_on;
   c->stream = c->s2;
   c->parity = par;
@@ -1085,7 +1184,9 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
   int r = hip_check(c, hipStreamBeginCapture(c->s2, hipStreamCaptureModeThreadLocal),
                     "begin capture");
   if (!r) {
-    for (int32_t k = 0; k < G && !r; ++k) {
+    const bool multi = fused && use_multi2d(c);
+    if (multi) r = run_multi2d(c, 0, G, src, smp, false, clk);
+    for (int32_t k = 0; k < G && !r && !multi; ++k) {
       if (fused) {
         r = do_fused(c);
       } else {
@@ -1123,6 +1224,8 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
   }
   c->stream = s0;
   c->parity = par0;
+  c->pe_parity = pe0;
+  set_psi_e(c);
   c->span_on = span0;
   if (!r)
     r = hip_check(c, hipGraphInstantiate(&c->graph[slot], g, nullptr, nullptr, 0),
@@ -1177,6 +1280,31 @@ int run_graph(pm_ctx* c, int64_t step0, int32_t nsteps, int32_t G, bool fused, b
               bool smp, bool dft) {
   int32_t s = 0;
   int r;
+  if (fused && use_multi2d(c)) {
+    // up to a block start, whole blocks, the rest: each an even number of
+    // launches
+    const int32_t lead = smp ? (int32_t)((G - step0 % G) % G) : 0;
+    if (lead > 0) {
+      s = std::min(lead, nsteps);
+      if ((r = run_multi2d(c, step0, s, src, smp, dft, nullptr))) return r;
+    }
+    const int32_t nrep = (nsteps - s) / G;
+    if (nrep > 0) {
+      if (smp && c->pend_n) {
+        if (dft) {
+          if ((r = flush_pending(c))) return r;
+        } else {
+          c->pend_n = 0;
+        }
+      }
+      if ((r = replay_blocks(c, step0 + s, nrep, G, fused, src, smp, dft))) return r;
+      s += nrep * G;
+    }
+    if (s < nsteps && (r = run_multi2d(c, step0 + s, nsteps - s, src, smp, dft, nullptr)))
+      return r;
+    c->span_on = c->timing;
+    return 0;
+  }
   auto direct = [&](int32_t k) {
     c->span_on = c->timing && (step0 + k) % c->timing_stride == 0;
     return eager_step(c, step0 + k, fused && k == 0 && (nsteps & 1), fused, src, smp, dft);
@@ -1232,12 +1360,19 @@ int pm_run(pm_ctx* c, int64_t step0, int32_t nsteps, uint32_t flags) {
     return 0;
   }
   int fvec = 0, fw = 0, fty = 0, fxs = 1;
-  const bool fused = c->fused_ok && c->fuse && fused_shape(c, &fvec, &fw, &fty, &fxs);
+  const bool multi = use_multi2d(c);
+  const bool fused =
+      multi || (c->fused_ok && c->fuse && fused_shape(c, &fvec, &fw, &fty, &fxs));
   if (flags & PM_RUN_GRAPH) {
     const int32_t G = smp ? p.sample_T : kGraphSteps;
     if (G % 2) return fail(c, PM_EINVAL, "graph replay needs an even sample_T (%d)", G);
     if (!c->s2) return fail(c, PM_ENOTSUP, "graph replay needs the context's second stream");
     return run_graph(c, step0, nsteps, G, fused, src, smp, dft);
+  }
+  if (multi) {
+    const int r = run_multi2d(c, step0, nsteps, src, smp, dft, nullptr);
+    c->span_on = c->timing;
+    return r;
   }
   // two steps per launch for the steps that fill pairs of passes (an even
   // number of passes, so the E-side CPML memory ends in its first set); the
@@ -1359,6 +1494,7 @@ int pm_set_tuning(pm_ctx* c, int fuse, int ty, int kchunk, int vec, int order) {
 int pm_fused_active(pm_ctx* c) {
   if (!c || !c->configured) return 0;
   int vec = 0, w = 0, ty = 0;
+  if (use_multi2d(c)) return c->fuse == 2 ? 2 : 1;
   if (!c->fused_ok) return 0;
   int xs = 1;
   if (!(c->fuse && fused_shape(c, &vec, &w, &ty, &xs))) return 0;

@@ -190,9 +190,19 @@ struct Tm2dBufs {
   void* Ho[2];
   const void* psh_in[2];
   void* psh_out[2];
+  const void* pse_in[2];  // E-side memory (x, y layers) read and written by
+  void* pse_out[2];       // launches of several steps
 };
 int launch_tm2d_fused(const KGrid& g, int precision, int ck, const Tm2dBufs& b, int chunk,
                       hipStream_t s);
+// ns (at most tm2d_multi_steps()) 2-D TM steps from set "i" to set "o"
+// (tm2d_multi.hip), with the sources of steps step .. (src, NULL for none;
+// relative to *clock when given) and their samples (smp; rows step mod sample_T
+// .., which must not wrap).
+int launch_tm2d_multi(const KGrid& g, int precision, int ck, const Tm2dBufs& b, const KAux* src,
+                      const KAux* smp, int64_t step, const int64_t* clock, int ns, int n_cu,
+                      hipStream_t s);
+int tm2d_multi_steps();
 // xs: row segments per padded row (1, or 2: rows of 2 x 64 vec w cells).
 int launch_yee_fused_f32(const KGrid& g, int ck, const FusedBufs& fb, int vec, int w, int ty,
                          int kchunk, int order, int xs, hipStream_t s);

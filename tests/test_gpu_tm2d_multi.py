@@ -1,0 +1,134 @@
+"""GPU: several 2-D TM steps per launch (the default for lossless and
+conductive 2-D runs) against the unfused kernels and O1.
+
+Widths and heights sit at the edges of the tiles (56 columns, 8 / 24 / 56
+rows), run lengths leave every remainder of the 4 steps a launch takes and
+cross the ends of the 128-row sample blocks.  The unfused kernels do the same
+operations per cell: 1e-13 relative L2 in FP64, 1e-6 in FP32; O1 at 1e-10 /
+1e-5, the bars of the other 2-D paths.
+"""
+
+import numpy as np
+import pytest
+
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+D = 20e-9
+FREQS = [187e12, 193e12, 200e12]
+
+
+def _sim(nx, ny, t, dtype, storage="auto", sigma=False, extra=False, seed=4):
+    import prismo_amd as pa
+
+    rng = np.random.default_rng(seed)
+    eps = rng.choice([1.0, 2.085, 12.1], size=(nx, ny, 1))
+    ma = {"eps_rel": eps}
+    if sigma:
+        ma["sigma_e"] = rng.choice([0.0, 300.0, 5e4], size=(nx, ny, 1))
+    s = 1 - 1e-9
+    px, py = (nx - 2 * t) * D, (ny - 2 * t) * D
+    sim = pa.Simulation(size=(px * s, py * s, 0.0), resolution=1 / D, pml_layers=t,
+                        courant_factor=0.99, scheme="yee", dtype=dtype,
+                        pml=pa.PMLParams(t) if t else None, material_arrays=ma,
+                        coefficient_storage=storage)
+    sim.add_source(pa.PlaneWaveSource(center=(0.3 * px, 0.5 * py, 0.0), size=(0.0, 0.8 * py, 0.0),
+                                      direction="+x", polarization="z", frequency=193e12,
+                                      pulse_width=2e-15))
+    if extra:
+        # overlaps the line above in Ez; a per-cell profile on Ez and Hy
+        sim.add_source(pa.ElectricDipole(position=(0.3 * px, 0.5 * py, 0.0), polarization="z",
+                                         frequency=200e12, pulse_width=1e-15, amplitude=0.3))
+        sim.add_source(pa.GaussianBeamSource(center=(0.5 * px, 0.5 * py, 0.0),
+                                             size=(0.0, 0.6 * py, 0.0), direction="x",
+                                             polarization="z", frequency=190e12,
+                                             beam_waist=0.2 * py, pulse_width=2e-15))
+    mon = pa.FieldMonitor(center=(0.6 * px, 0.5 * py, 0.0), size=(0.4 * px, 0.7 * py, 0.0),
+                          components=["Ez", "Hx", "Hy"], time_domain=False,
+                          frequencies=list(FREQS))
+    sim.add_monitor(mon)
+    return sim, mon
+
+
+def _out(sim, mon):
+    f = np.concatenate([sim.fields.to_numpy(c).ravel() for c in ("Ez", "Hx", "Hy")])
+    s = np.concatenate([mon.frequency_stack(c).ravel() for c in mon.components])
+    return f, s
+
+
+def _both(nx, ny, t, dtype, runs, bar, start=False, **kw):
+    import torch
+
+    outs = []
+    for fuse in (True, False):
+        sim, mon = _sim(nx, ny, t, dtype, **kw)
+        if start:      # fields everywhere from the first step on
+            rng = np.random.default_rng(8)
+            for c, amp in (("Ez", 1.0), ("Hx", 1 / 377), ("Hy", 1 / 377)):
+                f = amp * rng.normal(size=tuple(sim.fields[c].shape))
+                sim.fields[c] = torch.from_numpy(f.astype(np.float32).astype(np.float64))
+        eng = sim.solver.updater.engine_for(sim.fields)
+        if not fuse:
+            eng.ctx.set_tuning(0, 4, 8, 0, 2)
+        assert eng.ctx.fused_steps() == int(fuse)
+        for n in runs:
+            sim.run_steps(n)
+        outs.append(_out(sim, mon))
+    assert np.linalg.norm(outs[1][0]) > 0 and np.linalg.norm(outs[1][1]) > 0
+    for a, b in zip(*outs):
+        assert rel_l2(a, b) <= bar
+
+
+@pytest.mark.parametrize("shape,t", [((40, 30), 6), ((56, 8), 0), ((57, 25), 3), ((113, 33), 8),
+                                     ((9, 70), 0), ((120, 65), 20)])
+@pytest.mark.parametrize("runs", [[61], [64], [3, 2, 1, 1, 5, 140]])
+def test_fp64_equals_unfused(mi355x, shape, t, runs):
+    _both(*shape, t, np.float64, runs, 1e-13)
+
+
+@pytest.mark.parametrize("dtype,storage,bar", [(np.float64, "auto", 1e-13),
+                                               (np.float32, "auto", 1e-6),
+                                               (np.float32, "fp16", 1e-6)])
+def test_sources_of_every_kind(mi355x, dtype, storage, bar):
+    _both(90, 50, 8, dtype, [37, 100], bar, storage=storage, extra=True)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-13), (np.float32, 1e-6)])
+def test_conductive_media(mi355x, dtype, bar):
+    _both(75, 61, 7, dtype, [41], bar, sigma=True)
+
+
+@pytest.mark.parametrize("shape,dtype,bar", [((1000, 800), np.float64, 1e-13),
+                                             ((1000, 800), np.float32, 1e-6),
+                                             ((1500, 1201), np.float32, 1e-6)])
+def test_taller_tiles(mi355x, shape, dtype, bar):
+    """Grids large enough for 24- and 56-row tiles."""
+    _both(*shape, 10, dtype, [22], bar, start=True)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-10), (np.float32, 1e-5)])
+def test_against_oracle(mi355x, dtype, bar):
+    from oracle import compat as O0
+    from oracle.yee import YeeOracle
+
+    t, steps = 9, 150
+    sim, mon = _sim(130, 59, t, dtype)
+    sim.run_steps(steps)
+    eps = sim.solver.updater.eps_rel[:, :, 0]
+    one, zero = np.ones_like(eps), np.zeros_like(eps)
+    _, Cb, _, Db = O0.coefficients(eps, one, zero, zero, sim.dt)
+    from prismo_amd.core.coefficients import component_average
+
+    o1 = YeeOracle(130, 59, 1, sim.grid.spacing, sim.dt,
+                   {"Ez": component_average(Cb, "Ez", True)}, float(Db.flat[0]),
+                   pml=(t, t, t, t, 0, 0))
+    tt = 0.0
+    for _ in range(steps):
+        o1.step()
+        tt += sim.dt
+        for s in sim.sources:
+            s.update_fields(o1.F, tt, sim.dt)
+    got, _ = _out(sim, mon)
+    ref = np.concatenate([o1.F[c].ravel() for c in ("Ez", "Hx", "Hy")])
+    assert rel_l2(got, ref) <= bar

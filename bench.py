@@ -225,8 +225,8 @@ def copy_probe():
 
 
 def batch_probe(steps=8):
-    """The 256 coupler designs of the sweep, one batch (8-row tiles), a few
-    eager steps: one k_batch_tm launch per step for counter runs."""
+    """The 256 coupler designs of the sweep, one batch, a few
+    eager steps in one k_batch_tm launch for counter runs."""
     import numpy as np
     import torch
 
@@ -280,14 +280,14 @@ SWEEP_ALG_BYTES_PER_PML_CELL_AXIS = 16.0  # two FP32 psi read + written
 
 def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
     """Batched 256-coupler sweep through ParameterSweep's batched back end
-    (FP32 fields, FP16 Cb, one launch per step over every design of a group
+    (FP32 fields, FP16 Cb, one launch per eight steps over every design of a group
     of ``group``, the first group ``first`` designs so the GPU starts early,
     graph-replayed step loop, groups pipelined so the host builds and
     analyses while the GPU steps), timed end to end, against
     sequential plain FP64 runs of an evenly spaced sample of the same
     designs, after an untimed 64-step warm-up sweep of one group of each
     size.  Then all designs in one batch, the shape the workload is stated
-    in (one launch per step over all 256, the step loop replayed as a HIP
+    in (one launch per eight steps over all 256, the step loop replayed as a HIP
     graph), timed end to end (build, run, |S21|) after an untimed 64-step
     run of that batch size (kernels loaded, launch shape tuned); the batch
     kernel's roofline is taken on that run (HIP events)."""
@@ -299,7 +299,7 @@ def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
     from prismo_amd.optimization.sweep import BatchedRunner, ParameterSweep
 
     designs = W.coupler_designs(n_designs)
-    # rows per tile and launch shape from the autotuner (the untimed warm-up
+    # workgroup order from the autotuner (the untimed warm-up
     # below tunes each group size once; the timed run uses the cached picks)
     kw = {"chunk": "auto", "sample_T": 128}
     runner = BatchedRunner(build=lambda p: W.coupler_sim(p, backend=W.host_backend()),
@@ -327,7 +327,7 @@ def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
           f"(first group {first}, then groups of {group}, pipelined)", file=sys.stderr,
           flush=True)
 
-    # all designs in one batch: one launch per step over all of them
+    # all designs in one batch: one launch per eight steps over all of them
     sims = [W.coupler_sim(p, backend=W.host_backend()) for p in designs]
     BatchEngine(sims, dtype=np.float32, coefficient_storage="fp16", **kw).run_steps(64)
     torch.cuda.synchronize()
@@ -391,7 +391,7 @@ def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
         "max_abs_s31_err": err31,
         "cells_per_step": cells,
         "gcells_per_s": round(cells / (step_ms * 1e-3) / 1e9, 3),
-        "roofline": {"bound": "hbm", "kernel": "k_batch_tm (one launch per step, all designs)",
+        "roofline": {"bound": "valu", "kernel": "k_batch_tm (one launch per 8 steps, all designs)",
                      "achieved": round(alg / (step_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg / (step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "alg_bytes_per_step": alg, "step_ms": round(step_ms, 5),

@@ -1,6 +1,6 @@
 /*
  * pmbatch.h -- batched 2-D TM (Ez, Hx, Hy) time stepping of many uneven
- * grids in one launch per step, for parameter sweeps.
+ * grids, up to eight steps per launch, for parameter sweeps.
  *
  * The reference runs a sweep as one full Simulation per parameter set,
  * sequentially or in a process pool (src/prismo/optimization/sweep.py:
@@ -8,7 +8,7 @@
  * (src/prismo/core/simulation.py:147-164).  These entry points replace that
  * loop for a whole batch of 2-D designs at once: every design keeps its own
  * grid, materials, CPML, line sources and port sample lines; one kernel
- * advances all of them by one step; the samples of all ports of all designs
+ * advances all of them by up to eight steps; the samples of all ports of all designs
  * form one matrix whose spectra are one MFMA GEMM per block of steps.
  *
  * Scheme: the textbook Yee TM update of pmfdtd.h's PM_SCHEME_YEE in 2-D
@@ -42,12 +42,13 @@ typedef struct pm_batch_design {
   int32_t nx, ny;            /* grid nodes */
   int32_t sy, n_lines;       /* row pitch (elements, >= nx); sample lines used */
   int32_t pml[4];            /* CPML layers x-lo, x-hi, y-lo, y-hi */
-  void* ez[2];               /* ping-pong field sets (state alternates every step) */
+  void* ez[2];               /* ping-pong field sets (state alternates every launch) */
   void* hx[2];
   void* hy[2];
   void* psi_hx[2];           /* H-side CPML memory (dEz/dy at Hx, dEz/dx at Hy), ping-pong */
   void* psi_hy[2];
-  void* psi_ex;              /* E-side CPML memory of Ez (dHy/dx, dHx/dy terms), in place */
+  void* psi_ex;              /* E-side CPML memory of Ez (dHy/dx, dHx/dy terms); the second
+                                set is in the plan's workspace */
   void* psi_ey;
   const void* cb;            /* Cb at Ez points: field precision, or FP16 (coeff_kind CB_F16) */
   double cb_scale;           /* FP16 Cb = cb_scale * stored value (1 otherwise) */
@@ -73,7 +74,7 @@ typedef struct pm_batch_plan {
   pm_dft_group dft;                  /* spectra over all sample columns */
   const void* W_re;                  /* [nfreq][table_len] phasors * dt, field precision */
   const void* W_im;
-  int32_t nfreq, chunk;              /* chunk: rows per tile (>= 2) */
+  int32_t nfreq, chunk;              /* chunk: >= 2, no longer used (tiles follow a rule) */
   void* work;                        /* device workspace, pm_batch_workspace_bytes */
   int64_t work_bytes;
 } pm_batch_plan;
@@ -84,7 +85,8 @@ int pm_batch_create(int device, void* stream, pm_batch** out);
 int pm_batch_destroy(pm_batch* b);
 const char* pm_batch_last_error(pm_batch* b);
 
-/* Device workspace the plan needs (tile list, design table, step clock). */
+/* Device workspace the plan needs (tile list, design table, step clock, second
+ * E-side CPML memory: two arrays of ny_d * sy_d values per design). */
 int pm_batch_workspace_bytes(const pm_batch_plan* plan, int64_t* bytes);
 
 /* Validate and adopt a plan; uploads the design table and tile list into
@@ -115,14 +117,16 @@ int pm_batch_sync(pm_batch* b);
 int pm_batch_design_status(pm_batch* b, int32_t* out, int32_t n);
 
 /* Launch shape of the step kernel: waves (64 cells wide each) per
- * workgroup, 1, 2, 4 (default) or 8, and the workgroup order (1, default:
- * each run of 64 workgroups is grouped by XCD so neighbouring strips share
- * an L2; 0: launch order).  Rows per tile are the plan's `chunk`.  Results
- * do not depend on any of them.  Tunes what the reference's backends take as
+ * workgroup, 1, 2, 4 or 8 (checked, no longer used: a tile has eight), and the
+ * workgroup order (1, default: each run of 64 workgroups is grouped by XCD so
+ * neighbouring tiles share an L2; 0: launch order).  Results do not depend on
+ * it.  Tunes what the reference's backends take as
  * fixed launch constants (src/prismo/backends/cuda_kernels.py:230-265). */
 int pm_batch_set_tuning(pm_batch* b, int waves, int xcd_order);
 
-/* Average time (ms) per step kernel (which 0) or per flush (1) since enabled. */
+/* Average time (ms) per eager step (which 0: the launches' time over the steps
+ * they took), per flush (1) or per graph replay (2) since enabled; count: steps,
+ * flushes or replays. */
 int pm_batch_set_timing(pm_batch* b, int enable);
 int pm_batch_get_timing(pm_batch* b, int which, double* avg_ms, int64_t* count);
 

@@ -40,11 +40,11 @@ CANDIDATES2 = {
 # against 27) unless rows are asked for.
 CANDIDATES_2D = (1, 2, 3, 4, 8)
 
-# batched 2-D step: rows per tile (the plan's chunk), waves per workgroup,
-# XCD-grouped workgroup order
+# batched 2-D step: workgroup order.  Tiles follow a rule in the library; the
+# plan's chunk and the waves asked for do not change the launch
 BATCH_CANDIDATES = {
-    "chunk": (4, 8, 16, 32),
-    "waves": (2, 4, 8),
+    "chunk": (8,),
+    "waves": (4,),
     "xcd": (0, 1),
 }
 
@@ -181,10 +181,9 @@ def _batch_key(eng) -> str:
 def tune_batch(eng, steps: int = 16, candidates: dict | None = None,
                force: bool = False) -> dict:
     """Pick and apply the fastest launch shape of the batched step for the
-    configured, not yet run ``BatchEngine`` ``eng``: each candidate (rows per
-    tile, waves per workgroup, workgroup order) runs ``steps`` eager steps
-    timed with HIP events on the engine's stream; then the engine's state is
-    cleared back to the zeros a run starts from and it is re-planned with
+    configured, not yet run ``BatchEngine`` ``eng``: each candidate (workgroup
+    order) runs ``steps`` eager steps timed with HIP events on the engine's
+    stream; then the engine's state is cleared back to the zeros a run starts from and it is re-planned with
     the pick.  Results are bitwise the same under every shape (each cell's
     arithmetic does not depend on the tiling); cached per (precision,
     coefficient storage, designs per batch) like ``tune``.

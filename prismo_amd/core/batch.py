@@ -4,9 +4,9 @@ A parameter sweep in the reference runs one ``Simulation`` per parameter set
 (src/prismo/optimization/sweep.py:119-167), each its own Python step loop.
 ``BatchEngine`` takes the Simulations of a sweep as descriptions -- grid,
 materials, CPML, sources, monitors, exactly as they were built -- and
-advances all of them together: one kernel launch per step over every design,
-the step loop replayed as a captured HIP graph, the spectra of every port of
-every design one MFMA GEMM per block of steps.  Results land in each
+advances all of them together: one kernel launch takes every design up to
+eight steps on, the step loop is replayed as a captured HIP graph, and the
+spectra of every port of every design are one MFMA GEMM per block of steps.  Results land in each
 Simulation's own monitors, so analysis code reads them as after
 ``Simulation.run``.
 
@@ -66,8 +66,8 @@ class BatchEngine:
             if s.dt != self.dt or tuple(s.grid.spacing) != self.d:
                 raise NotImplementedError("every design must share dx, dy and dt")
         self.sample_T = int(sample_T)
-        # rows per tile; "auto": the autotuner picks them with the launch
-        # shape when the run starts (prismo_amd.autotune.tune_batch)
+        # "auto": the autotuner picks the workgroup order when the run starts
+        # (prismo_amd.autotune.tune_batch); tiles follow a rule in the library
         self.auto_tune = chunk == "auto"
         self.chunk = 8 if self.auto_tune else int(chunk)
         self.tuning = None
@@ -384,7 +384,7 @@ class BatchEngine:
                     a.zero_()
 
     def reconfigure(self, chunk: int):
-        """Re-plan with ``chunk`` rows per tile; the step counter restarts."""
+        """Re-plan; the step counter restarts."""
         self.chunk = int(chunk)
         self.plan.chunk = self.chunk
         self.stream.wait_stream(_torch().cuda.current_stream(self.device))

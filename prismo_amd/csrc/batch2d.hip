@@ -1,53 +1,48 @@
 // Batched 2-D TM stepping of many uneven grids (include/pmbatch.h).
 //
-// One launch advances every design by one step.  The work list holds one
-// tile per wave: (design, x0, r0, r1) = a strip of 64 x cells [x0, x0+64),
-// x0 a multiple of 64 (rows are padded to 64 cells, so every row access of
-// a wave is two whole 128-byte lines), and the rows [r0, r1).  The wave
-// marches up its rows once, carrying row j-1 in registers:
-//   H(n+1/2) at row j   from Ez(j), Ez(j-1) (registers) and Ez(i-1) (shuffle);
-//   E(n+1)   at row j-1 from Hx(j), Hx(j-1), Hy(i), Hy(i+1) (registers/shuffle).
-// The two values from outside the strip come from one extra load per row
-// (lanes 0..3: Ez(x0-1), and Ez, Hy and the Hy CPML state at x0+64): lane 0
-// takes Ez(x0-1) as its left neighbour, and Hy(n+1/2) at x0+64, which lane
-// 63's E update needs, is recomputed from them with the arithmetic of the
-// next strip's lane 0.  So every array is read once and written once per
-// step (plus one halo row per tile).  Reads come from field set
-// `par`, writes go to set par^1, so neighbouring tiles never see a
-// half-updated value; the H-side CPML memory is ping-ponged for the same
-// reason, the E-side memory is touched only by the owner and stays in place.
-// Sources are added after the E update, samples are taken after the sources,
-// as src/prismo/core/simulation.py:147-164 orders them.
+// One launch advances every design by up to eight steps: a workgroup takes one
+// tile of one design (tm2d_pass.h), and a table gives it the design and the
+// tile.  One step per launch moved 300 MB a step for 64 coupler grids of
+// 9.8 M cells together: 68 us at 4.5 TB/s, the rate of a large copy, so only
+// fewer passes over the state could make it faster; eight steps a pass take 146
+// us, 18 a step, two thirds of which the vector ALU is busy (a third of the tiles
+// of a coupler touch a CPML layer).  Reads come from field set `par`, writes go
+// to set par ^ 1, so neighbouring tiles never see a half-updated value; the CPML
+// memory of both field halves is ping-ponged for the same reason (the second
+// E-side set is in the workspace).  Sources are added after the E update, samples
+// are taken after the sources, as src/prismo/core/simulation.py:147-164 orders
+// them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <type_traits>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
 #include <vector>
 
 #include "../../include/pmbatch.h"
-#include "pm_internal.h"
+#include "tm2d_pass.h"
 
 namespace pm {
 namespace {
 
-constexpr int kStrip = 64;    // cells per wave
-constexpr int kMaxWaves = 8;  // waves per workgroup: 1, 2, 4 (default) or 8
-
 struct KWork {
-  int d, x0, r0, r1;
+  int d, x0, y0;
+};
+
+// A design and the second set of its E-side CPML memory.
+struct KDesign {
+  pm_batch_design d;
+  void* psi_ex1;
+  void* psi_ey1;
 };
 
 struct KBatch {
-  const pm_batch_design* des;
+  const KDesign* des;
   const KWork* work;
-  int n_work;
   int ncols, sample_T;
   int64_t* clock;
   int32_t* status;  // per design: bit 0 set once an Ez value was not finite
-  int waves;        // waves per workgroup (the launch's blockDim.x / 64)
   int xcd;          // 1: XCD-grouped workgroup order, 0: launch order
   double idx, idy;
   const double* tab_e;
@@ -56,332 +51,160 @@ struct KBatch {
   void* X;
 };
 
-// Loads of one row for the H update (fields, H-side CPML memory and the
-// y profile at nodes) and of one row for the E update (Cb, E-side CPML
-// memory, y profile at half nodes).  They are issued one iteration before
-// their use; the loop below alternates two register sets instead of copying
-// so no wait lands on the loop's back edge.
 template <typename T>
-struct RowH {
-  T ez, hx, hy, psx, psy;
-  T halo;  // lanes 0..3: Ez(x0-1), Ez(x0+64), Hy(x0+64), Hy CPML state at x0+64
+struct BatchY {
+  gptr<const T> p;  // 8 values per row
+  __device__ __forceinline__ T operator()(int k, int j) const { return p[8 * j + k]; }
 };
 
-// Element e of an array in global memory: a uniform base plus a 32-bit
-// byte offset, so one offset register serves every array of a row (the
-// host checks that a design's arrays fit 32-bit byte offsets).
+// Sources (one Ez and one Hy line) and sample lines of a tile.  Lane l holds
+// line l and the source values of step l of the pass: loaded beside the fields,
+// read back with lane broadcasts.  Lines that do not meet the tile are masked
+// out; most tiles have none.
 template <typename T>
-__device__ __forceinline__ T ldg(const void* base, uint32_t e) {
-  return *(gptr<const T>)((gptr<const char>)base + e * (uint32_t)sizeof(T));
-}
+struct BatchIo {
+  static constexpr bool kStatus = true;
+  static_assert(PM_BATCH_MAX_LINES <= 64 && kTmS <= 64, "one lane per entry");
+  const KBatch& k;
+  const pm_batch_design& D;
+  int64_t step;      // of the pass's first step
+  int x0, y0, rows;  // what the tile writes: columns x0 .., rows y0 ..
+  int comp, col, li, j0, j1;  // this lane's line
+  T ve, vh;
+  int se_i, se0, se1, sh_i, sh0, sh1;
+  bool hit_e, hit_h;
+  unsigned mask;
+  gptr<T> X;
 
-// Stores are non-temporal: the other field set is read one step later,
-// after every design's step, so caching it only displaces reused lines.
-template <typename T>
-__device__ __forceinline__ void stg(void* base, uint32_t e, T v) {
-  __builtin_nontemporal_store(v, (gptr<T>)((gptr<char>)base + e * (uint32_t)sizeof(T)));
-}
-
-// Value of v in lane l (l uniform), for the whole wave.
-template <typename T>
-__device__ __forceinline__ T lane_value(T v, int l) {
-  if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-  } else {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
-    return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);
+  __device__ __forceinline__ void first() {
+    const int lane = threadIdx.x & 63;
+    comp = col = li = j0 = j1 = 0;
+    if (lane < D.n_lines) {
+      const gptr<const pm_batch_line> L = (gptr<const pm_batch_line>)D.line + lane;
+      comp = L->comp;
+      li = L->i;
+      j0 = L->j0;
+      j1 = L->j1;
+      col = L->col;
+    }
+    se_i = D.src_e[0];
+    se0 = D.src_e[1];
+    se1 = D.src_e[2];
+    sh_i = D.src_h[0];
+    sh0 = D.src_h[1];
+    sh1 = D.src_h[2];
+    X = (gptr<T>)k.X + (step % k.sample_T) * (int64_t)k.ncols;
   }
-}
 
-// Bit 31 set exactly for Inf and NaN: the exponent field plus one carries
-// into the sign position only when the field is all ones.  Integer VALU
-// work, OR-ed into one register per lane (a compare would hold a lane mask
-// in scalar registers across the row loop), and no floating-point mode can
-// fold it away.
-template <typename T>
-__device__ __forceinline__ uint32_t nonfinite_bit(T v) {
-  if constexpr (sizeof(T) == 4)
-    return (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) + 0x00800000u;
-  else
-    return ((uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32) & 0x7ff00000u) + 0x00100000u;
-}
+  // sources act on the halo too, samples on what the tile writes
+  __device__ __forceinline__ bool meets(int i, int a, int b, int h) const {
+    return i >= x0 - h && i < x0 + kTmCols + h && a < y0 + rows + h && b > y0 - h && a < b;
+  }
 
-template <typename T, int CK>
-struct RowE {
-  using CbT = typename std::conditional<CK == PM_COEFF_CB_F16, unsigned short, T>::type;
-  CbT cb;
-  T pex, pey;
+  __device__ __forceinline__ void second(int ns) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = step - k.table_step0 + min(lane, ns - 1);
+    ve = (T)((gptr<const double>)k.tab_e)[row];
+    vh = (T)((gptr<const double>)k.tab_h)[row];
+    hit_e = meets(se_i, se0, se1, kTmS);
+    hit_h = meets(sh_i, sh0, sh1, kTmS);
+    mask = (unsigned)__ballot(meets(li, j0, j1, 0));
+  }
+
+  template <int R>
+  __device__ __forceinline__ void sources(int s, int i, int jb, T (&ez)[R], T (&hx)[R],
+                                          T (&hy)[R]) const {
+    if (hit_e) {
+      const T v = tm_bcast(ve, s);
+      tm_add([&](int) { return v; }, i == se_i, se0, se1, jb, ez);
+    }
+    if (hit_h) {
+      const T v = tm_bcast(vh, s);
+      tm_add([&](int) { return v; }, i == sh_i, sh0, sh1, jb, hy);
+    }
+  }
+
+  __device__ __forceinline__ int of(int v, int l) const { return __builtin_amdgcn_readlane(v, l); }
+
+  template <int R>
+  __device__ __forceinline__ void put(int t, int s, int i, int jb, const T (&f)[R]) const {
+    const int c0 = of(j0, t), c1 = of(j1, t);
+    const int p0 = max(c0, y0), p1 = min(c1, y0 + rows);  // rows the tile writes
+    const gptr<T> x = X + s * (int64_t)k.ncols + of(col, t) + (p0 - c0);
+    tm_put(x, 1, i == of(li, t), p0, p1, jb, f);
+  }
+
+  template <int R>
+  __device__ __forceinline__ void samples(int s, int i, int jb, const T (&ez)[R],
+                                          const T (&hx)[R], const T (&hy)[R]) const {
+    for (unsigned m = mask; m; m &= m - 1) {
+      const int t = __builtin_ctz(m), c = of(comp, t);
+      if (c == 0) put(t, s, i, jb, ez);
+      else if (c == 1) put(t, s, i, jb, hx);
+      else put(t, s, i, jb, hy);
+    }
+  }
 };
 
-template <typename T, int CK>
-__global__ __launch_bounds__(64 * kMaxWaves) void k_batch_tm(const KBatch k, int64_t step_arg,
-                                                             int use_clock, int s_rel,
-                                                             int par) {
+template <typename T, int CK, int R>
+__global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64_t step_arg,
+                                                           int use_clock, int s_rel, int ns,
+                                                           int par) {
+  __shared__ TmShared<T, R> sh;
   const int lane = threadIdx.x & 63;
-  // the wave index is uniform: make that visible so the tile and design
-  // descriptors are scalar loads
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // workgroups go round-robin over the 8 XCDs (b % 8); in each group of 64,
-  // XCD x takes work groups 8x .. 8x+7, so neighbouring strips (which read
-  // the same cache lines at their edges) share one L2
-  const int b = blockIdx.x, nb = gridDim.x;
-  const int wg = k.xcd && b < (nb & ~63) ? (b & ~63) + (b & 7) * 8 + ((b >> 3) & 7) : b;
-  const int item = wg * k.waves + wv;
-  if (item >= k.n_work) return;  // whole wave
-  const KWork w = k.work[item];
-  const pm_batch_design& D = k.des[w.d];
-  const int64_t step = use_clock ? (*k.clock + s_rel) : step_arg;
-  const int nx = D.nx, ny = D.ny;
-  const int64_t sy = D.sy;
-  const int x0 = w.x0;
-  const int i = x0 + lane;
-  const bool inx = i < nx;
-  const bool own = inx;
-  const int q = par, qn = par ^ 1;
-  // the design table holds generic pointers; they all address device
-  // memory, and saying so gives global (not flat) loads, whose counters the
-  // compiler can wait on per load
-  const void* const EzA = D.ez[q];
-  const void* const HxA = D.hx[q];
-  const void* const HyA = D.hy[q];
-  void* const EzB = D.ez[qn];
-  void* const HxB = D.hx[qn];
-  void* const HyB = D.hy[qn];
-  const void* const psHxA = D.psi_hx[q];
-  const void* const psHyA = D.psi_hy[q];
-  void* const psHxB = D.psi_hx[qn];
-  void* const psHyB = D.psi_hy[qn];
-  void* const psEx = D.psi_ex;
-  void* const psEy = D.psi_ey;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int b = k.xcd ? tm_order(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const KWork wk = k.work[b];
+  const KDesign& KD = k.des[wk.d];
+  const pm_batch_design& D = KD.d;
+  const int x0 = wk.x0, y0 = wk.y0;
+  const int nx = D.nx;
+  TmGrid g;
+  g.nx = nx;
+  g.ny = D.ny;
+  g.sy = g.xst = g.yst = (uint32_t)D.sy;
+  g.px0 = D.pml[0];
+  g.px1 = D.pml[1];
+  g.py0 = D.pml[2];
+  g.py1 = D.pml[3];
+  g.ez = D.ez[par];
+  g.hx = D.hx[par];
+  g.hy = D.hy[par];
+  g.ez_o = D.ez[par ^ 1];
+  g.hx_o = D.hx[par ^ 1];
+  g.hy_o = D.hy[par ^ 1];
+  g.ca = nullptr;
+  g.cb = D.cb;
+  g.ps[0] = D.psi_hy[par];
+  g.ps[1] = D.psi_hx[par];
+  g.ps[2] = par ? KD.psi_ex1 : D.psi_ex;
+  g.ps[3] = par ? KD.psi_ey1 : D.psi_ey;
+  g.ps_o[0] = D.psi_hy[par ^ 1];
+  g.ps_o[1] = D.psi_hx[par ^ 1];
+  g.ps_o[2] = par ? D.psi_ex : KD.psi_ex1;
+  g.ps_o[3] = par ? D.psi_ey : KD.psi_ey1;
+  g.full = true;
+  g.idx = k.idx;
+  g.idy = k.idy;
+  g.db = D.db;
+  g.cb_scale = D.cb_scale;
   const gptr<const T> prof = (gptr<const T>)D.prof;
-  // y profiles, 8 per row: read-only for the launch, so scalar loads when
-  // a row needs them (no vector registers held for them across the
-  // prefetch)
-  using CT = const T __attribute__((address_space(4)))*;
-  const CT pyr = (CT)(prof + 6 * (int64_t)nx);
-
-  // x profiles of this lane (identity outside the slabs)
-  const bool xpml = inx && (i < D.pml[0] || i >= nx - D.pml[1]);
-  T bex = 1, cex = 0, ikex = 1, bhx = 1, chx = 0, ikhx = 1;
+  const int i = x0 - kTmS + lane;
+  const bool xpml = i >= 0 && i < nx && (i < g.px0 || i >= nx - g.px1);
+  TmXProf<T> xp{(T)0, (T)0, (T)1, (T)0, (T)0, (T)1};
   if (xpml) {
-    bex = prof[i];
-    cex = prof[nx + i];
-    ikex = prof[2 * nx + i];
-    bhx = prof[3 * nx + i];
-    chx = prof[4 * nx + i];
-    ikhx = prof[5 * nx + i];
+    xp.be = prof[i];
+    xp.ce = prof[nx + i];
+    xp.ike = prof[2 * nx + i];
+    xp.bh = prof[3 * nx + i];
+    xp.ch = prof[4 * nx + i];
+    xp.ikh = prof[5 * nx + i];
   }
-  // the same for the cell right of the strip, x0+64 (uniform)
-  const int ir = x0 + kStrip;
-  const bool rin = ir < nx;
-  const int irc = min(ir, nx - 1);
-  const bool xpml_r = rin && (ir < D.pml[0] || ir >= nx - D.pml[1]);
-  T bhx_r = 1, chx_r = 0, ikhx_r = 1;
-  if (xpml_r) {
-    bhx_r = prof[3 * nx + ir];
-    chx_r = prof[4 * nx + ir];
-    ikhx_r = prof[5 * nx + ir];
-  }
-  const T db = (T)D.db;
-  const T idx = (T)k.idx, idy = (T)k.idy;
-  const int64_t trow = step - k.table_step0;
-  const T se = (T)k.tab_e[trow];
-  const T sh = (T)k.tab_h[trow];
-  const gptr<T> Xrow = (gptr<T>)k.X + (step % k.sample_T) * (int64_t)k.ncols;
-  // everything the row loop needs from the design table, read once: the
-  // loop's stores could alias the table as far as the compiler knows
-  const int pml_y0 = D.pml[2], pml_y1 = ny - D.pml[3];
-  const bool srcE = i == D.src_e[0];
-  const bool srcH = i == D.src_h[0];
-  const int se0 = D.src_e[1], se1 = D.src_e[2];
-  const int sh0 = D.src_h[1], sh1 = D.src_h[2];
-  const T cbs = (T)D.cb_scale;
-  using CbT = typename RowE<T, CK>::CbT;
-  const void* const cbp = D.cb;
-  // sample lines at this lane's column (bit l: line l)
-  unsigned lmask = 0;
-  const int nl = D.n_lines;
-  for (int l = 0; l < nl; ++l)
-    if (D.line[l].i == i) lmask |= 1u << l;
-  if (!own) lmask = 0;
-  const bool cbx = inx && i < nx - 1;
-
-  // Every load of the row loop is issued on every path, from a clamped
-  // in-range position whose value is masked where it is used (lanes outside
-  // the design, rows past the last, cells outside a CPML slab), so the
-  // compiler's memory-counter waits do not cover the prefetched rows.
-  const int ic = min(i, nx - 1);
-  // the halo load: lane 1 Ez, lane 2 Hy, lane 3 the Hy CPML state (element
-  // 0 outside the x slabs) at x0+64; every other lane Ez(x0-1) (element 0
-  // of the row for the first strip)
-  const gptr<const T> hbase = (gptr<const T>)(lane == 2 ? HyA : (lane == 3 ? psHyA : EzA));
-  const int hcol = (lane == 1 || lane == 2 || (lane == 3 && xpml_r)) ? irc : max(x0 - 1, 0);
-  const bool hrow = !(lane == 3 && !xpml_r);  // false: element 0
-  const uint32_t syu = (uint32_t)sy;
-  auto load_h = [&](int j, RowH<T>& r) __attribute__((always_inline)) {
-    const int jc = min(j, ny - 1);
-    const uint32_t o = (uint32_t)jc * syu + (uint32_t)ic;
-    r.halo = hbase[hrow ? (int64_t)jc * sy + hcol : 0];
-    r.ez = ldg<T>(EzA, o);
-    r.hx = ldg<T>(HxA, o);
-    r.hy = ldg<T>(HyA, o);
-    // the CPML states are used in the slabs only: elsewhere every lane
-    // reads element 0 (one cache line per wave, no extra HBM traffic) and
-    // the value is not used
-    r.psx = ldg<T>(psHxA, (j < pml_y0 || j >= pml_y1) ? o : 0u);
-    r.psy = ldg<T>(psHyA, xpml ? o : 0u);
-  };
-  auto load_e = [&](int jj, RowE<T, CK>& r) __attribute__((always_inline)) {
-    const int jc = min(jj, ny - 1);
-    const uint32_t o = (uint32_t)jc * syu + (uint32_t)ic;
-    r.cb = ldg<CbT>(cbp, o);
-    r.pex = ldg<T>(psEx, xpml ? o : 0u);
-    r.pey = ldg<T>(psEy, (jj < pml_y0 || jj >= pml_y1) ? o : 0u);
-  };
-
-  const int r0 = w.r0, r1 = w.r1;
-  const int jend = min(r1, ny - 1);
-  const int elast = max(jend - 1, r0);  // last E row the tile updates (or r0)
-  T ezp = (r0 >= 1 && inx) ? ldg<T>(EzA, (uint32_t)(r0 - 1) * syu + (uint32_t)i) : (T)0;
-  T hxp = 0, hyp = 0, hyp_r = 0;
-  uint32_t bad = 0;  // bit 31: this lane computed an Inf or NaN Ez
-
-  // one row: H(n+1/2) at row j from `cur`, E(n+1) at row j-1 from `ecur`;
-  // first loads row j+2 into `nxt` and the E row j+1 into `enxt` (two rows
-  // ahead: the loads of two rows are in flight while one is computed)
-  auto body = [&](int j, const RowH<T>& cur, RowH<T>& nxt, const RowE<T, CK>& ecur,
-                  RowE<T, CK>& enxt) __attribute__((always_inline)) {
-    // rows past the tile are not used: the clamp makes those loads re-read
-    // a row already in the cache instead of fetching the next tile's rows
-    load_h(min(j + 2, jend), nxt);
-    load_e(min(j + 1, elast), enxt);
-    const uint32_t o = (uint32_t)j * syu + (uint32_t)i;
-    const bool store_h = own && j < r1;
-    const bool yp = j < pml_y0 || j >= pml_y1;
-    const T ezc = inx ? cur.ez : (T)0;
-
-    // Hx(i, j) -= Db * dEz/dy (backward difference, Ez(j = -1) = 0)
-    T dy = (ezc - ezp) * idy;
-    if (yp) {
-      const CT q = pyr + 8 * j;
-      const T ps = q[3] * cur.psx + q[4] * dy;
-      if (store_h) stg<T>(psHxB, o, ps);
-      dy = dy * q[5] + ps;
-    }
-    const T hxn = (inx && i < nx - 1) ? cur.hx - db * dy : (T)0;
-
-    // Hy(i, j) += Db * dEz/dx, Ez(i-1) from the lane below (lane 0: the
-    // halo value, zero left of the grid)
-    const T ezh = x0 > 0 ? lane_value(cur.halo, 0) : (T)0;
-    const T ezs = __shfl_up(ezc, 1);
-    const T ezl = lane == 0 ? ezh : ezs;
-    T dx = (ezc - ezl) * idx;
-    if (xpml) {
-      const T ps = bhx * cur.psy + chx * dx;
-      if (store_h) stg<T>(psHyB, o, ps);
-      dx = dx * ikhx + ps;
-    }
-    const T hyn = (inx && j < ny - 1) ? cur.hy + db * dx : (T)0;
-    // Hy(n+1/2) at x0+64 for lane 63's E update: the next strip's lane 0
-    // arithmetic on the halo values (not stored)
-    T dxr = (lane_value(cur.halo, 1) - lane_value(ezc, 63)) * idx;
-    if (xpml_r) {
-      const T ps = bhx_r * lane_value(cur.halo, 3) + chx_r * dxr;
-      dxr = dxr * ikhx_r + ps;
-    }
-    const T hyn_r = (rin && j < ny - 1) ? lane_value(cur.halo, 2) + db * dxr : (T)0;
-
-    if (store_h) {
-      stg<T>(HxB, o, hxn);
-      const T hys = (srcH && j >= sh0 && j < sh1) ? hyn + sh : hyn;
-      stg<T>(HyB, o, hys);
-      if (lmask) {
-        // a constant trip count (lmask holds no bit at or past nl): stores
-        // in a loop of run-time length would make the compiler wait for
-        // every access in flight, the row prefetch included
-#pragma unroll
-        for (int l = 0; l < PM_BATCH_MAX_LINES; ++l) {
-          if (!((lmask >> l) & 1u)) continue;
-          const pm_batch_line L = D.line[l];
-          if (L.comp != 0 && j >= L.j0 && j < L.j1)
-            Xrow[L.col + (j - L.j0)] = L.comp == 2 ? hys : hxn;
-        }
-      }
-    }
-
-    if (j > r0) {
-      // Ez(i, jj) += Cb (dHy/dx - dHx/dy) with the new H of rows jj, jj+1
-      const int jj = j - 1;
-      const uint32_t oe = o - syu;
-      const T hys1 = __shfl_down(hyp, 1);
-      const T hyr = lane == 63 ? hyp_r : hys1;
-      const bool valid = cbx && jj < ny - 1;
-      T tx = (hyr - hyp) * idx;
-      if (xpml && valid) {
-        const T ps = bex * ecur.pex + cex * tx;
-        if (own) stg<T>(psEx, oe, ps);
-        tx = tx * ikex + ps;
-      }
-      T ty = (hxn - hxp) * idy;
-      if ((jj < pml_y0 || jj >= pml_y1) && valid) {
-        const CT q = pyr + 8 * jj;
-        const T ps = q[0] * ecur.pey + q[1] * ty;
-        if (own) stg<T>(psEy, oe, ps);
-        ty = ty * q[2] + ps;
-      }
-      T cb;
-      if constexpr (CK == PM_COEFF_CB_F16) {
-        __half_raw hr;
-        hr.x = ecur.cb;
-        cb = cbs * (T)__half2float(__half(hr));
-      } else {
-        cb = ecur.cb;
-      }
-      T ezn = (T)0;
-      if (valid) {
-        ezn = ezp + cb * (tx - ty);
-        if (srcE && jj >= se0 && jj < se1) ezn += se;
-        bad |= nonfinite_bit(ezn);
-      }
-      if (own) {
-        stg<T>(EzB, oe, ezn);
-        if (lmask) {
-#pragma unroll
-          for (int l = 0; l < PM_BATCH_MAX_LINES; ++l) {
-            if (!((lmask >> l) & 1u)) continue;
-            const pm_batch_line L = D.line[l];
-            if (L.comp == 0 && jj >= L.j0 && jj < L.j1) Xrow[L.col + (jj - L.j0)] = ezn;
-          }
-        }
-      }
-    }
-    ezp = ezc;
-    hxp = hxn;
-    hyp = hyn;
-    hyp_r = hyn_r;
-  };
-
-  // three register sets in rotation: iteration j computes from set
-  // (j - r0) % 3 and loads into set (j - r0 + 2) % 3
-  RowH<T> h0, h1, h2;
-  RowE<T, CK> e0, e1, e2;
-  load_h(r0, h0);
-  load_h(min(r0 + 1, jend), h1);
-  e0 = RowE<T, CK>{};  // E row r0 - 1: not updated by this tile
-  load_e(r0, e1);
-  for (int j = r0;;) {
-    body(j, h0, h2, e0, e2);
-    if (++j > jend) break;
-    body(j, h1, h0, e1, e0);
-    if (++j > jend) break;
-    body(j, h2, h1, e2, e1);
-    if (++j > jend) break;
-  }
-  // a diverged design is flagged once per tile (rare: a vector atomic from
-  // the lanes that saw it)
-  if (bad >> 31) atomicOr(k.status + w.d, 1);
+  const BatchY<T> yp{prof + 6 * (int64_t)nx};
+  BatchIo<T> io{k, D, use_clock ? *k.clock + s_rel : step_arg, x0, y0, tm_rows(R)};
+  const uint32_t bad = tm_tile<T, CK, R>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+  // a diverged design is flagged by the lanes that saw it (rare)
+  if (bad >> 31) atomicOr(k.status + wk.d, 1);
 }
 
 __global__ void k_clock_set(int64_t* clock, int64_t v) {
@@ -404,6 +227,7 @@ struct pm_batch {
   pm_batch_plan plan{};
   std::vector<pm_batch_design> des;
   std::vector<KWork> work;
+  int rows = 4;  // rows per wave of a tile
   KBatch kb{};
   KDft dft{};
   int64_t step = 0;   // absolute index of the next step
@@ -411,9 +235,10 @@ struct pm_batch {
   int64_t pend0 = 0;  // first step of the pending sample block
   int pend_n = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
-  int waves = 4;  // launch shape of the step kernel (pm_batch_set_tuning)
-  int xcd = 1;
+  int n_cu = 256;
+  int xcd = 1;  // workgroup order (pm_batch_set_tuning)
   bool timing = false;
+  int64_t timed_steps = 0;  // steps in spans[0]
   std::vector<std::pair<hipEvent_t, hipEvent_t>> spans[3];
   std::string err;
 };
@@ -455,24 +280,36 @@ struct BSpan {
 int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 // Workspace: the step clock at offset 0, then the design table, the tile
-// list and one status word per design.
-void layout(const pm_batch_plan& p, int64_t* des_off, int64_t* work_off, int64_t* status_off,
-            int64_t* total, int64_t n_work) {
-  *des_off = 256;
-  *work_off = align256(*des_off + (int64_t)sizeof(pm_batch_design) * p.n_design);
-  *status_off = align256(*work_off + (int64_t)sizeof(KWork) * n_work);
-  *total = align256(*status_off + (int64_t)sizeof(int32_t) * p.n_design);
-}
+// list, one status word per design and the second E-side CPML memory.
+struct Layout {
+  int64_t des, work, status, psi, total;
+};
 
-void build_work(const pm_batch_plan& p, std::vector<KWork>& work) {
+void build_work(const pm_batch_plan& p, int rows, std::vector<KWork>& work) {
   work.clear();
-  const int ch = p.chunk;
   for (int d = 0; d < p.n_design; ++d) {
     const pm_batch_design& D = p.design[d];
-    for (int r0 = 0; r0 < D.ny; r0 += ch)
-      for (int x0 = 0; x0 < D.nx; x0 += kStrip)
-        work.push_back(KWork{d, x0, r0, std::min(r0 + ch, D.ny)});
+    for (int y0 = 0; y0 < D.ny; y0 += tm_rows(rows))
+      for (int x0 = 0; x0 < D.nx; x0 += kTmCols) work.push_back(KWork{d, x0, y0});
   }
+}
+
+int64_t psi_bytes(const pm_batch_plan& p, const pm_batch_design& D) {
+  return align256((int64_t)D.ny * D.sy * (p.precision == PM_FP64 ? 8 : 4));
+}
+
+// (sized for the shortest tiles, whichever the device gets)
+Layout layout(const pm_batch_plan& p) {
+  std::vector<KWork> w;
+  build_work(p, 4, w);
+  Layout l{};
+  l.des = 256;
+  l.work = align256(l.des + (int64_t)sizeof(KDesign) * p.n_design);
+  l.status = align256(l.work + (int64_t)(sizeof(KWork) * w.size()));
+  l.psi = align256(l.status + (int64_t)sizeof(int32_t) * p.n_design);
+  l.total = l.psi;
+  for (int d = 0; d < p.n_design; ++d) l.total += 2 * psi_bytes(p, p.design[d]);
+  return l;
 }
 
 int validate(pm_batch* b, const pm_batch_plan& p) {
@@ -533,22 +370,31 @@ int validate(pm_batch* b, const pm_batch_plan& p) {
   return 0;
 }
 
-template <typename T>
-int launch_step(pm_batch* b, int64_t step_arg, int use_clock, int s_rel, int par) {
-  const int wv = b->kb.waves;
-  const int nb = ((int)b->work.size() + wv - 1) / wv;
-  if (b->plan.coeff_kind == PM_COEFF_CB_F16)
-    hipLaunchKernelGGL((k_batch_tm<T, PM_COEFF_CB_F16>), dim3(nb), dim3(64 * wv), 0,
-                       b->stream, b->kb, step_arg, use_clock, s_rel, par);
-  else
-    hipLaunchKernelGGL((k_batch_tm<T, PM_COEFF_CB>), dim3(nb), dim3(64 * wv), 0,
-                       b->stream, b->kb, step_arg, use_clock, s_rel, par);
-  return bhip(b, hipGetLastError(), "batch step launch");
+template <typename T, int CK>
+void launch_ck(pm_batch* b, int64_t step_arg, int use_clock, int s_rel, int ns, int par) {
+  const dim3 nb((unsigned)b->work.size()), nt(64 * kTmW);
+  if constexpr (sizeof(T) == 4) {
+    if (b->rows == 8) {
+      hipLaunchKernelGGL((k_batch_tm<T, CK, 8>), nb, nt, 0, b->stream, b->kb, step_arg,
+                         use_clock, s_rel, ns, par);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_batch_tm<T, CK, 4>), nb, nt, 0, b->stream, b->kb, step_arg, use_clock,
+                     s_rel, ns, par);
 }
 
-int step_once(pm_batch* b, int64_t step, int use_clock, int s_rel, int par) {
-  return b->plan.precision == PM_FP64 ? launch_step<double>(b, step, use_clock, s_rel, par)
-                                      : launch_step<float>(b, step, use_clock, s_rel, par);
+// ns steps from set `par` into the other
+int launch_steps(pm_batch* b, int64_t step, int use_clock, int s_rel, int ns, int par) {
+  const bool f16 = b->plan.coeff_kind == PM_COEFF_CB_F16;
+  if (b->plan.precision == PM_FP64) {
+    if (f16) launch_ck<double, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, par);
+    else launch_ck<double, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, par);
+  } else {
+    if (f16) launch_ck<float, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, par);
+    else launch_ck<float, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, par);
+  }
+  return bhip(b, hipGetLastError(), "batch step launch");
 }
 
 int flush_block(pm_batch* b, int64_t first, int rows, const int64_t* wclock) {
@@ -562,13 +408,15 @@ int flush_block(pm_batch* b, int64_t first, int rows, const int64_t* wclock) {
   return bhip(b, hipGetLastError(), "batch DFT launch");
 }
 
-int capture(pm_batch* b, int par) {
+int capture(pm_batch* b, int slot) {
+  int par = slot;
   const pm_batch_plan& p = b->plan;
   hipGraph_t g = nullptr;
   int r = bhip(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
                "begin capture");
   if (r) return r;
-  for (int s = 0; s < p.sample_T && !r; ++s) r = step_once(b, 0, 1, s, par ^ (s & 1));
+  for (int s = 0; s < p.sample_T && !r; s += kTmS, par ^= 1)
+    r = launch_steps(b, 0, 1, s, std::min(kTmS, p.sample_T - s), par);
   if (!r) r = flush_block(b, 0, p.sample_T, b->kb.clock);
   if (!r) {
     hipLaunchKernelGGL(k_clock_add, dim3(1), dim3(64), 0, b->stream, b->kb.clock,
@@ -582,7 +430,7 @@ int capture(pm_batch* b, int par) {
   }
   r = bhip(b, e, "end capture");
   if (r) return r;
-  r = bhip(b, hipGraphInstantiate(&b->graph[par], g, nullptr, nullptr, 0), "instantiate");
+  r = bhip(b, hipGraphInstantiate(&b->graph[slot], g, nullptr, nullptr, 0), "instantiate");
   (void)hipGraphDestroy(g);
   return r;
 }
@@ -610,6 +458,10 @@ int pm_batch_create(int device, void* stream, pm_batch** out) {
   if (e != hipSuccess) return (int)e;
   pm_batch* b = new pm_batch();
   b->device = device;
+  int cu = 0;
+  if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
+      cu > 0)
+    b->n_cu = cu;
   b->stream = (hipStream_t)stream;
   *out = b;
   return 0;
@@ -632,11 +484,7 @@ const char* pm_batch_last_error(pm_batch* b) { return b ? b->err.c_str() : "null
 
 int pm_batch_workspace_bytes(const pm_batch_plan* p, int64_t* bytes) {
   if (!p || !bytes || p->n_design < 1 || !p->design || p->chunk < 2) return PM_EINVAL;
-  std::vector<KWork> w;
-  build_work(*p, w);
-  int64_t a, c, st, t;
-  layout(*p, &a, &c, &st, &t, (int64_t)w.size());
-  *bytes = t;
+  *bytes = layout(*p).total;
   return 0;
 }
 
@@ -647,24 +495,31 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   drop_graphs(b);
   int r = validate(b, *p);
   if (r) return r;
+  const Layout l = layout(*p);
+  if (!p->work || p->work_bytes < l.total)
+    return bfail(b, PM_EINVAL, "workspace of %lld bytes required", (long long)l.total);
+  double cells = 0;
+  for (int d = 0; d < p->n_design; ++d) cells += (double)p->design[d].nx * p->design[d].ny;
+  b->rows = tm_pick_rows(cells, p->precision == PM_FP64 ? 8 : 4, b->n_cu);
   std::vector<KWork> work;
-  build_work(*p, work);
-  int64_t des_off, work_off, status_off, total;
-  layout(*p, &des_off, &work_off, &status_off, &total, (int64_t)work.size());
-  if (!p->work || p->work_bytes < total)
-    return bfail(b, PM_EINVAL, "workspace of %lld bytes required", (long long)total);
+  build_work(*p, b->rows, work);
   b->plan = *p;
   b->des.assign(p->design, p->design + p->n_design);
   b->plan.design = b->des.data();
   b->work = std::move(work);
   char* ws = (char*)p->work;
+  std::vector<KDesign> kd(b->des.size());
+  char* psi = ws + l.psi;
+  for (size_t d = 0; d < kd.size(); ++d) {
+    const int64_t n = psi_bytes(*p, b->des[d]);
+    kd[d] = KDesign{b->des[d], psi, psi + n};
+    psi += 2 * n;
+  }
   KBatch& k = b->kb;
   k.clock = (int64_t*)ws;
-  k.des = (const pm_batch_design*)(ws + des_off);
-  k.work = (const KWork*)(ws + work_off);
-  k.status = (int32_t*)(ws + status_off);
-  k.n_work = (int)b->work.size();
-  k.waves = b->waves;
+  k.des = (const KDesign*)(ws + l.des);
+  k.work = (const KWork*)(ws + l.work);
+  k.status = (int32_t*)(ws + l.status);
   k.xcd = b->xcd;
   k.ncols = p->ncols;
   k.sample_T = p->sample_T;
@@ -676,9 +531,8 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   k.X = p->X;
   b->dft = KDft{p->dft.col0, p->dft.col1, p->dft.f0, p->dft.f1, p->dft.acc_re,
                 p->dft.acc_im, p->dft.cmp_re, p->dft.cmp_im};
-  r = bhip(b, hipMemcpyAsync((void*)k.des, b->des.data(),
-                             sizeof(pm_batch_design) * b->des.size(), hipMemcpyHostToDevice,
-                             b->stream), "design table upload");
+  r = bhip(b, hipMemcpyAsync((void*)k.des, kd.data(), sizeof(KDesign) * kd.size(),
+                             hipMemcpyHostToDevice, b->stream), "design table upload");
   if (!r)
     r = bhip(b, hipMemcpyAsync((void*)k.work, b->work.data(), sizeof(KWork) * b->work.size(),
                                hipMemcpyHostToDevice, b->stream), "tile list upload");
@@ -688,7 +542,7 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   if (!r)
     r = bhip(b, hipMemcpyAsync(k.status, zeros.data(), sizeof(int32_t) * zeros.size(),
                                hipMemcpyHostToDevice, b->stream), "status upload");
-  // the uploads read pageable host memory owned by this object: finish them
+  // the uploads read pageable host memory: finish them
   if (!r) r = bhip(b, hipStreamSynchronize(b->stream), "upload sync");
   if (r) return r;
   b->step = p->table_step0;
@@ -732,23 +586,27 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
         r = bhip(b, hipGraphLaunch(b->graph[b->parity], b->stream), "graph launch");
       }
       if (r) return r;
+      b->parity ^= ((T + kTmS - 1) / kTmS) & 1;
       b->step += T;
       b->pend0 = b->step;
       left -= T;
       continue;
     }
     clock_ok = false;
+    // a launch does not cross the end of a sample block
+    const int m = (int)std::min<int64_t>({kTmS, left, T - b->step % T});
     int r;
     {
       BSpan sp(b, 0);
-      r = step_once(b, b->step, 0, 0, b->parity);
+      r = launch_steps(b, b->step, 0, 0, m, b->parity);
     }
     if (r) return r;
+    if (b->timing) b->timed_steps += m;
     if (b->pend_n == 0) b->pend0 = b->step;
-    ++b->pend_n;
+    b->pend_n += m;
     b->parity ^= 1;
-    ++b->step;
-    --left;
+    b->step += m;
+    left -= m;
     if (b->step % T == 0) {
       BSpan sp(b, 1);
       r = flush_block(b, b->pend0, b->pend_n, nullptr);
@@ -786,9 +644,8 @@ int pm_batch_set_tuning(pm_batch* b, int waves, int xcd_order) {
     return bfail(b, PM_EINVAL, "waves per workgroup must be 1, 2, 4 or 8");
   if (xcd_order != 0 && xcd_order != 1) return bfail(b, PM_EINVAL, "xcd_order must be 0 or 1");
   (void)hipSetDevice(b->device);
-  // a captured graph holds the old launch shape
+  // a captured graph holds the old workgroup order
   drop_graphs(b);
-  b->waves = b->kb.waves = waves;
   b->xcd = b->kb.xcd = xcd_order;
   return 0;
 }
@@ -811,6 +668,7 @@ int pm_batch_design_status(pm_batch* b, int32_t* out, int32_t n) {
 int pm_batch_set_timing(pm_batch* b, int enable) {
   if (!b) return PM_EINVAL;
   b->timing = enable != 0;
+  b->timed_steps = 0;
   for (auto& v : b->spans) {
     for (auto& ab : v) {
       (void)hipEventDestroy(ab.first);
@@ -834,6 +692,8 @@ int pm_batch_get_timing(pm_batch* b, int which, double* avg_ms, int64_t* count) 
       ++n;
     }
   }
+  // a launch holds several steps: class 0 counts those
+  if (which == 0 && n) n = b->timed_steps;
   *avg_ms = n ? tot / n : 0.0;
   *count = n;
   return 0;

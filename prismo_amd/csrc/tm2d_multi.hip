@@ -104,12 +104,10 @@ struct SimIo {
 #pragma unroll
     for (int k = 1; k < kTmS / 4; ++k) v = s / 4 == k ? tm_bcast(value[k], t * 4 + (s & 3)) : v;
     const bool in = i >= b0 && i < b1;
+    if (c0 >= jb + R || c1 <= jb) return;  // uniform
     if (of(kind, t) == 0) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int j = jb + r;
-        f[r] = in && j >= c0 && j < c1 ? f[r] + (T)v : f[r];
-      }
+      const T u = (T)v;
+      tm_add([&](int) { return u; }, in, c0, c1, jb, f);
       return;
     }
     // the profile's values of all rows from clamped positions, without a
@@ -128,11 +126,7 @@ struct SimIo {
 #pragma unroll
       for (int r = 0; r < R; ++r) u[r] = u[r] / d;
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int j = jb + r;
-      f[r] = in && j >= c0 && j < c1 ? f[r] + (T)u[r] : f[r];
-    }
+    tm_add([&](int r) { return (T)u[r]; }, in, c0, c1, jb, f);
   }
 
   template <int R>
@@ -147,26 +141,22 @@ struct SimIo {
   }
 
   template <int R>
-  __device__ __forceinline__ void put(int t, int s, int i, int jb, int t0, const T (&f)[R]) const {
+  __device__ __forceinline__ void put(int t, int s, int i, int jb, const T (&f)[R]) const {
     const int b0 = of(i0, t), b1 = of(i1, t), c0 = of(j0, t), c1 = of(j1, t), ni = b1 - b0;
     const bool in = i >= max(b0, x0) && i < min(b1, x0 + kTmCols);
-    const gptr<T> X = (gptr<T>)a.X + (a.xrow + s) * (int64_t)a.ncols + of(kind, t);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int j = jb + r, q = t0 + r;
-      if (q < kTmS || q >= rows + kTmS || j < c0 || j >= c1) continue;  // uniform
-      if (in) X[(int64_t)(j - c0) * ni + (i - b0)] = f[r];
-    }
+    const gptr<T> X = (gptr<T>)a.X + (a.xrow + s) * (int64_t)a.ncols + of(kind, t) + (i - b0);
+    const int p0 = max(c0, y0), p1 = min(c1, y0 + rows);  // rows the tile writes
+    tm_put(X + (int64_t)(p0 - c0) * ni, ni, in, p0, p1, jb, f);
   }
 
   template <int R>
-  __device__ __forceinline__ void samples(int s, int i, int jb, int t0, const T (&ez)[R],
+  __device__ __forceinline__ void samples(int s, int i, int jb, const T (&ez)[R],
                                           const T (&hx)[R], const T (&hy)[R]) const {
     for (unsigned m = bmask; m; m &= m - 1) {
       const int t = kMaxSrc + __builtin_ctz(m), c = of(comp, t);
-      if (c == PM_EZ) put(t, s, i, jb, t0, ez);
-      else if (c == PM_HX) put(t, s, i, jb, t0, hx);
-      else put(t, s, i, jb, t0, hy);
+      if (c == PM_EZ) put(t, s, i, jb, ez);
+      else if (c == PM_HX) put(t, s, i, jb, hx);
+      else put(t, s, i, jb, hy);
     }
   }
 };

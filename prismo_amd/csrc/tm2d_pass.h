@@ -6,10 +6,10 @@
 // pays a launch and a chain of row loads each time: a 540 x 290 FP64 grid took
 // 11.6 us a step with its sources and samples, of which its 157 k cells need
 // well under 1; a 2000 x 1500 FP32 one 26.6 us.  A pass of 8 steps reads the
-// state once, with a halo of 8 cells, and writes it once: 2.1 us and 5.0 us a
+// state once, with a halo of 8 cells, and writes it once: 2.0 us and 4.9 us a
 // step.  What is left is latency (a pass of the small grid waits for its loads,
 // 16 barriers and the source table) and, on large grids, the vector ALU:
-// about 15 instructions a cell and step, halo cells included.
+// 13 instructions a cell and step, halo cells included, 20 in a CPML layer.
 //
 // Tile: 8 waves stacked in y, each 64 columns (one per lane) by R rows in
 // registers; 8 cells on each side are halo (a step's E depends on fields one
@@ -78,6 +78,41 @@ __device__ __forceinline__ T tm_bcast(T v, int l) {
   }
 }
 
+// f[r] of rows j0 .. j1 - 1 (the wave's first row: jb) to x[(row - j0) stride], for
+// lanes with `in`.  A wave whose rows are all wanted, the usual case of a line
+// along y, or none, makes no test per row: with one, the tiles that sample took
+// twice as long as the others.
+template <typename T, int R>
+__device__ __forceinline__ void tm_put(gptr<T> x, int stride, bool in, int j0, int j1, int jb,
+                                       const T (&f)[R]) {
+  const int a = j0 - jb, b = j1 - jb;  // uniform
+  if (a >= R || b <= 0) return;
+  x -= (int64_t)a * stride;
+  if (a <= 0 && b >= R) {
+    if (in) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) x[r * stride] = f[r];
+    }
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (r >= a && r < b && in) x[r * stride] = f[r];
+}
+
+// f[r] += v[r] on rows j0 .. j1 - 1, for lanes with `in`.
+template <typename T, int R, class V>
+__device__ __forceinline__ void tm_add(const V& v, bool in, int j0, int j1, int jb, T (&f)[R]) {
+  const int a = j0 - jb, b = j1 - jb;
+  if (a <= 0 && b >= R) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) f[r] = in ? f[r] + v(r) : f[r];
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) f[r] = in && r >= a && r < b ? f[r] + v(r) : f[r];
+}
+
 // One grid as a pass sees it (uniform): offsets are 32-bit elements.
 struct TmGrid {
   int nx, ny;
@@ -104,8 +139,11 @@ struct TmXProf {
 
 template <typename T, int R>
 struct TmShared {
-  T e[kTmW][64], h[kTmW][64];  // last row of Ez, first row of Hx of each wave
-  T y[kTmW * R][6];            // y profiles of the rows (be ce ike bh ch ikh)
+  // Ez of each wave's last row (behind a row of zeros), Hx of each wave's first
+  // row (before one)
+  T e[kTmW + 1][64], h[kTmW + 1][64];
+  // y profiles of the rows, E (be ce ike -) and H (bh ch ikh -): 16-byte reads
+  alignas(16) T y[kTmW * R][2][4];
 };
 
 // ns steps of the tile (x0, y0: first column and row it writes) by this wave.
@@ -158,6 +196,11 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     else
       cb[r] = ((gptr<const T>)g.cb)[o];
     if constexpr (CK == PM_COEFF_CACB) ca[r] = ((gptr<const T>)g.ca)[o];
+    // positions without Ez hold 0 and stay so
+    if (!(ok && le_ok) || (YP && j >= ny - 1)) {
+      ez[r] = cb[r] = (T)0;
+      if constexpr (CK == PM_COEFF_CACB) ca[r] = (T)0;
+    }
     if constexpr (XP) {
       const uint32_t q = xpml ? xo + g.xst * (uint32_t)jc : 0u;
       const T h = ((gptr<const T>)g.ps[0])[q], f = ((gptr<const T>)g.ps[2])[q];
@@ -181,22 +224,24 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
       const bool in = ypml(j);
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
-        sh.y[w * R + lane][k] = in ? yp(k, j) : (T)(k % 3 == 2 ? 1 : 0);
+        sh.y[w * R + lane][k / 3][k % 3] = in ? yp(k, j) : (T)(k % 3 == 2 ? 1 : 0);
       }
     }
   }
+  if (w == 0) sh.e[0][lane] = (T)0;
+  if (w == kTmW - 1) sh.h[kTmW][lane] = (T)0;
   io.second(ns);
   uint32_t bad = 0;
   for (int s = 0; s < ns; ++s) {
-    // the row number is made opaque per step: the tests on it are one scalar
-    // compare each, but hoisted out of the loop they would hold a mask per row
-    // in SGPRs and spill
+    // the row number is made opaque per step: the tests of the sources and samples
+    // on it are one scalar compare each, but hoisted out of the loop they would
+    // hold a mask per row in SGPRs and spill
     int js = jb;
     asm volatile("" : "+s"(js));
     // H: backward differences of E
-    sh.e[w][lane] = ez[R - 1];
+    sh.e[w + 1][lane] = ez[R - 1];
     __syncthreads();
-    T below = w > 0 ? sh.e[w > 0 ? w - 1 : 0][lane] : (T)0;
+    T below = sh.e[w][lane];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       // (outside the layers the profiles leave a difference as it is, so every
@@ -204,9 +249,9 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
       T d1 = (ez[r] - below) * idy;
       T d2 = (ez[r] - tm_lane<0x138>(ez[r])) * idx;
       if constexpr (YP) {
-        const T* y = sh.y[w * R + r];
-        qhy[r] = tm_fma(y[3], qhy[r], y[4] * d1);
-        d1 = tm_fma(d1, y[5], qhy[r]);
+        const T* y = sh.y[w * R + r][1];
+        qhy[r] = tm_fma(y[0], qhy[r], y[1] * d1);
+        d1 = tm_fma(d1, y[2], qhy[r]);
       }
       if constexpr (XP) {
         qhx[r] = tm_fma(xp.bh, qhx[r], xp.ch * d2);
@@ -219,10 +264,9 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     // E: forward differences of H
     sh.h[w][lane] = hx[0];
     __syncthreads();
-    const T above = w + 1 < kTmW ? sh.h[w + 1 < kTmW ? w + 1 : 0][lane] : (T)0;
+    const T above = sh.h[w + 1][lane];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int j = js + r;
       T e1 = (tm_lane<0x130>(hy[r]) - hy[r]) * idx;
       T e2 = ((r + 1 < R ? hx[r + 1 < R ? r + 1 : 0] : above) - hx[r]) * idy;
       if constexpr (XP) {
@@ -230,7 +274,7 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
         e1 = tm_fma(e1, xp.ike, qex[r]);
       }
       if constexpr (YP) {
-        const T* y = sh.y[w * R + r];
+        const T* y = sh.y[w * R + r][0];
         qey[r] = tm_fma(y[0], qey[r], y[1] * e2);
         e2 = tm_fma(e2, y[2], qey[r]);
       }
@@ -240,15 +284,10 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
         v = tm_fma(cb[r], c, ca[r] * ez[r]);
       else
         v = tm_fma(cb[r], c, ez[r]);
-      // cells beyond the grid stay 0 (only tiles at its edges have any)
-      if constexpr (XP) v = le_ok ? v : (T)0;
-      if constexpr (YP) {
-        if (j < 0 || j >= ny - 1) v = (T)0;
-      }
       ez[r] = v;
     }
     io.sources(s, i, js, ez, hx, hy);
-    io.samples(s, i, js, w * R, ez, hx, hy);
+    io.samples(s, i, js, ez, hx, hy);
   }
   const bool mine = lane >= kTmS && lane < 64 - kTmS && lin;
   if (!mine) return 0;

@@ -53,7 +53,10 @@ def component_average(A: np.ndarray, comp: str, is_2d: bool) -> np.ndarray:
         if comp == "Ey" or comp == "Hx":
             return 0.5 * (A[:-1, :] + A[1:, :])
         if comp == "Ez":
-            return 0.25 * (A[:-1, :-1] + A[1:, :-1] + A[:-1, 1:] + A[1:, 1:])
+            s = A[:-1, :-1] + A[1:, :-1]
+            s += A[:-1, 1:]
+            s += A[1:, 1:]
+            return 0.25 * s
         if comp == "Hz":
             return A
         raise ValueError(comp)

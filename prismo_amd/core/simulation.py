@@ -265,8 +265,8 @@ class Simulation:
     def _use_graph(self, eng, T: int) -> bool:
         if not self.graph or T % 2:
             return False
-        # two steps per launch (large grids) are not captured
-        return eng.ctx.fused_steps() != 2
+        # 3-D, two steps per launch (large grids): not captured
+        return self.grid.is_2d or eng.ctx.fused_steps() != 2
 
     def _small_grid(self) -> bool:
         """Launch-bound: 2-D, or 3-D up to 2^21 cells."""

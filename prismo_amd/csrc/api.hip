@@ -39,6 +39,7 @@ struct pm_ctx {
   // 2-D compat gate flags: the set the next H update fills (0 / 1) and the
   // set the E update of the current step reads
   int flag_set = 0, flag_set_e = 0;
+  bool flags_carried = false;  // flag_set is already filled for the next H update
   int parity = 0;
   // two steps per launch: plan eligible, and which E-side CPML memory set
   // holds the state (0 = plan.psi_e, 1 = plan.psi_e2)
@@ -329,7 +330,8 @@ int launch_status(pm_ctx* c, const char* what) {
 
 // The gate flag sets of a 2-D compat step: `set` filled before the H
 // update and read by it and the E update, the other one cleared by the H
-// kernel for the next step.
+// kernel and, with another step to come in this run, filled for it by the E
+// and source kernels (flags_carried).
 KGrid flag_grid(const pm_ctx* c, int set) {
   KGrid g = c->g;
   g.flags = c->g.flags + 8 * set;
@@ -343,7 +345,8 @@ int do_h(pm_ctx* c) {
   if (p.scheme == PM_SCHEME_COMPAT) {
     if (p.ndim == 2) {
       const KGrid g = flag_grid(c, c->flag_set);
-      launch_compat_flags2d(g, c->stream);
+      if (!c->flags_carried) launch_compat_flags2d(g, c->stream);
+      c->flags_carried = false;
       launch_compat_h(g, p.coeff_kind, c->stream);
       c->flag_set_e = c->flag_set;
       c->flag_set ^= 1;
@@ -356,15 +359,36 @@ int do_h(pm_ctx* c) {
   return launch_status(c, "H update launch");
 }
 
-int do_e(pm_ctx* c) {
+// Steps of this context may carry the gate flags on.  Not where source boxes of
+// one component overlap (a cell's flag is only right after the last of them) or
+// reach past the component's extent (those cells count for no gate).
+bool carries_flags(const pm_ctx* c) {
+  const pm_plan& p = c->plan;
+  if (p.scheme != PM_SCHEME_COMPAT || p.ndim != 2 || !c->aux.src_merge) return false;
+  for (int t = 0; t < c->aux.n_src; ++t) {
+    const KSrc& s = c->aux.src[t];
+    const bool x = s.comp == PM_EZ || s.comp == PM_EY, y = s.comp == PM_EZ || s.comp == PM_EX;
+    if ((x && s.i1 > p.nx - 1) || (y && s.j1 > p.ny - 1)) return false;
+  }
+  return true;
+}
+
+// carry: the flags of the next step's H update are filled (the caller gives
+// next_flags() to the source kernels when src).
+int do_e(pm_ctx* c, bool carry = false, bool src = false) {
   Span sp(c, 1);
   const pm_plan& p = c->plan;
   if (p.scheme == PM_SCHEME_COMPAT)
-    launch_compat_e(p.ndim == 2 ? flag_grid(c, c->flag_set_e) : c->g, p.coeff_kind, c->stream);
+    launch_compat_e(p.ndim == 2 ? flag_grid(c, c->flag_set_e) : c->g, p.coeff_kind, carry,
+                    c->aux.src_dev, src ? c->aux.n_src : 0, c->stream);
   else
     launch_yee_e(c->g, p.precision, p.coeff_kind, c->stream);
+  c->flags_carried = carry;
   return launch_status(c, "E update launch");
 }
+
+// The flag set the next H update reads (after do_h: the one its kernel cleared).
+int* next_flags(const pm_ctx* c) { return c->g.flags + 8 * c->flag_set; }
 
 // Cells per lane and waves per row of the fused kernel for this plan.
 // Launch shape of the fused kernel: the tuned one, else (rows per workgroup
@@ -995,6 +1019,7 @@ int pm_configure(pm_ctx* c, const pm_plan* plan) {
   c->pend_n = 0;
   // both gate flag sets start cleared (2-D compat)
   c->flag_set = c->flag_set_e = 0;
+  c->flags_carried = false;
   if (p.scheme == PM_SCHEME_COMPAT && p.ndim == 2) {
     launch_compat_flags_clear(c->g.flags, c->stream);
     int r = launch_status(c, "flag clear launch");
@@ -1094,25 +1119,28 @@ int64_t* step_clock(const pm_ctx* c) {
 
 // One step launched directly: fields (in place, or one ping-pong step),
 // sources, samples.
-int eager_step(pm_ctx* c, int64_t n, bool in_place, bool fused, bool src, bool smp, bool dft) {
+// more: another step of the run follows this one directly.
+int eager_step(pm_ctx* c, int64_t n, bool in_place, bool fused, bool src, bool smp, bool dft,
+               bool more = false) {
   Span whole(c, 2);
   int r;
   if (fused && !in_place) {
     r = do_fused(c);
   } else {
     r = do_h(c);
-    if (!r) r = do_e(c);
+    if (!r) r = do_e(c, more && carries_flags(c), src);
   }
   if (r) return r;
+  int* const fill = c->flags_carried ? next_flags(c) : nullptr;
   const KAux& ax = c->parity ? c->aux2 : c->aux;
   if (src && smp && ax.io_merge) {
     if ((r = sample_pre(c, n, dft))) return r;
-    launch_sources_sample(ax, n, n, c->stream);
+    launch_sources_sample(ax, n, n, c->stream, nullptr, fill);
     if ((r = launch_status(c, "source and sample launch"))) return r;
     return sample_post(c, n, dft);
   }
   if (src) {
-    launch_sources(ax, n, c->stream);
+    launch_sources(ax, n, c->stream, nullptr, fill);
     if ((r = launch_status(c, "source launch"))) return r;
   }
   if (smp && (r = sample_step(c, n, dft))) return r;
@@ -1191,17 +1219,18 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
         r = do_fused(c);
       } else {
         r = do_h(c);
-        if (!r) r = do_e(c);
+        if (!r) r = do_e(c, k + 1 < G && carries_flags(c), src);
       }
       if (r) break;
+      int* const fill = c->flags_carried ? next_flags(c) : nullptr;
       const KAux& ax = c->parity ? c->aux2 : c->aux;
       if (src && smp && ax.io_merge) {
-        launch_sources_sample(ax, k, k, c->stream, clk);
+        launch_sources_sample(ax, k, k, c->stream, clk, fill);
         r = launch_status(c, "source and sample launch");
         continue;
       }
       if (src) {
-        launch_sources(ax, k, c->stream, clk);
+        launch_sources(ax, k, c->stream, clk, fill);
         r = launch_status(c, "source launch");
       }
       if (!r && smp) {
@@ -1403,7 +1432,8 @@ int pm_run(pm_ctx* c, int64_t step0, int32_t nsteps, uint32_t flags) {
     // its first step in place, so the call ends with the state in the first
     // set
     const int32_t one = two ? head : nsteps;
-    if ((r = eager_step(c, n, s == 0 && (one & 1), fused, src, smp, dft))) return r;
+    if ((r = eager_step(c, n, s == 0 && (one & 1), fused, src, smp, dft, s + 1 < nsteps)))
+      return r;
     ++s;
   }
   c->span_on = c->timing;

@@ -29,9 +29,20 @@ __device__ __forceinline__ int64_t source_row(int64_t row, const int64_t* clock)
   return clock ? row + *clock : row;
 }
 
+// The gate flag a cell of component c sets with its value after the source (2-D
+// compat steps, compat.hip: Ez Ex Ey Hz, non-zero or NaN); fill null: none.
+template <typename T>
+__device__ __forceinline__ void source_flag(int* fill, int c, T v) {
+  const int a = c == PM_EZ ? 0 : c == PM_EX ? 1 : c == PM_EY ? 2 : c == PM_HZ ? 3 : -1;
+  if (!fill || a < 0) return;
+  if (v != v) fill[2 * a + 1] = 1;
+  else if (v != (T)0) fill[2 * a] = 1;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_source(const KSrc s, int64_t row, int64_t sy,
-                                                int64_t sz, T* F, const int64_t* clock) {
+                                                int64_t sz, T* F, const int64_t* clock,
+                                                int* fill) {
   const int ni = s.i1 - s.i0, nj = s.j1 - s.j0, nk = s.k1 - s.k0;
   const int64_t n = (int64_t)ni * nj * nk;
   const double a = s.table[source_row(row, clock)];
@@ -46,7 +57,9 @@ __global__ __launch_bounds__(256) void k_source(const KSrc s, int64_t row, int64
       if (s.divisor != 0.0) v = v / s.divisor;
     }
     const int64_t off = (int64_t)(s.i0 + i) + (int64_t)(s.j0 + j) * sy + (int64_t)(s.k0 + k) * sz;
-    F[off] = F[off] + (T)v;
+    const T f = F[off] + (T)v;
+    F[off] = f;
+    source_flag(fill, s.comp, f);
   }
 }
 
@@ -75,7 +88,8 @@ __device__ __forceinline__ T* field_of(int c, T* f0, T* f1, T* f2, T* f3, T* f4,
 template <typename T>
 __global__ __launch_bounds__(256) void k_source_all(const KSrc* tab, int64_t row, int64_t sy,
                                                     int64_t sz, T* f0, T* f1, T* f2, T* f3,
-                                                    T* f4, T* f5, const int64_t* clock) {
+                                                    T* f4, T* f5, const int64_t* clock,
+                                                    int* fill) {
   const KSrc s = tab[blockIdx.y];  // a kernel argument: global memory
   const int ni = s.i1 - s.i0, nj = s.j1 - s.j0, nk = s.k1 - s.k0;
   const int64_t n = (int64_t)ni * nj * nk;
@@ -93,7 +107,9 @@ __global__ __launch_bounds__(256) void k_source_all(const KSrc* tab, int64_t row
       if (s.divisor != 0.0) v = v / s.divisor;
     }
     const int64_t off = (int64_t)(s.i0 + i) + (int64_t)(s.j0 + j) * sy + (int64_t)(s.k0 + k) * sz;
-    F[off] = F[off] + (T)v;
+    const T f = F[off] + (T)v;
+    F[off] = f;
+    source_flag(fill, s.comp, f);
   }
 }
 
@@ -124,7 +140,7 @@ __global__ __launch_bounds__(256) void k_source_sample(const KSrc* stab, int n_s
                                                        const KSbox* btab, int64_t row,
                                                        int64_t sy, int64_t sz, T* f0, T* f1,
                                                        T* f2, T* f3, T* f4, T* f5, T* Xrow,
-                                                       const int64_t* clock) {
+                                                       const int64_t* clock, int* fill) {
   const int y = blockIdx.y;
   if (y < n_src) {
     const KSrc s = stab[y];
@@ -145,7 +161,9 @@ __global__ __launch_bounds__(256) void k_source_sample(const KSrc* stab, int n_s
       }
       const int64_t off =
           (int64_t)(s.i0 + i) + (int64_t)(s.j0 + j) * sy + (int64_t)(s.k0 + k) * sz;
-      F[off] = F[off] + (T)v;
+      const T f = F[off] + (T)v;
+      F[off] = f;
+      source_flag(fill, s.comp, f);
     }
     return;
   }
@@ -171,10 +189,12 @@ static int blocks_for(int64_t n) {
 }
 
 template <typename T>
-static void launch_source_all(const KAux& a, int64_t row, hipStream_t s, const int64_t* clock) {
+static void launch_source_all(const KAux& a, int64_t row, hipStream_t s, const int64_t* clock,
+                              int* fill) {
   T* const* F = (T* const*)a.F;
   hipLaunchKernelGGL(k_source_all<T>, dim3(blocks_for(a.src_max), a.n_src), dim3(256), 0, s,
-                     a.src_dev, row, a.sy, a.sz, F[0], F[1], F[2], F[3], F[4], F[5], clock);
+                     a.src_dev, row, a.sy, a.sz, F[0], F[1], F[2], F[3], F[4], F[5], clock,
+                     fill);
 }
 
 template <typename T>
@@ -186,13 +206,13 @@ static void launch_sample_all(const KAux& a, int64_t row, hipStream_t s) {
                      (T*)a.X + row * (int64_t)a.ncols);
 }
 
-void launch_sources(const KAux& a, int64_t step, hipStream_t s, const int64_t* clock) {
+void launch_sources(const KAux& a, int64_t step, hipStream_t s, const int64_t* clock, int* fill) {
   const int64_t row = step - a.table_step0;
   if (a.n_src > 1 && a.src_merge && a.src_max > 0) {
     if (a.precision == PM_FP64)
-      launch_source_all<double>(a, row, s, clock);
+      launch_source_all<double>(a, row, s, clock, fill);
     else
-      launch_source_all<float>(a, row, s, clock);
+      launch_source_all<float>(a, row, s, clock, fill);
     return;
   }
   for (int t = 0; t < a.n_src; ++t) {
@@ -201,15 +221,15 @@ void launch_sources(const KAux& a, int64_t step, hipStream_t s, const int64_t* c
     if (n <= 0) continue;
     if (a.precision == PM_FP64)
       hipLaunchKernelGGL(k_source<double>, dim3(blocks_for(n)), dim3(256), 0, s, src, row,
-                         a.sy, a.sz, (double*)a.F[src.comp], clock);
+                         a.sy, a.sz, (double*)a.F[src.comp], clock, fill);
     else
       hipLaunchKernelGGL(k_source<float>, dim3(blocks_for(n)), dim3(256), 0, s, src, row,
-                         a.sy, a.sz, (float*)a.F[src.comp], clock);
+                         a.sy, a.sz, (float*)a.F[src.comp], clock, fill);
   }
 }
 
 void launch_sources_sample(const KAux& a, int64_t step, int64_t row, hipStream_t s,
-                           const int64_t* clock) {
+                           const int64_t* clock, int* fill) {
   const int64_t srow = step - a.table_step0;
   const int64_t xrow = row % a.sample_T;
   const dim3 grid(blocks_for(std::max(a.src_max, a.sbox_max)), a.n_src + a.n_sbox);
@@ -217,12 +237,12 @@ void launch_sources_sample(const KAux& a, int64_t step, int64_t row, hipStream_t
     double* const* F = (double* const*)a.F;
     hipLaunchKernelGGL(k_source_sample<double>, grid, dim3(256), 0, s, a.src_dev, a.n_src,
                        a.sbox_dev, srow, a.sy, a.sz, F[0], F[1], F[2], F[3], F[4], F[5],
-                       (double*)a.X + xrow * (int64_t)a.ncols, clock);
+                       (double*)a.X + xrow * (int64_t)a.ncols, clock, fill);
   } else {
     float* const* F = (float* const*)a.F;
     hipLaunchKernelGGL(k_source_sample<float>, grid, dim3(256), 0, s, a.src_dev, a.n_src,
                        a.sbox_dev, srow, a.sy, a.sz, F[0], F[1], F[2], F[3], F[4], F[5],
-                       (float*)a.X + xrow * (int64_t)a.ncols, clock);
+                       (float*)a.X + xrow * (int64_t)a.ncols, clock, fill);
   }
 }
 

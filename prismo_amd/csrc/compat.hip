@@ -32,10 +32,15 @@
 namespace pm {
 
 // flags[2a] = some element non-zero and not NaN, flags[2a+1] = some NaN,
-// for a = 0: Ez, 1: Ex, 2: Ey, 3: Hz (2-D plane, padded layout), computed
-// before every H update into one of two sets of eight words that steps
-// alternate: the H kernel of a step clears the other set, which the next
-// step's flags kernel fills (both sets start cleared at configure).
+// for a = 0: Ez, 1: Ex, 2: Ey, 3: Hz (2-D plane, padded layout), as they stand
+// before an H update, in one of two sets of eight words that steps alternate:
+// the H kernel of a step clears the other set (both start cleared at
+// configure).  Within a run that set is filled by the step's E kernel, for the
+// cells no source adds to, and by its source kernel for the others; only a
+// run's first step, and H updates asked for by themselves, take k_flags2d.  As a
+// launch of its own in every step it was 6.5 us of the 18 a 540 x 290 step took:
+// each wave's atomics went to one cache line.  All a flag needs is one plain
+// store of 1 by any wave (the kernel's end makes it visible).
 __global__ void k_flags_clear(int* f) {
   if (threadIdx.x < 16) f[threadIdx.x] = 0;
 }
@@ -43,10 +48,22 @@ __global__ void k_flags_clear(int* f) {
 constexpr int kFlagRows = 4;
 
 // One column i per thread and kFlagRows rows per workgroup (the loads of a
-// thread have no loop-carried address, so they overlap); a wave ORs a flag
-// only when its cells set it and it was not yet seen set (every wave
-// ORing into the same eight words serialises the kernel; a stale read only
-// costs an atomic that changes nothing).
+// thread have no loop-carried address, so they overlap).
+// Flag bits (bit 2a: non-zero and not NaN, bit 2a+1: NaN) of one value of array a.
+__device__ __forceinline__ unsigned flag_bits(double v, int a) {
+  if (v != v) return 2u << (2 * a);
+  return v != 0.0 ? 1u << (2 * a) : 0u;
+}
+
+// The flags some lane of the wave has bits for.
+__device__ __forceinline__ void set_flags(int* flags, unsigned bits) {
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const unsigned long long m = __ballot((bits >> b) & 1u);
+    if (m && (int)(threadIdx.x & 63) == __builtin_ctzll(m)) flags[b] = 1;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_flags2d(const KGrid g) {
   const double* A[4] = {(const double*)g.E[2], (const double*)g.E[0],
                         (const double*)g.E[1], (const double*)g.H[2]};
@@ -62,18 +79,10 @@ __global__ __launch_bounds__(256) void k_flags2d(const KGrid g) {
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       if (A[a] == nullptr || i >= ex[a] || j >= ey[a]) continue;
-      const double v = A[a][off];
-      if (v != v) bits |= 2u << (2 * a);
-      else if (v != 0.0) bits |= 1u << (2 * a);
+      bits |= flag_bits(A[a][off], a);
     }
   }
-  for (int m = 32; m >= 1; m >>= 1) bits |= (unsigned)__shfl_xor((int)bits, m);
-  if ((threadIdx.x % warpSize) == 0 && bits) {
-    volatile const int* fv = g.flags;
-#pragma unroll
-    for (int b = 0; b < 8; ++b)
-      if (((bits >> b) & 1u) && !fv[b]) atomicOr(&g.flags[b], 1);
-  }
+  set_flags(g.flags, bits);
 }
 
 template <int CK>
@@ -131,8 +140,12 @@ __global__ __launch_bounds__(kBX* kBY) void k_compat_h2d(const KGrid g) {
   }
 }
 
+// fill: flags_next is filled from the updated cells outside the n_src source
+// boxes.
 template <int CK>
-__global__ __launch_bounds__(kBX* kBY) void k_compat_e2d(const KGrid g) {
+__global__ __launch_bounds__(kBX* kBY) void k_compat_e2d(const KGrid g, bool fill,
+                                                         const KSrc* src, int n_src) {
+  static_assert(kBX == 64, "a row of threads is a wave");
   const int i = blockIdx.x * kBX + threadIdx.x;
   const int j = blockIdx.y * kBY + threadIdx.y;
   if (i >= g.nx || j >= g.ny) return;
@@ -141,25 +154,42 @@ __global__ __launch_bounds__(kBX* kBY) void k_compat_e2d(const KGrid g) {
   const int64_t off = (int64_t)i + (int64_t)j * g.sy;
   const double* Hx = (const double*)g.H[0];
   const double* Hy = (const double*)g.H[1];
+  unsigned bits = 0;
   if (i < g.nx - 1 && j < g.ny - 1) {
     double* Ez = (double*)g.E[2];
     const double cx = (Hy[off + 1] - Hy[off]) / g.dx;
     const double cy = (Hx[off + g.sy] - Hx[off]) / g.dy;
-    Ez[off] = eco_a<CK>(g, 2, off) * Ez[off] + eco_b(g, 2, off) * (cx - cy);
+    const double v = eco_a<CK>(g, 2, off) * Ez[off] + eco_b(g, 2, off) * (cx - cy);
+    Ez[off] = v;
+    bits |= flag_bits(v, 0);
   }
   if (te_any) {
     const double* Hz = (const double*)g.H[2];
     if (j < g.ny - 1) {
       double* Ex = (double*)g.E[0];
       const double c = (Hz[off + g.sy] - Hz[off]) / g.dy;
-      Ex[off] = eco_a<CK>(g, 0, off) * Ex[off] + eco_b(g, 0, off) * c;
+      const double v = eco_a<CK>(g, 0, off) * Ex[off] + eco_b(g, 0, off) * c;
+      Ex[off] = v;
+      bits |= flag_bits(v, 1);
     }
     if (i < g.nx - 1) {
       double* Ey = (double*)g.E[1];
       const double c = (Hz[off + 1] - Hz[off]) / g.dx;
-      Ey[off] = eco_a<CK>(g, 1, off) * Ey[off] - eco_b(g, 1, off) * c;
+      const double v = eco_a<CK>(g, 1, off) * Ey[off] - eco_b(g, 1, off) * c;
+      Ey[off] = v;
+      bits |= flag_bits(v, 2);
     }
+    bits |= flag_bits(Hz[off], 3);
   }
+  if (!fill) return;
+  // (where the TE half was skipped, Ex, Ey and Hz are all zero: no flags)
+  for (int t = 0; t < n_src; ++t) {
+    const KSrc s = src[t];
+    if (i >= s.i0 && i < s.i1 && j >= s.j0 && j < s.j1 && s.k0 < s.k1)
+      bits &= ~(s.comp == PM_EZ ? 3u : s.comp == PM_EX ? 12u : s.comp == PM_EY ? 48u
+                : s.comp == PM_HZ ? 192u : 0u);
+  }
+  set_flags(g.flags_next, bits);
 }
 
 // ------------------------------------------------------------------ 3-D
@@ -246,12 +276,15 @@ void launch_compat_h(const KGrid& g, int ck, hipStream_t s) {
   }
 }
 
-void launch_compat_e(const KGrid& g, int ck, hipStream_t s) {
+void launch_compat_e(const KGrid& g, int ck, bool fill, const KSrc* src, int n_src,
+                     hipStream_t s) {
   dim3 block(kBX, kBY);
   dim3 grid((g.nx + kBX - 1) / kBX, (g.ny + kBY - 1) / kBY, g.ndim == 3 ? g.nz : 1);
   if (g.ndim == 2) {
-    if (ck == PM_COEFF_FULL) hipLaunchKernelGGL(k_compat_e2d<PM_COEFF_FULL>, grid, block, 0, s, g);
-    else hipLaunchKernelGGL(k_compat_e2d<PM_COEFF_CB>, grid, block, 0, s, g);
+    if (ck == PM_COEFF_FULL)
+      hipLaunchKernelGGL(k_compat_e2d<PM_COEFF_FULL>, grid, block, 0, s, g, fill, src, n_src);
+    else
+      hipLaunchKernelGGL(k_compat_e2d<PM_COEFF_CB>, grid, block, 0, s, g, fill, src, n_src);
   } else {
     if (ck == PM_COEFF_FULL) hipLaunchKernelGGL(k_compat_e3d<PM_COEFF_FULL>, grid, block, 0, s, g);
     else hipLaunchKernelGGL(k_compat_e3d<PM_COEFF_CB>, grid, block, 0, s, g);

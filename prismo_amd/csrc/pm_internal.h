@@ -74,7 +74,8 @@ struct KGrid {
   int ade_j0, ade_j1, ade_k0, ade_k1;  // union of the boxes' j and k ranges
   const KAde* ade;  // device copy of the ADE boxes (in scratch)
   int* flags;       // compat gating flags of this step (scratch)
-  int* flags_next;  // the other set, cleared by the 2-D compat H kernel
+  int* flags_next;  // the other set: cleared by the 2-D compat H kernel, then filled for
+                    // the next step by its E and source kernels within a run
 };
 
 // scratch layout (caller-owned, PM_SCRATCH_BYTES)
@@ -179,7 +180,9 @@ void launch_yee_e(const KGrid& g, int precision, int coeff_kind, hipStream_t s);
 void launch_compat_flags2d(const KGrid& g, hipStream_t s);
 void launch_compat_flags_clear(int* flags, hipStream_t s);
 void launch_compat_h(const KGrid& g, int coeff_kind, hipStream_t s);
-void launch_compat_e(const KGrid& g, int coeff_kind, hipStream_t s);
+// fill (2-D): flags_next is filled too, from the cells outside src[0 .. n_src).
+void launch_compat_e(const KGrid& g, int coeff_kind, bool fill, const KSrc* src, int n_src,
+                     hipStream_t s);
 // One fused 2-D TM step (tm2d.hip): Ez, Hx, Hy of set "i" -> set "o", the
 // H-side CPML memory of the x (Hy) and y (Hx) slabs likewise, the E-side
 // memory of the plan updated in place; rows per tile `chunk`.
@@ -231,8 +234,9 @@ bool fused2_grid_ok(const KGrid& g);  // x CPML layers fit the kernel's LDS slot
 // (packed field sets, Cb, CPML memory pairs and profiles within 4 GiB).
 bool fused_addressable(const KGrid& g, const FusedBufs& fb, int esz);
 // With `clock`, `step` is relative: the table row is step + *clock - table_step0.
+// fill: gate flags set from the cells the sources add to (2-D compat steps).
 void launch_sources(const KAux& a, int64_t step, hipStream_t s,
-                    const int64_t* clock = nullptr);
+                    const int64_t* clock = nullptr, int* fill = nullptr);
 // *clock = v (add false) or *clock += v, in one thread of a kernel (so it can
 // be captured in a graph).
 void launch_clock(int64_t* clock, int64_t v, bool add, hipStream_t s);
@@ -240,7 +244,7 @@ void launch_sample(const KAux& a, int64_t step, hipStream_t s);
 // Sources of step `step` (relative with `clock`, as launch_sources) and the
 // samples into X row `row`, one launch (a.io_merge must hold).
 void launch_sources_sample(const KAux& a, int64_t step, int64_t row, hipStream_t s,
-                           const int64_t* clock = nullptr);
+                           const int64_t* clock = nullptr, int* fill = nullptr);
 void launch_dft(const KDft& d, const void* X, int ncols, const void* W_re, const void* W_im,
                 int64_t table_len, int64_t wcol0, int rows, int precision, hipStream_t s,
                 const int64_t* wclock = nullptr);

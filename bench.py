@@ -276,6 +276,7 @@ def cpu_baseline(n=256, steps=3):
 
 SWEEP_ALG_BYTES_PER_CELL = 26.0  # 2-D TM: Ez, Hx, Hy FP32 read + written, FP16 Cb
 SWEEP_ALG_BYTES_PER_PML_CELL_AXIS = 16.0  # two FP32 psi read + written
+SWEEP_STEPS_PER_LAUNCH = 8  # a launch reads and writes the state once
 
 
 def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
@@ -355,7 +356,8 @@ def sweep_bench(n_designs=256, steps=4000, seq_sample=32, group=64, first=16):
         t = W.COUPLER_PML
         slab += 2 * t * ny + 2 * t * nx
     del eng, sims
-    alg = SWEEP_ALG_BYTES_PER_CELL * cells + SWEEP_ALG_BYTES_PER_PML_CELL_AXIS * slab
+    alg = (SWEEP_ALG_BYTES_PER_CELL * cells +
+           SWEEP_ALG_BYTES_PER_PML_CELL_AXIS * slab) / SWEEP_STEPS_PER_LAUNCH
     step_ms = gpu_ms / steps
 
     idx = np.unique(np.linspace(0, n_designs - 1, seq_sample).round().astype(int))

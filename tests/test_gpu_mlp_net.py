@@ -48,6 +48,20 @@ def test_forward_layers(mi355x, M, n_in, hidden, depth, n_out):
             assert _rel(Y.cpu().numpy(), z) <= 1e-5
 
 
+@pytest.mark.parametrize("M,hidden", [(70, 40), (3000, 256), (300, 520)])
+def test_activations_are_those_of_erf(mi355x, M, hidden):
+    """Hidden values are z (1 + erf(z / sqrt 2)) / 2 in FP32 to the last bit, in the
+    whole-network kernels and in the per-layer ones (520 units): one bit more or
+    less turns some of their BF16 roundings, 2^-9 each, and the outputs with them."""
+    import torch
+
+    net = _net(4, hidden, 3, 8)
+    X = _t(np.random.default_rng(1).uniform(-3, 3, (M, 4)))
+    _, (acts, zs) = net.forward(X, keep=True)
+    for k, z in enumerate(zs):
+        assert torch.equal(acts[k + 1], 0.5 * z * (1.0 + torch.erf(z * 0.70710678118654752))), k
+
+
 @pytest.mark.parametrize("hidden,n_out", [(40, 30), (128, 100), (256, 256), (300, 64)])
 def test_tall_and_short_workgroups_agree(mi355x, hidden, n_out):
     """Enough rows for 128- (or 64-) row workgroups, with a ragged last one,

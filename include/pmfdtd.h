@@ -75,7 +75,11 @@ enum pm_coeff_kind {
  *   kind 0: value = table[n]                                  (point, plane)
  *   kind 1: value = (table[n] * profile[c]) / divisor  (divisor 0 = none)
  * profile is in box order (i fastest).  table is indexed by the absolute
- * step index n minus pm_plan.table_step0. */
+ * step index n minus pm_plan.table_step0.  A box may reach past its
+ * component's extent up to the grid's node counts: those cells keep what is
+ * added to them, and the curls beside those of E and monitors read it.  Plans
+ * where that is so (an E box, or an H box and a monitor box of the component
+ * past its extent) take the unfused kernels. */
 typedef struct pm_source {
   int32_t comp, kind;
   int32_t i0, i1, j0, j1, k0, k1;

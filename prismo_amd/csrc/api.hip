@@ -156,6 +156,31 @@ bool box_ok(int i0, int i1, int j0, int j1, int k0, int k1, const pm_plan& p) {
          i1 <= p.nx && j1 <= p.ny && k1 <= p.nz;
 }
 
+// The box holds cells past its component's extent (E half a cell short of the
+// grid along the other two axes, H along its own).
+template <class B>
+bool past_extent(const pm_plan& p, const B& b) {
+  if (b.i0 >= b.i1 || b.j0 >= b.j1 || b.k0 >= b.k1) return false;
+  const int a = b.comp % 3;
+  const bool e = b.comp < 3;
+  return ((a == 0) != e && b.i1 > p.nx - 1) || ((a == 1) != e && b.j1 > p.ny - 1) ||
+         (p.ndim == 3 && (a == 2) != e && b.k1 > p.nz - 1);
+}
+
+// No source adds to a cell past its component's extent that something reads: the
+// curls of H read E there, of H only monitors.  The fused kernels hold those
+// cells at zero, each in its own way; the unfused ones keep the value.
+bool sources_inside(const pm_plan& p) {
+  for (int s = 0; s < p.n_src; ++s) {
+    const pm_source& q = p.src[s];
+    if (!past_extent(p, q)) continue;
+    if (q.comp < 3) return false;
+    for (int t = 0; t < p.n_sbox; ++t)
+      if (p.sbox[t].comp == q.comp && past_extent(p, p.sbox[t])) return false;
+  }
+  return true;
+}
+
 // Kernel form of one dispersive box.  The box carries the reference's
 // coefficients (src/prismo/materials/dispersion.py:189-231, 267-286); used
 // as they stand (P+ = c0 E+ + c1 E + ..., J+ = c0 E+ + c1 J) the drive term
@@ -1003,7 +1028,9 @@ int pm_configure(pm_ctx* c, const pm_plan* plan) {
     c->split_ok = p.coeff_kind != PM_COEFF_FULL && gxr < p.nx && gxr >= p.pml[0] &&
                   gxr < p.nx - p.pml[1];
   }
-  c->fused_ok = p.ndim == 2
+  const bool inside = sources_inside(p);
+  c->fused_ok = !inside ? false
+                : p.ndim == 2
                     ? fused2d_eligible(p)
                     : fused_eligible(p) &&
                           fused_addressable(c->g, fused_bufs(p, true), p.precision == PM_FP64 ? 8 : 4) &&
@@ -1011,7 +1038,7 @@ int pm_configure(pm_ctx* c, const pm_plan* plan) {
   c->parity = 0;
   c->pe_parity = 0;
   set_psi_e(c);
-  c->multi2d_ok = multi2d_eligible(p);
+  c->multi2d_ok = inside && multi2d_eligible(p);
   c->fused2_ok = fused2_eligible(c);
   c->src_kind0 = true;
   for (int s = 0; s < x.n_src; ++s)

@@ -330,11 +330,13 @@ int pm_sync(pm_ctx* ctx);
 /* Average kernel time (ms) since timing was enabled, measured with HIP
  * events on the context stream around every launch of kernel class `which`
  * (0 = H update, 1 = E update, 2 = whole step, 3 = fused H+E step,
- * 4 = spectral flush of one sample block, 5 = launch of two (2-D: up to eight) steps, 6 = one graph
- * replay of a PM_RUN_GRAPH block, timed on the second stream); enabled (and reset) by
- * pm_set_timing.  enable = 0 turns timing off; enable = s >= 1 times the
- * kernels of every s-th step of pm_run (steps whose index is a multiple of
- * s), so a long run can be timed with few events. */
+ * 4 = spectral flush of one sample block, 5 = launch of two (2-D: up to
+ * eight) steps, 6 = one graph replay of a PM_RUN_GRAPH block, timed on the
+ * second stream); enabled (and reset) by pm_set_timing.  A 2-D launch of
+ * several steps counts as one in class 5 and as its steps in class 2.
+ * enable = 0 turns timing off; enable = s >= 1 times the kernels of every
+ * s-th step of pm_run (steps whose index is a multiple of s; 2-D launches of
+ * several steps that hold one), so a long run can be timed with few events. */
 int pm_set_timing(pm_ctx* ctx, int enable);
 int pm_get_timing(pm_ctx* ctx, int which, double* avg_ms, int64_t* count);
 

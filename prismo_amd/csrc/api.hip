@@ -59,7 +59,11 @@ struct pm_ctx {
   bool span_on = false;   // timing, and the current step is one of those
   std::vector<hipEvent_t> pool;
   size_t pool_used = 0;
-  std::vector<std::pair<hipEvent_t, hipEvent_t>> spans[7];
+  struct TimedSpan {
+    hipEvent_t a, b;
+    int count;  // what it stands for in its class (steps of a 2-D launch in class 2, else 1)
+  };
+  std::vector<TimedSpan> spans[7];
   // graph replay (PM_RUN_GRAPH): one captured block of steps per starting
   // buffer set (fused steps) or gate flag set (2-D compat steps), with the
   // run flags it was captured for
@@ -113,9 +117,9 @@ hipEvent_t take_event(pm_ctx* c) {
 
 struct Span {
   pm_ctx* c;
-  int which;
+  int which, count;
   hipEvent_t a = nullptr;
-  Span(pm_ctx* ctx, int w) : c(ctx), which(w) {
+  Span(pm_ctx* ctx, int w, int n = 1) : c(ctx), which(w), count(n) {
     if (c->span_on) {
       a = take_event(c);
       if (a) (void)hipEventRecord(a, c->stream);
@@ -126,7 +130,7 @@ struct Span {
       hipEvent_t b = take_event(c);
       if (b) {
         (void)hipEventRecord(b, c->stream);
-        c->spans[which].push_back({a, b});
+        c->spans[which].push_back({a, b, count});
       }
     }
   }
@@ -644,7 +648,7 @@ FusedBufs fused2_bufs(const pm_ctx* c) {
 // (fields and both halves' CPML memory), with their sources and samples; with
 // clock, n counts from the step it holds.
 int do_multi2d(pm_ctx* c, int64_t n, int m, bool src, bool smp, const int64_t* clock) {
-  Span sp(c, 5);
+  Span whole(c, 2, m), sp(c, 5);
   const pm_plan& p = c->plan;
   const bool a_in = c->parity == 0, e_in = c->pe_parity == 0;
   Tm2dBufs b{};
@@ -1196,13 +1200,13 @@ int run_multi2d(pm_ctx* c, int64_t step0, int32_t nsteps, bool src, bool smp, bo
   int r;
   for (int32_t s = 0; s < nsteps;) {
     const int64_t n = step0 + s;
-    c->span_on = !clock && c->timing && n % c->timing_stride == 0;
     int m = cut ? cut : multi2d_len(c, n, nsteps - s, smp);
     cut = 0;
     if (odd) {
       odd = false;
       if (m == 1 && clock) return fail(c, PM_EINVAL, "odd one-step block in a captured run");
       if (m == 1) {
+        c->span_on = c->timing && n % c->timing_stride == 0;
         if ((r = eager_step(c, n, true, true, src, smp, dft))) return r;
         ++s;
         continue;
@@ -1210,6 +1214,8 @@ int run_multi2d(pm_ctx* c, int64_t step0, int32_t nsteps, bool src, bool smp, bo
       m -= 1;
       cut = 1;
     }
+    // a launch is timed when one of its steps is a multiple of the stride
+    c->span_on = !clock && c->timing && (n + m - 1) / c->timing_stride * c->timing_stride >= n;
     if (smp && !clock && (r = sample_pre(c, n, dft))) return r;
     if ((r = do_multi2d(c, n, m, src, smp, clock))) return r;
     if (smp && !clock)
@@ -1321,7 +1327,7 @@ int replay_blocks(pm_ctx* c, int64_t n0, int32_t nrep, int32_t G, bool fused, bo
       hipEvent_t b = take_event(c);
       if (b) {
         (void)hipEventRecord(b, c->s2);
-        c->spans[6].push_back({a, b});
+        c->spans[6].push_back({a, b, 1});
       }
     }
   }
@@ -1581,12 +1587,12 @@ int pm_get_timing(pm_ctx* c, int which, double* avg_ms, int64_t* count) {
   if (r) return r;
   double tot = 0;
   int64_t n = 0;
-  for (auto& ab : c->spans[which]) {
+  for (auto& s : c->spans[which]) {
     float ms = 0;
-    hipError_t e = hipEventElapsedTime(&ms, ab.first, ab.second);
+    hipError_t e = hipEventElapsedTime(&ms, s.a, s.b);
     if (e != hipSuccess) return hip_check(c, e, "event elapsed");
     tot += ms;
-    ++n;
+    n += s.count;
   }
   *avg_ms = n ? tot / n : 0.0;
   *count = n;

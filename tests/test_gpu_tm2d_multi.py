@@ -132,3 +132,35 @@ def test_against_oracle(mi355x, dtype, bar):
     got, _ = _out(sim, mon)
     ref = np.concatenate([o1.F[c].ravel() for c in ("Ez", "Hx", "Hy")])
     assert rel_l2(got, ref) <= bar
+
+
+@pytest.mark.parametrize("start,n", [(0, 40), (1, 40), (5, 59), (8, 1)])
+@pytest.mark.parametrize("stride", [1, 2, 4, 8, 10, 50])
+def test_timing_stride(mi355x, start, n, stride):
+    """Every launch that holds a step that is a multiple of the stride is timed:
+    once in class 5, as its steps in class 2; a step taken by itself in place
+    counts in class 2 alone."""
+    sim, _ = _sim(60, 40, 5, np.float32)
+    eng = sim.solver.updater.engine_for(sim.fields)
+    eng.ctx.set_timing(True, stride=stride)
+    eng.run(start, n)
+    cuts, at = [], start                 # an even number of launches of up to 8
+    while at < start + n:
+        cuts.append(min(8, start + n - at))
+        at += cuts[-1]
+    alone = 0
+    if len(cuts) % 2:
+        if cuts[0] == 1:
+            alone = 1
+        else:
+            cuts[:1] = [cuts[0] - 1, 1]
+    at, launches, steps = start, 0, 0
+    for k, m in enumerate(cuts):
+        if any((at + i) % stride == 0 for i in range(m)):
+            launches += not (alone and k == 0)
+            steps += m
+        at += m
+    ms5, n5 = eng.ctx.timing(5)
+    ms2, n2 = eng.ctx.timing(2)
+    assert (n5, n2) == (launches, steps)
+    assert (ms5 > 0) == (launches > 0) and (ms2 > 0) == (steps > 0)

@@ -316,7 +316,8 @@ int pm_row_split_active(pm_ctx* ctx);
 /* Launch shape the next one-step fused launch takes: out[0..3] = cells per
  * lane, waves per row segment, rows per workgroup, row segments (the
  * tuning asked for, or what it falls back to); returns 1, or 0 (out all 0)
- * when the step is not fused. */
+ * when no such launch is taken: the step is not fused, or 2-D runs take
+ * several steps per launch, whose tiles follow a rule of their own. */
 int pm_fused_shape(pm_ctx* ctx, int32_t* out);
 
 /* Steps per fused launch pm_run will use with the current plan and tuning

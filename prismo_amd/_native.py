@@ -304,7 +304,8 @@ class Context:
         self._check(self.lib.pm_set_row_split(self.h, int(segments)), "pm_set_row_split")
 
     def fused_shape(self):
-        """(vec, w, ty, xs) of the next one-step fused launch, or None."""
+        """(vec, w, ty, xs) of the next one-step fused launch, or None when the
+        run takes none (unfused, or several 2-D steps per launch)."""
         out = (i32 * 4)()
         if not self.lib.pm_fused_shape(self.h, out):
             return None

@@ -419,11 +419,7 @@ int do_e(pm_ctx* c, bool carry = false, bool src = false) {
 // The flag set the next H update reads (after do_h: the one its kernel cleared).
 int* next_flags(const pm_ctx* c) { return c->g.flags + 8 * c->flag_set; }
 
-// Cells per lane and waves per row of the fused kernel for this plan.
-// Launch shape of the fused kernel: the tuned one, else (rows per workgroup
-// and then cells per lane relaxed) the first that fits the workgroup and LDS
-// limits.  False if none does.
-// Rows per tile of the 2-D pass: kchunk once pm_set_tuning has set it, else
+// Rows per tile of the 2-D one-pass step: kchunk once pm_set_tuning has set it, else
 // 3.  A wave's rows run one after another (two rows of loads in flight), so
 // short tiles and many waves suit the small grids 2-D runs have: on a
 // 540 x 290 FP64 grid 2 and 3 rows per tile step in 7.3 us, 8 rows in
@@ -487,10 +483,14 @@ int auto_planes(const pm_ctx* c, int w, int ty, int xs) {
   return best;
 }
 
-// Rows in xs segments (pm_set_row_split: 1 or 2; 0 = whole rows when a
-// shape fits them, else two segments).
+// Launch shape of the fused one-step kernel: cells per lane, waves per row,
+// rows per workgroup (planes are chosen by the caller) in xs segments
+// (pm_set_row_split: 1 or 2; 0 = whole rows when a shape fits them, else two
+// segments); the tuned one, else (rows per workgroup and then cells per lane
+// relaxed) the first that fits the workgroup and LDS limits.  False if none
+// does.
 bool fused_shape(const pm_ctx* c, int* vec, int* w, int* ty, int* xs) {
-  const int sy = (int)c->plan.sy;  // padded row, 128 / 256 / 512
+  const int sy = (int)c->plan.sy;  // padded row
   if (c->plan.ndim == 2) {
     // the 2-D pass: one cell per lane, a wave per 64-cell strip, tiles of
     // rows2d rows
@@ -1514,7 +1514,7 @@ int pm_set_row_split(pm_ctx* c, int segments) {
 int pm_fused_shape(pm_ctx* c, int32_t* out) {
   if (!c || !out) return PM_EINVAL;
   out[0] = out[1] = out[2] = out[3] = 0;
-  if (!c->configured || !c->fused_ok || !c->fuse) return 0;
+  if (!c->configured || !c->fused_ok || !c->fuse || use_multi2d(c)) return 0;
   int vec = 0, w = 0, ty = 0, xs = 1;
   if (!fused_shape(c, &vec, &w, &ty, &xs)) return 0;
   out[0] = vec;

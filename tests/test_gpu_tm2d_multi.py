@@ -164,3 +164,13 @@ def test_timing_stride(mi355x, start, n, stride):
     ms2, n2 = eng.ctx.timing(2)
     assert (n5, n2) == (launches, steps)
     assert (ms5 > 0) == (launches > 0) and (ms2 > 0) == (steps > 0)
+
+
+def test_shape_of_one_step_launches_only(mi355x):
+    sim, _ = _sim(60, 40, 5, np.float32)
+    eng = sim.solver.updater.engine_for(sim.fields)
+    assert eng.ctx.fused_shape() is None and eng.ctx.fused_steps() == 1
+    eng.ctx.set_tuning(1, 4, 5, 0, 2)
+    assert eng.ctx.fused_shape()[2] == 5
+    eng.ctx.set_tuning(2, 4, 8, 0, 2)
+    assert eng.ctx.fused_shape() is None and eng.ctx.fused_steps() == 2

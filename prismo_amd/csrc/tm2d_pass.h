@@ -298,15 +298,19 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     if (kTmS % R != 0 && (t < kTmS || t >= kTmW * R - kTmS)) continue;  // uniform
     if (YP && j >= ny) continue;
     const uint32_t o = (uint32_t)j * g.sy + (uint32_t)i;
+    // positions past a component's extent stay 0 in memory (next to an Inf or NaN
+    // their zero coefficient does not keep them so)
+    const bool ly_ok = !YP || j < ny - 1;
+    const T e = le_ok && ly_ok ? ez[r] : (T)0;
     if constexpr (IO::kStatus) {
       if constexpr (sizeof(T) == 4)
-        bad |= (__builtin_bit_cast(uint32_t, ez[r]) & 0x7f800000u) + 0x00800000u;
+        bad |= (__builtin_bit_cast(uint32_t, e) & 0x7f800000u) + 0x00800000u;
       else
-        bad |= ((uint32_t)(__builtin_bit_cast(uint64_t, ez[r]) >> 32) & 0x7ff00000u) + 0x00100000u;
+        bad |= ((uint32_t)(__builtin_bit_cast(uint64_t, e) >> 32) & 0x7ff00000u) + 0x00100000u;
     }
-    ((gptr<T>)g.ez_o)[o] = ez[r];
-    ((gptr<T>)g.hx_o)[o] = hx[r];
-    ((gptr<T>)g.hy_o)[o] = hy[r];
+    ((gptr<T>)g.ez_o)[o] = e;
+    ((gptr<T>)g.hx_o)[o] = le_ok ? hx[r] : (T)0;
+    ((gptr<T>)g.hy_o)[o] = ly_ok ? hy[r] : (T)0;
     if constexpr (XP) {
       if (xpml) {
         const uint32_t q = xo + g.xst * (uint32_t)j;

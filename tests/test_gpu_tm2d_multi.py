@@ -174,3 +174,32 @@ def test_shape_of_one_step_launches_only(mi355x):
     assert eng.ctx.fused_shape()[2] == 5
     eng.ctx.set_tuning(2, 4, 8, 0, 2)
     assert eng.ctx.fused_shape() is None and eng.ctx.fused_steps() == 2
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("t", [0, 6])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_a_diverged_run_leaves_nothing_behind(mi355x, dtype, t, bad):
+    """Fields that are not finite leave the cells past each component's extent
+    at zero, so a run after zeroing the fields is that of a new simulation (an
+    odd count: its first step is taken in place)."""
+    ny = 41
+    outs = []
+    for spoiled in (True, False):
+        sim, _ = _sim(70, ny, t, dtype)
+        eng = sim.solver.updater.engine_for(sim.fields)
+        if spoiled:
+            sim.fields["Ez"] = bad
+            eng.run(0, 16)
+            for c in ("Ez", "Hx", "Hy"):
+                f = sim.fields[c]                      # a view [i, j] of rows of sy
+                pad = f.as_strided((f.stride(1), ny), (1, f.stride(1))).clone()
+                pad[:f.shape[0], :f.shape[1]] = 0
+                assert bool((pad == 0).all()), c
+            sim.fields.zero_fields()
+            eng.reset_state()
+        sim.fields["Ez"][20, 20] = 1.0
+        eng.run(0, 25)
+        outs.append(np.concatenate([sim.fields.to_numpy(c).ravel() for c in ("Ez", "Hx", "Hy")]))
+    assert np.isfinite(outs[1]).all() and np.linalg.norm(outs[1]) > 0
+    assert np.array_equal(*outs)

@@ -419,6 +419,15 @@ int do_e(pm_ctx* c, bool carry = false, bool src = false) {
 // The flag set the next H update reads (after do_h: the one its kernel cleared).
 int* next_flags(const pm_ctx* c) { return c->g.flags + 8 * c->flag_set; }
 
+// Flags carried by a step after which a call failed are dropped: its sources
+// may be missing and the caller may change the fields.
+int drop_carried(pm_ctx* c) {
+  if (!c->flags_carried) return 0;
+  c->flags_carried = false;
+  launch_compat_flags_clear(next_flags(c), 1, c->stream);
+  return launch_status(c, "flag clear launch");
+}
+
 // Rows per tile of the 2-D one-pass step: kchunk once pm_set_tuning has set it, else
 // 3.  A wave's rows run one after another (two rows of loads in flight), so
 // short tiles and many waves suit the small grids 2-D runs have: on a
@@ -1052,7 +1061,7 @@ int pm_configure(pm_ctx* c, const pm_plan* plan) {
   c->flag_set = c->flag_set_e = 0;
   c->flags_carried = false;
   if (p.scheme == PM_SCHEME_COMPAT && p.ndim == 2) {
-    launch_compat_flags_clear(c->g.flags, c->stream);
+    launch_compat_flags_clear(c->g.flags, 2, c->stream);
     int r = launch_status(c, "flag clear launch");
     if (r) return r;
   }
@@ -1086,13 +1095,15 @@ int pm_configure_static(pm_ctx* c, const pm_plan* plan) {
 int pm_update_h(pm_ctx* c) {
   if (!c) return PM_EINVAL;
   if (!c->configured) return fail(c, PM_ENOPLAN, "pm_update_h before pm_configure");
-  return do_h(c);
+  const int r = drop_carried(c);
+  return r ? r : do_h(c);
 }
 
 int pm_update_e(pm_ctx* c) {
   if (!c) return PM_EINVAL;
   if (!c->configured) return fail(c, PM_ENOPLAN, "pm_update_e before pm_configure");
-  return do_e(c);
+  const int r = drop_carried(c);
+  return r ? r : do_e(c);
 }
 
 namespace {
@@ -1236,7 +1247,7 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
   const pm_plan& p = c->plan;
   int64_t* clk = step_clock(c);
   hipStream_t s0 = c->stream;
-  const int par0 = c->parity, pe0 = c->pe_parity;
+  const int par0 = c->parity, pe0 = c->pe_parity, fl0 = c->flag_set;
   const bool span0 = c->span_on;
   c->stream = c->s2;
   c->parity = par;
@@ -1288,6 +1299,8 @@ int capture_block(pm_ctx* c, int par, int slot, int32_t G, bool fused, bool src,
   c->parity = par0;
   c->pe_parity = pe0;
   set_psi_e(c);
+  c->flag_set = fl0;  // (a block holds an even number of steps)
+  c->flags_carried = false;
   c->span_on = span0;
   if (!r)
     r = hip_check(c, hipGraphInstantiate(&c->graph[slot], g, nullptr, nullptr, 0),
@@ -1421,6 +1434,7 @@ int pm_run(pm_ctx* c, int64_t step0, int32_t nsteps, uint32_t flags) {
     if (nsteps == 1 && smp) return sample_step(c, step0, dft);
     return 0;
   }
+  if (const int r = drop_carried(c)) return r;
   int fvec = 0, fw = 0, fty = 0, fxs = 1;
   const bool multi = use_multi2d(c);
   const bool fused =

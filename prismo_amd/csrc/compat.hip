@@ -41,14 +41,10 @@ namespace pm {
 // launch of its own in every step it was 6.5 us of the 18 a 540 x 290 step took:
 // each wave's atomics went to one cache line.  All a flag needs is one plain
 // store of 1 by any wave (the kernel's end makes it visible).
-__global__ void k_flags_clear(int* f) {
-  if (threadIdx.x < 16) f[threadIdx.x] = 0;
+__global__ void k_flags_clear(int* f, int n) {
+  if ((int)threadIdx.x < n) f[threadIdx.x] = 0;
 }
 
-constexpr int kFlagRows = 4;
-
-// One column i per thread and kFlagRows rows per workgroup (the loads of a
-// thread have no loop-carried address, so they overlap).
 // Flag bits (bit 2a: non-zero and not NaN, bit 2a+1: NaN) of one value of array a.
 __device__ __forceinline__ unsigned flag_bits(double v, int a) {
   if (v != v) return 2u << (2 * a);
@@ -64,6 +60,10 @@ __device__ __forceinline__ void set_flags(int* flags, unsigned bits) {
   }
 }
 
+constexpr int kFlagRows = 4;
+
+// One column i per thread and kFlagRows rows per workgroup (the loads of a
+// thread have no loop-carried address, so they overlap).
 __global__ __launch_bounds__(256) void k_flags2d(const KGrid g) {
   const double* A[4] = {(const double*)g.E[2], (const double*)g.E[0],
                         (const double*)g.E[1], (const double*)g.H[2]};
@@ -255,8 +255,8 @@ __global__ __launch_bounds__(kBX* kBY) void k_compat_e3d(const KGrid g) {
   }
 }
 
-void launch_compat_flags_clear(int* flags, hipStream_t s) {
-  hipLaunchKernelGGL(k_flags_clear, dim3(1), dim3(64), 0, s, flags);
+void launch_compat_flags_clear(int* flags, int sets, hipStream_t s) {
+  hipLaunchKernelGGL(k_flags_clear, dim3(1), dim3(64), 0, s, flags, 8 * sets);
 }
 
 void launch_compat_flags2d(const KGrid& g, hipStream_t s) {

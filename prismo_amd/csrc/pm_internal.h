@@ -178,7 +178,7 @@ struct FusedBufs {
 void launch_yee_h(const KGrid& g, int precision, int coeff_kind, hipStream_t s);
 void launch_yee_e(const KGrid& g, int precision, int coeff_kind, hipStream_t s);
 void launch_compat_flags2d(const KGrid& g, hipStream_t s);
-void launch_compat_flags_clear(int* flags, hipStream_t s);
+void launch_compat_flags_clear(int* flags, int sets, hipStream_t s);
 void launch_compat_h(const KGrid& g, int coeff_kind, hipStream_t s);
 // fill (2-D): flags_next is filled too, from the cells outside src[0 .. n_src).
 void launch_compat_e(const KGrid& g, int coeff_kind, bool fill, const KSrc* src, int n_src,

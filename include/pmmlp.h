@@ -96,8 +96,8 @@ int pm_mlp_net_forward(void* stream, int32_t batch, int32_t M, int32_t layers,
  * lr[s] (a host array) and decay weight_decay on the weights.  Row r of member
  * q is row idx[q * stride_idx + r] of X and T (shared by the members).  packed
  * (train != 0) holds P's weights and is kept up to date; work:
- * batch * pm_mlp_net_work(.., batch_rows) elements; loss[s * batch + q], zeroed
- * by the caller. */
+ * batch * pm_mlp_net_work(.., batch_rows) elements, 16-byte aligned (else
+ * PM_EINVAL); loss[s * batch + q], zeroed by the caller. */
 int64_t pm_mlp_net_work(int32_t layers, const int32_t* sizes, int32_t rows);
 int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t* sizes, float* P,
                      float* G, float* m, float* v, int64_t stride_p, uint16_t* packed,

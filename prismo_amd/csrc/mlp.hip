@@ -1070,8 +1070,11 @@ int pm_mlp_net_train(void* stream, int32_t batch, int32_t layers, const int32_t*
                      float* work, const float* lr, float beta1, float beta2, float eps,
                      float weight_decay, int32_t t0, float* loss) {
   NetDesc d;
+  // (work is read and written 16 bytes at a time)
   if (!net_desc(layers, sizes, &d) || !P || !G || !m || !v ||
-      !packed_ok(packed, stride_packed) || !X || !T || !idx || !work || !lr || !loss || batch < 1 || batch > 65535 || rows < 1 || batch_rows < 1 || t0 < 0)
+      !packed_ok(packed, stride_packed) || !X || !T || !idx || !work ||
+      (uintptr_t)work % 16 != 0 || !lr || !loss || batch < 1 || batch > 65535 || rows < 1 ||
+      batch_rows < 1 || t0 < 0)
     return PM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   const size_t lds = (size_t)16 * d.kp * sizeof(unsigned short) + d.ngrad * sizeof(float);

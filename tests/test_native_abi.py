@@ -42,6 +42,19 @@ def test_errors_without_device_are_reported():
     assert rc != 0 and not h.value
 
 
+@pytest.mark.parametrize("off", [2, 4, 8, 12])
+def test_net_train_refuses_an_unaligned_workspace(off):
+    """Host check, before anything is launched."""
+    lib = N.load()
+    sizes = (C.c_int32 * 2)(4, 4)
+    buf = (C.c_char * 8192)()
+    base = (C.addressof(buf) + 15) // 16 * 16
+    rc = lib.pm_mlp_net_train(None, 1, 1, sizes, base, base, base, base, 20, base, 512, base, base,
+                              base, 1, None, 1, 1, base + off, base, 0.9, 0.999, 1e-8, 0.0, 0,
+                              base)
+    assert rc == -1
+
+
 PROBE = r"""
 #include <stddef.h>
 #include <stdio.h>

@@ -47,8 +47,8 @@ typedef struct pm_batch_design {
   void* hy[2];
   void* psi_hx[2];           /* H-side CPML memory (dEz/dy at Hx, dEz/dx at Hy), ping-pong */
   void* psi_hy[2];
-  void* psi_ex;              /* E-side CPML memory of Ez (dHy/dx, dHx/dy terms); the second
-                                set is in the plan's workspace */
+  void* psi_ex;              /* E-side CPML memory of Ez (dHy/dx, dHx/dy terms), current
+                                whenever a call returns */
   void* psi_ey;
   const void* cb;            /* Cb at Ez points: field precision, or FP16 (coeff_kind CB_F16) */
   double cb_scale;           /* FP16 Cb = cb_scale * stored value (1 otherwise) */

@@ -8,8 +8,9 @@
 // us, 18 a step, two thirds of which the vector ALU is busy (a third of the tiles
 // of a coupler touch a CPML layer).  Reads come from field set `par`, writes go
 // to set par ^ 1, so neighbouring tiles never see a half-updated value; the CPML
-// memory of both field halves is ping-ponged for the same reason (the second
-// E-side set is in the workspace).  Sources are added after the E update, samples
+// memory of both field halves is ping-ponged for the same reason.  The plan has
+// one E-side set; the second is in the workspace, and calls begin and end with
+// the state in the plan's.  Sources are added after the E update, samples
 // are taken after the sources, as src/prismo/core/simulation.py:147-164 orders
 // them.
 #include <hip/hip_runtime.h>
@@ -207,6 +208,34 @@ __global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64
   if (bad >> 31) atomicOr(k.status + wk.d, 1);
 }
 
+// The layers of every design (blockIdx.y) from the plan's E-side CPML memory to the
+// workspace's (pack) or back: at the ends of a call whose state is in set 1.
+template <typename T>
+__global__ __launch_bounds__(256) void k_batch_psi(const KDesign* des, int pack) {
+  const KDesign& KD = des[blockIdx.y];
+  const pm_batch_design& D = KD.d;
+  const int sx = D.pml[0] + D.pml[1], sl = D.pml[2] + D.pml[3];
+  const int64_t n = (int64_t)sx * D.ny, m = n + (int64_t)sl * D.nx;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < m;
+       e += (int64_t)gridDim.x * 256) {
+    T *full, *second;
+    int64_t o;
+    if (e < n) {
+      const int s = (int)(e % sx);
+      full = (T*)D.psi_ex;
+      second = (T*)KD.psi_ex1;
+      o = e / sx * D.sy + (s < D.pml[0] ? s : D.nx - sx + s);
+    } else {
+      const int s = (int)((e - n) / D.nx), i = (int)((e - n) % D.nx);
+      full = (T*)D.psi_ey;
+      second = (T*)KD.psi_ey1;
+      o = (int64_t)(s < D.pml[2] ? s : D.ny - sl + s) * D.sy + i;
+    }
+    if (pack) second[o] = full[o];
+    else full[o] = second[o];
+  }
+}
+
 __global__ void k_clock_set(int64_t* clock, int64_t v) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *clock = v;
 }
@@ -397,6 +426,28 @@ int launch_steps(pm_batch* b, int64_t step, int use_clock, int s_rel, int ns, in
   return bhip(b, hipGetLastError(), "batch step launch");
 }
 
+// With the state in set 1: its E-side CPML memory from the plan's arrays into
+// the workspace (before steps, pack) or back (after them).
+int move_psi(pm_batch* b, bool pack) {
+  if (b->parity == 0) return 0;
+  int64_t most = 0;
+  for (const pm_batch_design& D : b->des)
+    most = std::max(most, (int64_t)(D.pml[0] + D.pml[1]) * D.ny +
+                              (int64_t)(D.pml[2] + D.pml[3]) * D.nx);
+  if (most == 0) return 0;
+  const unsigned nb = (unsigned)std::min<int64_t>((most + 255) / 256, 256);
+  for (size_t d0 = 0; d0 < b->des.size(); d0 += 65535) {
+    const dim3 grid(nb, (unsigned)std::min<size_t>(b->des.size() - d0, 65535));
+    if (b->plan.precision == PM_FP64)
+      hipLaunchKernelGGL(k_batch_psi<double>, grid, dim3(256), 0, b->stream, b->kb.des + d0,
+                         pack ? 1 : 0);
+    else
+      hipLaunchKernelGGL(k_batch_psi<float>, grid, dim3(256), 0, b->stream, b->kb.des + d0,
+                         pack ? 1 : 0);
+  }
+  return bhip(b, hipGetLastError(), "batch CPML memory launch");
+}
+
 int flush_block(pm_batch* b, int64_t first, int rows, const int64_t* wclock) {
   const pm_batch_plan& p = b->plan;
   if (p.nfreq == 0 || rows == 0) return 0;
@@ -570,6 +621,10 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
     return bfail(b, PM_EINVAL, "graph replay needs a non-default stream");
   int64_t left = nsteps;
   bool clock_ok = false;
+  if (left > 0) {
+    const int r = move_psi(b, true);
+    if (r) return r;
+  }
   while (left > 0) {
     if (graphs && b->step % T == 0 && b->pend_n == 0 && left >= T) {
       int r = 0;
@@ -615,7 +670,7 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
       b->pend0 = b->step;
     }
   }
-  return 0;
+  return nsteps > 0 ? move_psi(b, false) : 0;
 }
 
 int pm_batch_flush(pm_batch* b) {

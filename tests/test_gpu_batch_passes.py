@@ -53,3 +53,68 @@ def test_tall_tiles(mi355x, storage):
     """With 1.2 M cells and more in the batch a tile has 48 rows."""
     _same(_run([(33, 81)], np.float32, storage, 32, [90], True),
           _run([(33, 81), (1100, 1100)], np.float32, storage, 32, [90], True))
+
+
+def _engine(dtype, n):
+    from prismo_amd.core.batch import BatchEngine
+
+    sims = [_design(nx, ny, 8, dtype, 100 + k)[0] for k, (nx, ny) in enumerate([(33, 17), (60, 40)])]
+    eng = BatchEngine(sims, dtype=dtype, sample_T=20)
+    eng._build(n)
+    return eng
+
+
+def _replan(eng, at):
+    """The plan again from the state a call left, at step `at`: the sets swapped
+    where that is in set 1, CPML memory of Ez as it stands."""
+    swap = eng.ctx.parity()
+    eng.ctx.sync()
+    for des in eng._arr:
+        for name in eng._FIELD_ARRAYS if swap else ():
+            a = getattr(des, name)
+            a[0], a[1] = a[1], a[0]
+    p = eng.plan
+    p.src_e_table += 8 * at
+    p.src_h_table += 8 * at
+    p.table_step0, p.table_len, p.nfreq = at, p.table_len - at, 0
+    eng.ctx.configure(p, keep=[eng._arr])
+    return swap
+
+
+def _state(eng, swap=0):
+    eng.ctx.sync()
+    q = eng.ctx.parity() ^ swap
+    return [t.cpu().numpy() for b in eng._bufs
+            for t in [b[n][q] for n in eng._FIELD_ARRAYS] + [b["psi_ex"], b["psi_ey"]]]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("cut", [1, 8, 11, 16, 29])
+def test_state_between_calls(mi355x, dtype, cut):
+    """After any call the design's arrays hold the whole state: fields and H-side
+    memory in the set of pm_batch_parity, E-side memory in its one array.  A run
+    goes on from them in a new plan, and from zeros put into them."""
+    import torch
+
+    n = 50
+    ref = _engine(dtype, n)
+    ref.ctx.run(n, graph=False)
+    a = _engine(dtype, n)
+    a.ctx.run(cut, graph=False)
+    swap = _replan(a, cut)
+    a.ctx.run(n - cut, graph=False)
+    for x, y in zip(_state(a, swap), _state(ref)):
+        assert np.array_equal(x, y)
+    assert np.linalg.norm(_state(ref)[-2]) > 0
+
+    z = _engine(dtype, n)
+    z.ctx.run(cut, graph=False)
+    z.ctx.sync()
+    z._arena.zero_()
+    z.stream.wait_stream(torch.cuda.current_stream())
+    z.ctx.run(n - cut, graph=False)
+    fresh = _engine(dtype, n)
+    _replan(fresh, cut)
+    fresh.ctx.run(n - cut, graph=False)
+    for x, y in zip(_state(z), _state(fresh)):
+        assert np.array_equal(x, y)

@@ -9,8 +9,9 @@
 // of a coupler touch a CPML layer).  Reads come from field set `par`, writes go
 // to set par ^ 1, so neighbouring tiles never see a half-updated value; the CPML
 // memory of both field halves is ping-ponged for the same reason.  The plan has
-// one E-side set; the second is in the workspace, and calls begin and end with
-// the state in the plan's.  Sources are added after the E update, samples
+// one E-side set, which spans the grid; the second, in the workspace, holds the
+// layers alone (28 k values, not 334 k, for 540 x 290 cells with 16 layers a
+// side), and calls begin and end with the state in the plan's.  Sources are added after the E update, samples
 // are taken after the sources, as src/prismo/core/simulation.py:147-164 orders
 // them.
 #include <hip/hip_runtime.h>
@@ -31,7 +32,8 @@ struct KWork {
   int d, x0, y0;
 };
 
-// A design and the second set of its E-side CPML memory.
+// A design and the second set of its E-side CPML memory: x layers (pml[0] +
+// pml[1] values per row), y layers (pml[2] + pml[3] rows of sy).
 struct KDesign {
   pm_batch_design d;
   void* psi_ex1;
@@ -64,18 +66,21 @@ struct BatchY {
 // out; most tiles have none.
 template <typename T>
 struct BatchIo {
-  static constexpr bool kStatus = true;
+  static constexpr bool kStatus = true, kPackedE = true;
   static_assert(PM_BATCH_MAX_LINES <= 64 && kTmS <= 64, "one lane per entry");
   const KBatch& k;
   const pm_batch_design& D;
   int64_t step;      // of the pass's first step
   int x0, y0, rows;  // what the tile writes: columns x0 .., rows y0 ..
+  int par;           // the set read
   int comp, col, li, j0, j1;  // this lane's line
   T ve, vh;
   int se_i, se0, se1, sh_i, sh0, sh1;
   bool hit_e, hit_h;
   unsigned mask;
   gptr<T> X;
+
+  __device__ __forceinline__ bool packed(bool out) const { return (par != 0) != out; }
 
   __device__ __forceinline__ void first() {
     const int lane = threadIdx.x & 63;
@@ -202,7 +207,8 @@ __global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64
     xp.ikh = prof[5 * nx + i];
   }
   const BatchY<T> yp{prof + 6 * (int64_t)nx};
-  BatchIo<T> io{k, D, use_clock ? *k.clock + s_rel : step_arg, x0, y0, tm_rows(R)};
+  BatchIo<T> io{k, D, use_clock ? *k.clock + s_rel : step_arg, x0, y0, tm_rows(R),
+                par};
   const uint32_t bad = tm_tile<T, CK, R>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
   // a diverged design is flagged by the lanes that saw it (rare)
   if (bad >> 31) atomicOr(k.status + wk.d, 1);
@@ -218,21 +224,18 @@ __global__ __launch_bounds__(256) void k_batch_psi(const KDesign* des, int pack)
   const int64_t n = (int64_t)sx * D.ny, m = n + (int64_t)sl * D.nx;
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < m;
        e += (int64_t)gridDim.x * 256) {
-    T *full, *second;
-    int64_t o;
+    T *full, *layers;
     if (e < n) {
       const int s = (int)(e % sx);
-      full = (T*)D.psi_ex;
-      second = (T*)KD.psi_ex1;
-      o = e / sx * D.sy + (s < D.pml[0] ? s : D.nx - sx + s);
+      full = (T*)D.psi_ex + e / sx * D.sy + (s < D.pml[0] ? s : D.nx - sx + s);
+      layers = (T*)KD.psi_ex1 + e;
     } else {
       const int s = (int)((e - n) / D.nx), i = (int)((e - n) % D.nx);
-      full = (T*)D.psi_ey;
-      second = (T*)KD.psi_ey1;
-      o = (int64_t)(s < D.pml[2] ? s : D.ny - sl + s) * D.sy + i;
+      full = (T*)D.psi_ey + (int64_t)(s < D.pml[2] ? s : D.ny - sl + s) * D.sy + i;
+      layers = (T*)KD.psi_ey1 + (int64_t)s * D.sy + i;
     }
-    if (pack) second[o] = full[o];
-    else full[o] = second[o];
+    if (pack) *layers = *full;
+    else *full = *layers;
   }
 }
 
@@ -323,8 +326,11 @@ void build_work(const pm_batch_plan& p, int rows, std::vector<KWork>& work) {
   }
 }
 
-int64_t psi_bytes(const pm_batch_plan& p, const pm_batch_design& D) {
-  return align256((int64_t)D.ny * D.sy * (p.precision == PM_FP64 ? 8 : 4));
+// Second E-side CPML memory of the x (axis 0) or y layers of a design; without
+// layers one value is still read.
+int64_t psi_bytes(const pm_batch_plan& p, const pm_batch_design& D, int axis) {
+  const int64_t n = (int64_t)(D.pml[2 * axis] + D.pml[2 * axis + 1]) * (axis ? D.sy : D.ny);
+  return align256(std::max<int64_t>(n, 1) * (p.precision == PM_FP64 ? 8 : 4));
 }
 
 // (sized for the shortest tiles, whichever the device gets)
@@ -337,7 +343,8 @@ Layout layout(const pm_batch_plan& p) {
   l.status = align256(l.work + (int64_t)(sizeof(KWork) * w.size()));
   l.psi = align256(l.status + (int64_t)sizeof(int32_t) * p.n_design);
   l.total = l.psi;
-  for (int d = 0; d < p.n_design; ++d) l.total += 2 * psi_bytes(p, p.design[d]);
+  for (int d = 0; d < p.n_design; ++d)
+    l.total += psi_bytes(p, p.design[d], 0) + psi_bytes(p, p.design[d], 1);
   return l;
 }
 
@@ -562,9 +569,9 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   std::vector<KDesign> kd(b->des.size());
   char* psi = ws + l.psi;
   for (size_t d = 0; d < kd.size(); ++d) {
-    const int64_t n = psi_bytes(*p, b->des[d]);
+    const int64_t n = psi_bytes(*p, b->des[d], 0);
     kd[d] = KDesign{b->des[d], psi, psi + n};
-    psi += 2 * n;
+    psi += n + psi_bytes(*p, b->des[d], 1);
   }
   KBatch& k = b->kb;
   k.clock = (int64_t*)ws;

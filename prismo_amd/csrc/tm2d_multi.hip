@@ -35,7 +35,8 @@ struct SimIoArgs {
 // Boxes that do not meet the tile are masked out; most tiles have none.
 template <typename T>
 struct SimIo {
-  static constexpr bool kStatus = false;
+  static constexpr bool kStatus = false, kPackedE = false;
+  __device__ __forceinline__ static constexpr bool packed(bool) { return false; }
   static_assert(kMaxSrc * 4 <= 64 && kMaxSrc + kMaxSbox <= 64 && kTmS % 4 == 0, "lanes");
   const SimIoArgs& a;
   int x0, y0, rows;  // what the tile writes: columns x0 .., rows y0 ..

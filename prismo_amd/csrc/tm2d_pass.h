@@ -151,7 +151,9 @@ struct TmShared {
 // io.first() and io.second() issue their own loads before and behind the fields';
 // io.sources(s, ...), io.samples(s, ...) act on the registers after step s.  With
 // IO::kStatus, returns bit 31 set when an Ez value this lane wrote is Inf or NaN
-// (a value that was stays so: it is looked at after the last step).
+// (a value that was stays so: it is looked at after the last step).  With
+// IO::kPackedE, where g.full, the E set that is read or the one that is written
+// holds the layers alone (io.packed(false), io.packed(true)).
 template <typename T, int CK, int R, bool XP, bool YP, class YProf, class IO>
 __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& xp, bool xpml,
                                             const YProf& yp, IO& io, int ns, int x0, int y0,
@@ -171,12 +173,19 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
   T qhx[XP ? R : 1], qex[XP ? R : 1];  // x layers: Hy and Ez terms
   T qhy[YP ? R : 1], qey[YP ? R : 1];  // y layers: Hx and Ez terms
   // (lanes outside the layers read position 0 of a row)
-  const uint32_t xo = !xpml ? 0u
-                      : g.full ? (uint32_t)ic
-                               : (uint32_t)(i < g.px0 ? i : g.px0 + (i - (nx - g.px1)));
+  const uint32_t xslab = (uint32_t)(i < g.px0 ? i : g.px0 + (i - (nx - g.px1)));
+  const uint32_t xo = !xpml ? 0u : g.full ? (uint32_t)ic : xslab;
   auto yrow = [&](int j) {  // y layers: row of the memory array
     if (g.full) return (uint32_t)j;
     return (uint32_t)(j < g.py0 ? j : g.py0 + (j - (ny - g.py1)));
+  };
+  // where IO::kPackedE: positions in the E set that is read (out false) or written
+  auto xe = [&](bool out, uint32_t row) {
+    return io.packed(out) ? xslab + (uint32_t)(g.px0 + g.px1) * row : xo + g.xst * row;
+  };
+  auto ye = [&](bool out, int j) {
+    const int gap = io.packed(out) ? ny - g.py0 - g.py1 : 0;
+    return (uint32_t)(j < g.py0 ? j : j - gap);
   };
   auto ypml = [&](int j) { return j >= 0 && j < ny && (j < g.py0 || j >= ny - g.py1); };
   io.first();
@@ -203,14 +212,18 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     }
     if constexpr (XP) {
       const uint32_t q = xpml ? xo + g.xst * (uint32_t)jc : 0u;
-      const T h = ((gptr<const T>)g.ps[0])[q], f = ((gptr<const T>)g.ps[2])[q];
+      uint32_t qe = q;
+      if constexpr (IO::kPackedE) qe = xpml ? xe(false, (uint32_t)jc) : 0u;
+      const T h = ((gptr<const T>)g.ps[0])[q], f = ((gptr<const T>)g.ps[2])[qe];
       qhx[r] = ok && xpml ? h : (T)0;
       qex[r] = ok && xpml ? f : (T)0;
     }
     if constexpr (YP) {
       const bool in = ypml(j);
       const uint32_t q = in ? (uint32_t)ic + g.yst * yrow(j) : 0u;
-      const T h = ((gptr<const T>)g.ps[1])[q], f = ((gptr<const T>)g.ps[3])[q];
+      uint32_t qe = q;
+      if constexpr (IO::kPackedE) qe = in ? (uint32_t)ic + g.yst * ye(false, j) : 0u;
+      const T h = ((gptr<const T>)g.ps[1])[q], f = ((gptr<const T>)g.ps[3])[qe];
       qhy[r] = ok && in ? h : (T)0;
       qey[r] = ok && in ? f : (T)0;
     }
@@ -314,15 +327,19 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     if constexpr (XP) {
       if (xpml) {
         const uint32_t q = xo + g.xst * (uint32_t)j;
+        uint32_t qe = q;
+        if constexpr (IO::kPackedE) qe = xe(true, (uint32_t)j);
         ((gptr<T>)g.ps_o[0])[q] = qhx[r];
-        ((gptr<T>)g.ps_o[2])[q] = qex[r];
+        ((gptr<T>)g.ps_o[2])[qe] = qex[r];
       }
     }
     if constexpr (YP) {
       if (ypml(j)) {
         const uint32_t q = (uint32_t)i + g.yst * yrow(j);
+        uint32_t qe = q;
+        if constexpr (IO::kPackedE) qe = (uint32_t)i + g.yst * ye(true, j);
         ((gptr<T>)g.ps_o[1])[q] = qhy[r];
-        ((gptr<T>)g.ps_o[3])[q] = qey[r];
+        ((gptr<T>)g.ps_o[3])[qe] = qey[r];
       }
     }
   }

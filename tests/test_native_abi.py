@@ -55,6 +55,26 @@ def test_net_train_refuses_an_unaligned_workspace(off):
     assert rc == -1
 
 
+@pytest.mark.parametrize("precision,esz", [(N.FP32, 4), (N.FP64, 8)])
+def test_batch_workspace_holds_layers_not_grids(precision, esz):
+    """The second E-side CPML memory of a batch: what its layers take, beside the
+    tables (under 2 % of one array of the grid)."""
+    d = (N.pm_batch_design * 3)()
+    layers = grid = 0
+    for q, (nx, ny, t) in enumerate([(700, 500, 16), (701, 503, 0), (640, 900, 7)]):
+        d[q].nx, d[q].ny, d[q].sy = nx, ny, (nx + 63) // 64 * 64
+        for k in range(4):
+            d[q].pml[k] = t
+        layers += 2 * t * (ny + d[q].sy) * esz
+        grid += ny * d[q].sy * esz
+    p = N.pm_batch_plan()
+    p.precision, p.coeff_kind, p.n_design, p.chunk = precision, N.COEFF_CB, 3, 8
+    p.design = C.cast(d, C.POINTER(N.pm_batch_design))
+    n = C.c_int64()
+    assert N.load().pm_batch_workspace_bytes(C.byref(p), C.byref(n)) == 0
+    assert layers <= n.value <= layers + 0.02 * grid
+
+
 PROBE = r"""
 #include <stddef.h>
 #include <stdio.h>

@@ -1,8 +1,7 @@
 """GPU: batched 2-D TM stepping (include/pmbatch.h, prismo_amd/core/batch.py)
 against the O1 oracle, design by design.
 
-Designs of uneven size (strip and chunk tails, several tiles per design)
-with CPML, a PlaneWaveSource line (Ez and Hy) and a FieldMonitor port line
+Designs of uneven size (tile tails, several tiles per design) with CPML, a PlaneWaveSource line (Ez and Hy) and a FieldMonitor port line
 (Ez, Hy) with spectra.  FP64: fields and spectra within 1e-10 relative L2 of
 O1; FP32 fields with FP16 Cb: within 1e-5 of O1 fed the same dequantised
 Cb.  Graph replay of the step loop gives the same bits as eager launches.
@@ -15,9 +14,7 @@ from tests.conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 D = 20e-9
-# with 8-cell CPML: 86, 146, 61 and 68 cells along x; strips of 64 cells
-# give tails, a one-strip design and (68) a strip whose right neighbour
-# cell, x = 64, lies in the x CPML
+# with 8-cell CPML: 86, 146, 61 and 68 cells along x, two to four tiles of 48
 SIZES = [(70, 40), (130, 25), (45, 90), (52, 33)]
 FREQS = [187e12, 193e12, 200e12, 205e12]
 
@@ -135,9 +132,10 @@ def _spectra(built):
 
 
 def test_batch_launch_shapes_and_autotune_are_bitwise(mi355x):
-    """Every launch shape (rows per tile, waves per workgroup, workgroup
-    order) gives the same bits, and so does the autotuner's pick; the tuner
-    leaves the engine at the zero state a run starts from."""
+    """Both workgroup orders, whatever rows per tile and waves are asked for beside
+    them (taken and not used), give the same bits, and so does the autotuner's
+    pick; the tuner leaves the engine at the zero state a run starts from.  The
+    tiles themselves: test_gpu_batch_passes."""
     from prismo_amd import autotune
     from prismo_amd.core.batch import BatchEngine
 

@@ -1,23 +1,27 @@
 """GPU: the batched step's passes of up to eight steps.
 
-A cell's arithmetic depends neither on the tile it lies in nor on how a run is
-cut into passes, so everything here is compared bit for bit.
+A cell's arithmetic depends neither on the tile it lies in (48 columns by 16
+rows, or by 48 in FP32 from 1.18 M cells in the batch on) nor on how a run is
+cut into passes, so everything here is compared bit for bit, and at the tiles'
+edges with the O1 oracle (1e-10 relative L2 in FP64, 1e-5 in FP32).
 """
 
 import numpy as np
 import pytest
 
+from tests.conftest import rel_l2
 from tests.test_gpu_batch import _design
 
 pytestmark = pytest.mark.gpu
 
 
-def _run(sizes, dtype, storage, T, runs, graph):
+def _run(sizes, dtype, storage, T, runs, graph, xcd=1):
     from prismo_amd.core.batch import BatchEngine
 
     built = [_design(nx, ny, 8, dtype, 100 + k) for k, (nx, ny) in enumerate(sizes)]
     eng = BatchEngine([b[0] for b in built], dtype=dtype, coefficient_storage=storage,
                       sample_T=T)
+    eng.ctx.set_tuning(4, xcd)
     eng._build(sum(runs))
     for n in runs:
         eng.ctx.run(n, graph=graph)
@@ -53,6 +57,38 @@ def test_tall_tiles(mi355x, storage):
     """With 1.2 M cells and more in the batch a tile has 48 rows."""
     _same(_run([(33, 81)], np.float32, storage, 32, [90], True),
           _run([(33, 81), (1100, 1100)], np.float32, storage, 32, [90], True))
+
+
+@pytest.mark.parametrize("tall", [False, True])
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-10), (np.float32, 1e-5)])
+def test_tile_edges_match_oracle(mi355x, dtype, bar, tall):
+    """Designs one cell short of a tile's edge, on it and past it, alone and (tall)
+    beside one that takes an FP32 batch to 48-row tiles."""
+    from prismo_amd.core.batch import BatchEngine
+    from tests.test_gpu_batch import _drive, _oracle
+
+    t, steps = 8, 61
+    cells = [(47, 33), (48, 32), (49, 47), (96, 48), (97, 49), (144, 65)]
+    sizes = [(nx - 2 * t, ny - 2 * t) for nx, ny in cells] + ([(1100, 1100)] if tall else [])
+    built = [_design(nx, ny, t, dtype, 100 + k) for k, (nx, ny) in enumerate(sizes)]
+    eng = BatchEngine([b[0] for b in built], dtype=dtype, sample_T=20)
+    eng.run_steps(steps)
+    for d, (nx, ny) in enumerate(cells):
+        sim, eps = built[d]
+        assert tuple(sim.grid.dimensions[:2]) == (nx, ny)
+        o1, ref = _oracle(sim, eps, t, eng.cb_host[d])
+        _drive(o1, ref, sim, steps)
+        got = eng.fields(d)
+        a = np.concatenate([got[c].ravel() for c in ("Ez", "Hx", "Hy")])
+        b = np.concatenate([o1.F[c].ravel() for c in ("Ez", "Hx", "Hy")])
+        assert np.linalg.norm(b) > 0 and rel_l2(a, b) <= bar, d
+
+
+@pytest.mark.parametrize("sizes", [[(33, 17), (81, 49)], [(33, 81), (1100, 1100)]])
+def test_workgroup_order(mi355x, sizes):
+    """Grouped by XCD or in launch order, 16- and 48-row tiles: the same bits."""
+    _same(_run(sizes, np.float32, "fp16", 20, [45], True, xcd=0),
+          _run(sizes, np.float32, "fp16", 20, [45], True, xcd=1))
 
 
 def _engine(dtype, n):

@@ -1,9 +1,10 @@
 """GPU: several 2-D TM steps per launch (the default for lossless and
 conductive 2-D runs) against the unfused kernels and O1.
 
-Widths and heights sit at the edges of the tiles (56 columns, 8 / 24 / 56
-rows), run lengths leave every remainder of the 4 steps a launch takes and
-cross the ends of the 128-row sample blocks.  The unfused kernels do the same
+A tile is 48 columns by 16 rows, or by 48 (FP32 from 1.18 M cells on 256
+compute units on); a launch takes up to 8 steps.  Widths and heights sit at the
+edges of the tiles, run lengths leave every remainder of the 8 steps and cross
+the ends of the 128-row sample blocks.  The unfused kernels do the same
 operations per cell: 1e-13 relative L2 in FP64, 1e-6 in FP32; O1 at 1e-10 /
 1e-5, the bars of the other 2-D paths.
 """
@@ -87,6 +88,16 @@ def test_fp64_equals_unfused(mi355x, shape, t, runs):
     _both(*shape, t, np.float64, runs, 1e-13)
 
 
+@pytest.mark.parametrize("shape,t", [((47, 33), 5), ((48, 32), 0), ((49, 16), 3), ((96, 17), 4),
+                                     ((97, 49), 0), ((95, 48), 9), ((40, 15), 0), ((144, 47), 8)])
+@pytest.mark.parametrize("runs", [[9, 135], [6, 7, 131], [2, 12, 4, 5]])
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-13), (np.float32, 1e-6)])
+def test_tile_edges_equal_unfused(mi355x, shape, t, runs, dtype, bar):
+    """One cell short of a tile's edge, on it and past it, in both directions,
+    from fields everywhere."""
+    _both(*shape, t, dtype, runs, bar, start=True)
+
+
 @pytest.mark.parametrize("dtype,storage,bar", [(np.float64, "auto", 1e-13),
                                                (np.float32, "auto", 1e-6),
                                                (np.float32, "fp16", 1e-6)])
@@ -103,8 +114,18 @@ def test_conductive_media(mi355x, dtype, bar):
                                              ((1000, 800), np.float32, 1e-6),
                                              ((1500, 1201), np.float32, 1e-6)])
 def test_taller_tiles(mi355x, shape, dtype, bar):
-    """Grids large enough for 24- and 56-row tiles."""
+    """Many 16-row tiles, and a grid large enough for 48-row ones."""
     _both(*shape, 10, dtype, [22], bar, start=True)
+
+
+@pytest.mark.parametrize("shape", [(1152, 1152), (1153, 1103), (1199, 1057)])
+@pytest.mark.parametrize("kw", [{}, {"storage": "fp16"}, {"sigma": True}, {"extra": True}],
+                         ids=["cb", "fp16", "conductive", "sources"])
+def test_48_row_tiles(mi355x, shape, kw):
+    """FP32 grids of 1.18 M cells and more (24 tiles of 48 rows exactly, 23 less one
+    row, 22 and one row), with every kind of coefficients and sources, past the end
+    of a sample block."""
+    _both(*shape, 10, np.float32, [133, 6, 15], 1e-6, start=True, **kw)
 
 
 @pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-10), (np.float32, 1e-5)])

@@ -41,7 +41,8 @@ CANDIDATES2 = {
 CANDIDATES_2D = (1, 2, 3, 4, 8)
 
 # batched 2-D step: workgroup order.  Tiles follow a rule in the library; the
-# plan's chunk and the waves asked for do not change the launch
+# plan's chunk and the waves asked for are checked and do not change the launch,
+# so there is one of each (candidates of a caller's own may hold more)
 BATCH_CANDIDATES = {
     "chunk": (8,),
     "waves": (4,),
@@ -183,10 +184,10 @@ def tune_batch(eng, steps: int = 16, candidates: dict | None = None,
     """Pick and apply the fastest launch shape of the batched step for the
     configured, not yet run ``BatchEngine`` ``eng``: each candidate (workgroup
     order) runs ``steps`` eager steps timed with HIP events on the engine's
-    stream; then the engine's state is cleared back to the zeros a run starts from and it is re-planned with
-    the pick.  Results are bitwise the same under every shape (each cell's
-    arithmetic does not depend on the tiling); cached per (precision,
-    coefficient storage, designs per batch) like ``tune``.
+    stream; then the engine's state is cleared back to the zeros a run starts
+    from and it is re-planned with the pick.  Results are bitwise the same
+    under either (each cell's arithmetic does not depend on the tiling); cached
+    per (precision, coefficient storage, designs per batch) like ``tune``.
 
     Returns {"chunk", "waves", "xcd", "ms", "cached"}."""
     _load_file()

@@ -69,7 +69,8 @@ class BatchEngine:
                 raise NotImplementedError("every design must share dx, dy and dt")
         self.sample_T = int(sample_T)
         # "auto": the autotuner picks the workgroup order when the run starts
-        # (prismo_amd.autotune.tune_batch); tiles follow a rule in the library
+        # (prismo_amd.autotune.tune_batch).  Tiles follow a rule in the library:
+        # a number is checked (>= 2) and changes nothing
         self.auto_tune = chunk == "auto"
         self.chunk = 8 if self.auto_tune else int(chunk)
         self.tuning = None
@@ -367,13 +368,6 @@ class BatchEngine:
             p.W_re, p.W_im = Wre.data_ptr(), Wim.data_ptr()
         p.chunk = self.chunk
         wsb = self.ctx.workspace_bytes(p)
-        if self.auto_tune:
-            from ..autotune import BATCH_CANDIDATES
-
-            for c in BATCH_CANDIDATES["chunk"]:
-                p.chunk = c
-                wsb = max(wsb, self.ctx.workspace_bytes(p))
-            p.chunk = self.chunk
         ws = self._alloc((wsb,), torch.uint8)
         p.work, p.work_bytes = ws.data_ptr(), wsb
         self.plan = p

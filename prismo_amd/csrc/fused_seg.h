@@ -5,10 +5,11 @@
 // 512 cells; every other width (a grid 64, 180 or 301 cells long) stepped H
 // and E in two launches, which moves every field twice.  Segments of 64
 // cells divide any padded row (the pitch is a multiple of 64), so no lane is
-// idle beyond the padding, and a workgroup of TY + 1 waves needs registers
-// for few waves: FP64 takes 7-row tiles here where whole rows of 256 cells
-// fit 2 or 3.  The price is the x halo of every segment (one lane-spread load
-// per plane and the recomputed H of one cell).
+// idle beyond the padding, and a workgroup is TY + 1 waves whatever the row:
+// FP64 takes 3 rows in 4 waves here, two workgroups on a compute unit, where
+// whole rows of 256 cells fit 2 rows in 12 waves.  The price is the x halo of
+// every segment (one lane-spread load per plane and the recomputed H of one
+// cell).
 #pragma once
 #include "fused_kernel.h"
 

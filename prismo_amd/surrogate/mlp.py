@@ -3,13 +3,14 @@ BF16 MFMA kernels (include/pmmlp.h), with FP32 master weights.
 
 Layers: ``n_in -> hidden x depth (GELU) -> n_out``.  Networks of up to 12
 layers and 512 units a layer run whole: the forward pass is one launch (a
-workgroup takes its rows through all layers), a training minibatch three
-(forward with loss and backward, all weight and bias gradients, Adam).  Wider
-or deeper ones, and ``backward`` on its own, take one GEMM per layer with the
-bias and GELU (or its derivative) fused into its epilogue.  Loss: weighted
-MSE.  Optimiser: Adam (decoupled weight decay) on the FP32 masters; products
-round their operands to BF16 and sum in FP32.  ``SurrogateEnsemble`` trains several members from different seeds;
-their spread is the predictive uncertainty.
+workgroup takes its rows through all layers), a training minibatch two
+(forward with loss and backward, then all weight and bias gradients with
+Adam).  Wider or deeper ones, and ``backward`` on its own, take one GEMM per
+layer with the bias and GELU (or its derivative) fused into its epilogue.
+Loss: weighted MSE.  Optimiser: Adam (decoupled weight decay) on the FP32
+masters; products round their operands to BF16 and sum in FP32.
+``SurrogateEnsemble`` trains several members from different seeds; their
+spread is the predictive uncertainty.
 """
 
 from __future__ import annotations
@@ -464,6 +465,9 @@ class SurrogateEnsemble:
         return hist
 
     def predict(self, X, chunk: int = 16384):
+        """Mean and standard deviation over the members.  Networks that run whole
+        take all rows in one launch; the per-layer path ``chunk`` rows at a
+        time."""
         torch = _torch()
         m0, nm, Pn = self.members[0], len(self.members), self.P.shape[1]
         if m0._rows_ok(X, m0.sizes[0]) and all(

@@ -85,7 +85,7 @@ int pm_batch_create(int device, void* stream, pm_batch** out);
 int pm_batch_destroy(pm_batch* b);
 const char* pm_batch_last_error(pm_batch* b);
 
-/* Device workspace the plan needs (tile list, design table, step clock, a second
+/* Device workspace the plan needs (tile lists, design table, step clock, a second
  * E-side CPML memory of the layers: (pml[0] + pml[1]) * ny_d values and
  * (pml[2] + pml[3]) * sy_d per design). */
 int pm_batch_workspace_bytes(const pm_batch_plan* plan, int64_t* bytes);

@@ -43,6 +43,7 @@ struct KDesign {
 struct KBatch {
   const KDesign* des;
   const KWork* work;
+  const KWork* work1;  // of one step
   int ncols, sample_T;
   int64_t* clock;
   int32_t* status;  // per design: bit 0 set once an Ez value was not finite
@@ -64,7 +65,7 @@ struct BatchY {
 // line l and the source values of step l of the pass: loaded beside the fields,
 // read back with lane broadcasts.  Lines that do not meet the tile are masked
 // out; most tiles have none.
-template <typename T>
+template <typename T, int S>
 struct BatchIo {
   static constexpr bool kStatus = true, kPackedE = true;
   static_assert(PM_BATCH_MAX_LINES <= 64 && kTmS <= 64, "one lane per entry");
@@ -72,7 +73,7 @@ struct BatchIo {
   const pm_batch_design& D;
   int64_t step;      // of the pass's first step
   int x0, y0, rows;  // what the tile writes: columns x0 .., rows y0 ..
-  int par;           // the set read
+  int pe;            // the E-side memory set read
   int comp, col, li, j0, j1;  // this lane's line
   T ve, vh;
   int se_i, se0, se1, sh_i, sh0, sh1;
@@ -80,7 +81,7 @@ struct BatchIo {
   unsigned mask;
   gptr<T> X;
 
-  __device__ __forceinline__ bool packed(bool out) const { return (par != 0) != out; }
+  __device__ __forceinline__ bool packed(bool out) const { return (pe != 0) != (S > 1 && out); }
 
   __device__ __forceinline__ void first() {
     const int lane = threadIdx.x & 63;
@@ -104,7 +105,7 @@ struct BatchIo {
 
   // sources act on the halo too, samples on what the tile writes
   __device__ __forceinline__ bool meets(int i, int a, int b, int h) const {
-    return i >= x0 - h && i < x0 + kTmCols + h && a < y0 + rows + h && b > y0 - h && a < b;
+    return i >= x0 - h && i < x0 + tm_cols(S) + h && a < y0 + rows + h && b > y0 - h && a < b;
   }
 
   __device__ __forceinline__ void second(int ns) {
@@ -112,8 +113,8 @@ struct BatchIo {
     const int64_t row = step - k.table_step0 + min(lane, ns - 1);
     ve = (T)((gptr<const double>)k.tab_e)[row];
     vh = (T)((gptr<const double>)k.tab_h)[row];
-    hit_e = meets(se_i, se0, se1, kTmS);
-    hit_h = meets(sh_i, sh0, sh1, kTmS);
+    hit_e = meets(se_i, se0, se1, S);
+    hit_h = meets(sh_i, sh0, sh1, S);
     mask = (unsigned)__ballot(meets(li, j0, j1, 0));
   }
 
@@ -152,15 +153,21 @@ struct BatchIo {
   }
 };
 
-template <typename T, int CK, int R>
+// S = 8: up to eight steps; S = 1: one step, whose tiles have a halo of one cell
+// (62 columns by 30 rows written of 64 by 32, not 48 by 16) and whose E-side
+// memory is updated in place, as no halo cell's E is used.  par: field set read,
+// pe: E-side memory set read.  Calls of one step (32 designs of 532 x 332 cells):
+// with S = 8 46 us FP32, 131 FP64; with S = 1 33 and 82 (one step per launch and
+// no halo: 42 and 84).
+template <typename T, int CK, int R, int S>
 __global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64_t step_arg,
                                                            int use_clock, int s_rel, int ns,
-                                                           int par) {
+                                                           int par, int pe) {
   __shared__ TmShared<T, R> sh;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int b = k.xcd ? tm_order(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-  const KWork wk = k.work[b];
+  const KWork wk = (S > 1 ? k.work : k.work1)[b];
   const KDesign& KD = k.des[wk.d];
   const pm_batch_design& D = KD.d;
   const int x0 = wk.x0, y0 = wk.y0;
@@ -183,19 +190,20 @@ __global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64
   g.cb = D.cb;
   g.ps[0] = D.psi_hy[par];
   g.ps[1] = D.psi_hx[par];
-  g.ps[2] = par ? KD.psi_ex1 : D.psi_ex;
-  g.ps[3] = par ? KD.psi_ey1 : D.psi_ey;
+  g.ps[2] = pe ? KD.psi_ex1 : D.psi_ex;
+  g.ps[3] = pe ? KD.psi_ey1 : D.psi_ey;
   g.ps_o[0] = D.psi_hy[par ^ 1];
   g.ps_o[1] = D.psi_hx[par ^ 1];
-  g.ps_o[2] = par ? D.psi_ex : KD.psi_ex1;
-  g.ps_o[3] = par ? D.psi_ey : KD.psi_ey1;
+  const bool second = (pe != 0) != (S > 1);
+  g.ps_o[2] = second ? KD.psi_ex1 : D.psi_ex;
+  g.ps_o[3] = second ? KD.psi_ey1 : D.psi_ey;
   g.full = true;
   g.idx = k.idx;
   g.idy = k.idy;
   g.db = D.db;
   g.cb_scale = D.cb_scale;
   const gptr<const T> prof = (gptr<const T>)D.prof;
-  const int i = x0 - kTmS + lane;
+  const int i = x0 - S + lane;
   const bool xpml = i >= 0 && i < nx && (i < g.px0 || i >= nx - g.px1);
   TmXProf<T> xp{(T)0, (T)0, (T)1, (T)0, (T)0, (T)1};
   if (xpml) {
@@ -207,9 +215,8 @@ __global__ __launch_bounds__(64 * kTmW, 4) void k_batch_tm(const KBatch k, int64
     xp.ikh = prof[5 * nx + i];
   }
   const BatchY<T> yp{prof + 6 * (int64_t)nx};
-  BatchIo<T> io{k, D, use_clock ? *k.clock + s_rel : step_arg, x0, y0, tm_rows(R),
-                par};
-  const uint32_t bad = tm_tile<T, CK, R>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+  BatchIo<T, S> io{k, D, use_clock ? *k.clock + s_rel : step_arg, x0, y0, tm_rows(R, S), pe};
+  const uint32_t bad = tm_tile<T, CK, R, S>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
   // a diverged design is flagged by the lanes that saw it (rare)
   if (bad >> 31) atomicOr(k.status + wk.d, 1);
 }
@@ -258,15 +265,16 @@ struct pm_batch {
   bool configured = false;
   pm_batch_plan plan{};
   std::vector<pm_batch_design> des;
-  std::vector<KWork> work;
-  int rows = 4;  // rows per wave of a tile
+  std::vector<KWork> work, work1;  // tiles of up to eight steps, of one
+  int rows = 4;                    // rows per wave of a tile
   KBatch kb{};
   KDft dft{};
   int64_t step = 0;   // absolute index of the next step
-  int parity = 0;
+  int parity = 0;     // field set that holds the state
+  int pe = 0;         // E-side memory set
   int64_t pend0 = 0;  // first step of the pending sample block
   int pend_n = 0;
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t graph[4] = {};  // per starting sets: parity + 2 pe
   int n_cu = 256;
   int xcd = 1;  // workgroup order (pm_batch_set_tuning)
   bool timing = false;
@@ -312,17 +320,17 @@ struct BSpan {
 int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 // Workspace: the step clock at offset 0, then the design table, the tile
-// list, one status word per design and the second E-side CPML memory.
+// lists, one status word per design and the second E-side CPML memory.
 struct Layout {
-  int64_t des, work, status, psi, total;
+  int64_t des, work, work1, status, psi, total;
 };
 
-void build_work(const pm_batch_plan& p, int rows, std::vector<KWork>& work) {
+void build_work(const pm_batch_plan& p, int rows, int halo, std::vector<KWork>& work) {
   work.clear();
   for (int d = 0; d < p.n_design; ++d) {
     const pm_batch_design& D = p.design[d];
-    for (int y0 = 0; y0 < D.ny; y0 += tm_rows(rows))
-      for (int x0 = 0; x0 < D.nx; x0 += kTmCols) work.push_back(KWork{d, x0, y0});
+    for (int y0 = 0; y0 < D.ny; y0 += tm_rows(rows, halo))
+      for (int x0 = 0; x0 < D.nx; x0 += tm_cols(halo)) work.push_back(KWork{d, x0, y0});
   }
 }
 
@@ -335,12 +343,14 @@ int64_t psi_bytes(const pm_batch_plan& p, const pm_batch_design& D, int axis) {
 
 // (sized for the shortest tiles, whichever the device gets)
 Layout layout(const pm_batch_plan& p) {
-  std::vector<KWork> w;
-  build_work(p, 4, w);
+  std::vector<KWork> w, w1;
+  build_work(p, 4, kTmS, w);
+  build_work(p, 4, 1, w1);
   Layout l{};
   l.des = 256;
   l.work = align256(l.des + (int64_t)sizeof(KDesign) * p.n_design);
-  l.status = align256(l.work + (int64_t)(sizeof(KWork) * w.size()));
+  l.work1 = align256(l.work + (int64_t)(sizeof(KWork) * w.size()));
+  l.status = align256(l.work1 + (int64_t)(sizeof(KWork) * w1.size()));
   l.psi = align256(l.status + (int64_t)sizeof(int32_t) * p.n_design);
   l.total = l.psi;
   for (int d = 0; d < p.n_design; ++d)
@@ -407,36 +417,44 @@ int validate(pm_batch* b, const pm_batch_plan& p) {
 }
 
 template <typename T, int CK>
-void launch_ck(pm_batch* b, int64_t step_arg, int use_clock, int s_rel, int ns, int par) {
-  const dim3 nb((unsigned)b->work.size()), nt(64 * kTmW);
+void launch_ck(pm_batch* b, int64_t step_arg, int use_clock, int s_rel, int ns, int par, int pe) {
+  const dim3 nt(64 * kTmW), nb((unsigned)(ns == 1 ? b->work1 : b->work).size());
+  if (ns == 1) {
+    hipLaunchKernelGGL((k_batch_tm<T, CK, 4, 1>), nb, nt, 0, b->stream, b->kb, step_arg,
+                       use_clock, s_rel, ns, par, pe);
+    return;
+  }
   if constexpr (sizeof(T) == 4) {
     if (b->rows == 8) {
-      hipLaunchKernelGGL((k_batch_tm<T, CK, 8>), nb, nt, 0, b->stream, b->kb, step_arg,
-                         use_clock, s_rel, ns, par);
+      hipLaunchKernelGGL((k_batch_tm<T, CK, 8, kTmS>), nb, nt, 0, b->stream, b->kb, step_arg,
+                         use_clock, s_rel, ns, par, pe);
       return;
     }
   }
-  hipLaunchKernelGGL((k_batch_tm<T, CK, 4>), nb, nt, 0, b->stream, b->kb, step_arg, use_clock,
-                     s_rel, ns, par);
+  hipLaunchKernelGGL((k_batch_tm<T, CK, 4, kTmS>), nb, nt, 0, b->stream, b->kb, step_arg,
+                     use_clock, s_rel, ns, par, pe);
 }
 
-// ns steps from set `par` into the other
-int launch_steps(pm_batch* b, int64_t step, int use_clock, int s_rel, int ns, int par) {
+// ns steps from field set `par` into the other, and, more than one, from E-side
+// memory set `pe` into the other; both are advanced.
+int launch_steps(pm_batch* b, int64_t step, int use_clock, int s_rel, int ns, int* par, int* pe) {
   const bool f16 = b->plan.coeff_kind == PM_COEFF_CB_F16;
   if (b->plan.precision == PM_FP64) {
-    if (f16) launch_ck<double, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, par);
-    else launch_ck<double, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, par);
+    if (f16) launch_ck<double, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, *par, *pe);
+    else launch_ck<double, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, *par, *pe);
   } else {
-    if (f16) launch_ck<float, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, par);
-    else launch_ck<float, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, par);
+    if (f16) launch_ck<float, PM_COEFF_CB_F16>(b, step, use_clock, s_rel, ns, *par, *pe);
+    else launch_ck<float, PM_COEFF_CB>(b, step, use_clock, s_rel, ns, *par, *pe);
   }
+  *par ^= 1;
+  if (ns > 1) *pe ^= 1;
   return bhip(b, hipGetLastError(), "batch step launch");
 }
 
-// With the state in set 1: its E-side CPML memory from the plan's arrays into
-// the workspace (before steps, pack) or back (after them).
+// With the E-side CPML memory's state in set 1: from the plan's arrays into the
+// workspace (before steps, pack) or back (after them).
 int move_psi(pm_batch* b, bool pack) {
-  if (b->parity == 0) return 0;
+  if (b->pe == 0) return 0;
   int64_t most = 0;
   for (const pm_batch_design& D : b->des)
     most = std::max(most, (int64_t)(D.pml[0] + D.pml[1]) * D.ny +
@@ -467,14 +485,14 @@ int flush_block(pm_batch* b, int64_t first, int rows, const int64_t* wclock) {
 }
 
 int capture(pm_batch* b, int slot) {
-  int par = slot;
+  int par = slot & 1, pe = slot >> 1;
   const pm_batch_plan& p = b->plan;
   hipGraph_t g = nullptr;
   int r = bhip(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
                "begin capture");
   if (r) return r;
-  for (int s = 0; s < p.sample_T && !r; s += kTmS, par ^= 1)
-    r = launch_steps(b, 0, 1, s, std::min(kTmS, p.sample_T - s), par);
+  for (int s = 0; s < p.sample_T && !r; s += kTmS)
+    r = launch_steps(b, 0, 1, s, std::min(kTmS, p.sample_T - s), &par, &pe);
   if (!r) r = flush_block(b, 0, p.sample_T, b->kb.clock);
   if (!r) {
     hipLaunchKernelGGL(k_clock_add, dim3(1), dim3(64), 0, b->stream, b->kb.clock,
@@ -559,12 +577,14 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   double cells = 0;
   for (int d = 0; d < p->n_design; ++d) cells += (double)p->design[d].nx * p->design[d].ny;
   b->rows = tm_pick_rows(cells, p->precision == PM_FP64 ? 8 : 4, b->n_cu);
-  std::vector<KWork> work;
-  build_work(*p, b->rows, work);
+  std::vector<KWork> work, work1;
+  build_work(*p, b->rows, kTmS, work);
+  build_work(*p, 4, 1, work1);
   b->plan = *p;
   b->des.assign(p->design, p->design + p->n_design);
   b->plan.design = b->des.data();
   b->work = std::move(work);
+  b->work1 = std::move(work1);
   char* ws = (char*)p->work;
   std::vector<KDesign> kd(b->des.size());
   char* psi = ws + l.psi;
@@ -577,6 +597,7 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   k.clock = (int64_t*)ws;
   k.des = (const KDesign*)(ws + l.des);
   k.work = (const KWork*)(ws + l.work);
+  k.work1 = (const KWork*)(ws + l.work1);
   k.status = (int32_t*)(ws + l.status);
   k.xcd = b->xcd;
   k.ncols = p->ncols;
@@ -594,6 +615,9 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   if (!r)
     r = bhip(b, hipMemcpyAsync((void*)k.work, b->work.data(), sizeof(KWork) * b->work.size(),
                                hipMemcpyHostToDevice, b->stream), "tile list upload");
+  if (!r)
+    r = bhip(b, hipMemcpyAsync((void*)k.work1, b->work1.data(), sizeof(KWork) * b->work1.size(),
+                               hipMemcpyHostToDevice, b->stream), "tile list upload");
   // status words start clear (an upload, not a memset: nothing here is
   // captured, but the same holds for every buffer a graph reads)
   const std::vector<int32_t> zeros((size_t)p->n_design, 0);
@@ -604,7 +628,7 @@ int pm_batch_configure(pm_batch* b, const pm_batch_plan* p) {
   if (!r) r = bhip(b, hipStreamSynchronize(b->stream), "upload sync");
   if (r) return r;
   b->step = p->table_step0;
-  b->parity = 0;
+  b->parity = b->pe = 0;
   b->pend0 = b->step;
   b->pend_n = 0;
   b->configured = true;
@@ -635,7 +659,8 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
   while (left > 0) {
     if (graphs && b->step % T == 0 && b->pend_n == 0 && left >= T) {
       int r = 0;
-      if (!b->graph[b->parity]) r = capture(b, b->parity);
+      const int slot = b->parity + 2 * b->pe;
+      if (!b->graph[slot]) r = capture(b, slot);
       if (r) return r;
       if (!clock_ok) {
         hipLaunchKernelGGL(k_clock_set, dim3(1), dim3(64), 0, b->stream, b->kb.clock, b->step);
@@ -645,10 +670,13 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
       }
       {
         BSpan sp(b, 2);
-        r = bhip(b, hipGraphLaunch(b->graph[b->parity], b->stream), "graph launch");
+        r = bhip(b, hipGraphLaunch(b->graph[slot], b->stream), "graph launch");
       }
       if (r) return r;
-      b->parity ^= ((T + kTmS - 1) / kTmS) & 1;
+      // (T is even: no launch of the block holds one step)
+      const int odd = ((T + kTmS - 1) / kTmS) & 1;
+      b->parity ^= odd;
+      b->pe ^= odd;
       b->step += T;
       b->pend0 = b->step;
       left -= T;
@@ -660,13 +688,12 @@ int pm_batch_run(pm_batch* b, int32_t nsteps, uint32_t flags) {
     int r;
     {
       BSpan sp(b, 0);
-      r = launch_steps(b, b->step, 0, 0, m, b->parity);
+      r = launch_steps(b, b->step, 0, 0, m, &b->parity, &b->pe);
     }
     if (r) return r;
     if (b->timing) b->timed_steps += m;
     if (b->pend_n == 0) b->pend0 = b->step;
     b->pend_n += m;
-    b->parity ^= 1;
     b->step += m;
     left -= m;
     if (b->step % T == 0) {

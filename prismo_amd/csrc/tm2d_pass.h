@@ -36,8 +36,10 @@ namespace pm {
 
 constexpr int kTmS = 8;                 // steps per pass (halo width)
 constexpr int kTmW = 8;                 // waves per workgroup
-constexpr int kTmCols = 64 - 2 * kTmS;  // columns a tile writes
-__host__ __device__ constexpr int tm_rows(int R) { return kTmW * R - 2 * kTmS; }  // and rows
+// columns and rows a tile with a halo of S cells writes
+__host__ __device__ constexpr int tm_cols(int S) { return 64 - 2 * S; }
+__host__ __device__ constexpr int tm_rows(int R, int S = kTmS) { return kTmW * R - 2 * S; }
+constexpr int kTmCols = tm_cols(kTmS);
 
 template <int CTRL>
 __device__ __forceinline__ int tm_dpp32(int fill, int v) {
@@ -146,7 +148,8 @@ struct TmShared {
   alignas(16) T y[kTmW * R][2][4];
 };
 
-// ns steps of the tile (x0, y0: first column and row it writes) by this wave.
+// ns (at most S) steps of the tile (x0, y0: first column and row it writes) by
+// this wave.
 // yp(k, j): y profile k (be ce ike bh ch ikh) at row j, for one j per lane.
 // io.first() and io.second() issue their own loads before and behind the fields';
 // io.sources(s, ...), io.samples(s, ...) act on the registers after step s.  With
@@ -154,15 +157,15 @@ struct TmShared {
 // (a value that was stays so: it is looked at after the last step).  With
 // IO::kPackedE, where g.full, the E set that is read or the one that is written
 // holds the layers alone (io.packed(false), io.packed(true)).
-template <typename T, int CK, int R, bool XP, bool YP, class YProf, class IO>
+template <typename T, int CK, int R, int S, bool XP, bool YP, class YProf, class IO>
 __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& xp, bool xpml,
                                             const YProf& yp, IO& io, int ns, int x0, int y0,
                                             int w, TmShared<T, R>& sh) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int nx = g.nx, ny = g.ny;
-  const int i = x0 - kTmS + lane;        // this lane's column
-  const int jb = y0 - kTmS + w * R;      // this wave's first row
+  const int i = x0 - S + lane;        // this lane's column
+  const int jb = y0 - S + w * R;      // this wave's first row
   // (without XP every column of the tile is inside the grid, without YP every row)
   const bool lin = !XP || (i >= 0 && i < nx);        // the column exists
   const bool le_ok = !XP || (i >= 0 && i < nx - 1);  // and holds Ez
@@ -302,13 +305,13 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
     io.sources(s, i, js, ez, hx, hy);
     io.samples(s, i, js, ez, hx, hy);
   }
-  const bool mine = lane >= kTmS && lane < 64 - kTmS && lin;
+  const bool mine = lane >= S && lane < 64 - S && lin;
   if (!mine) return 0;
-  if (kTmS % R == 0 && (w * R < kTmS || w * R >= kTmW * R - kTmS)) return 0;  // all halo
+  if (S % R == 0 && (w * R < S || w * R >= kTmW * R - S)) return 0;  // all halo
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int t = w * R + r, j = jb + r;
-    if (kTmS % R != 0 && (t < kTmS || t >= kTmW * R - kTmS)) continue;  // uniform
+    if (S % R != 0 && (t < S || t >= kTmW * R - S)) continue;  // uniform
     if (YP && j >= ny) continue;
     const uint32_t o = (uint32_t)j * g.sy + (uint32_t)i;
     // positions past a component's extent stay 0 in memory (next to an Inf or NaN
@@ -350,17 +353,17 @@ __device__ __forceinline__ uint32_t tm_pass(const TmGrid& g, const TmXProf<T>& x
 // workgroup): XP for tiles that reach an x layer or the grid's first or last
 // column, YP the same in y (an axis without layers then reads element 0 of
 // some array, unused, and stores nothing).
-template <typename T, int CK, int R, class YProf, class IO>
+template <typename T, int CK, int R, int S = kTmS, class YProf, class IO>
 __device__ __forceinline__ uint32_t tm_tile(const TmGrid& g, const TmXProf<T>& xp, bool xpml,
                                             const YProf& yp, IO& io, int ns, int x0, int y0,
                                             int w, TmShared<T, R>& sh) {
-  const bool hasx = x0 - kTmS < g.px0 || x0 - kTmS + 64 > g.nx - max(g.px1, 1);
-  const bool hasy = y0 - kTmS < g.py0 || y0 - kTmS + kTmW * R > g.ny - max(g.py1, 1);
+  const bool hasx = x0 - S < g.px0 || x0 - S + 64 > g.nx - max(g.px1, 1);
+  const bool hasy = y0 - S < g.py0 || y0 - S + kTmW * R > g.ny - max(g.py1, 1);
   if (hasx && hasy)
-    return tm_pass<T, CK, R, true, true>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
-  if (hasx) return tm_pass<T, CK, R, true, false>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
-  if (hasy) return tm_pass<T, CK, R, false, true>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
-  return tm_pass<T, CK, R, false, false>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+    return tm_pass<T, CK, R, S, true, true>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+  if (hasx) return tm_pass<T, CK, R, S, true, false>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+  if (hasy) return tm_pass<T, CK, R, S, false, true>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
+  return tm_pass<T, CK, R, S, false, false>(g, xp, xpml, yp, io, ns, x0, y0, w, sh);
 }
 
 // Workgroup order: groups of 64 of which XCD x takes 8 neighbours, so tiles

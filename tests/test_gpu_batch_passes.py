@@ -59,6 +59,31 @@ def test_tall_tiles(mi355x, storage):
           _run([(33, 81), (1100, 1100)], np.float32, storage, 32, [90], True))
 
 
+@pytest.mark.parametrize("dtype,storage", [(np.float64, "auto"), (np.float32, "auto"),
+                                           (np.float32, "fp16")])
+@pytest.mark.parametrize("runs,graph", [([1] * 101, False), ([1] * 7 + [9, 1, 20, 64], True),
+                                        ([8, 1, 1, 8, 1, 82], True)])
+def test_launches_of_one_step(mi355x, dtype, storage, runs, graph):
+    """A step by itself takes tiles of 62 columns by 30 rows and updates the E-side
+    memory in place; before and after passes of more, graphs from every pair of
+    sets."""
+    sizes = [(46, 44), (47, 45), (109, 17)]  # 62 x 60, 63 x 61 and 125 x 33 cells
+    _same(_run(sizes, dtype, storage, 20, [101], False),
+          _run(sizes, dtype, storage, 20, runs, graph))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("T", [1, 3, 9])
+def test_sample_blocks_that_leave_one_step(mi355x, dtype, T):
+    """Blocks of 1, 3 and 9 rows: passes of 1, 3, and 8 and 1 steps."""
+    a = _run([(46, 44), (33, 17)], dtype, "auto", T, [37], False)
+    b = _run([(46, 44), (33, 17)], dtype, "auto", 64, [37], False)
+    for c in ("Ez", "Hx", "Hy"):
+        assert np.linalg.norm(b[0][c]) > 0 and np.array_equal(a[0][c], b[0][c]), c
+    # (a spectrum is summed block by block: the same samples in another order)
+    assert rel_l2(a[1], b[1]) <= (1e-12 if dtype is np.float64 else 1e-5)
+
+
 @pytest.mark.parametrize("tall", [False, True])
 @pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-10), (np.float32, 1e-5)])
 def test_tile_edges_match_oracle(mi355x, dtype, bar, tall):

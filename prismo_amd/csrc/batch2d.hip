@@ -4,16 +4,16 @@
 // tile of one design (tm2d_pass.h), and a table gives it the design and the
 // tile.  One step per launch moved 300 MB a step for 64 coupler grids of
 // 9.8 M cells together: 68 us at 4.5 TB/s, the rate of a large copy, so only
-// fewer passes over the state could make it faster; eight steps a pass take 146
+// fewer passes over the state could make it faster; eight steps a pass take 148
 // us, 18 a step, two thirds of which the vector ALU is busy (a third of the tiles
 // of a coupler touch a CPML layer).  Reads come from field set `par`, writes go
 // to set par ^ 1, so neighbouring tiles never see a half-updated value; the CPML
 // memory of both field halves is ping-ponged for the same reason.  The plan has
 // one E-side set, which spans the grid; the second, in the workspace, holds the
 // layers alone (28 k values, not 334 k, for 540 x 290 cells with 16 layers a
-// side), and calls begin and end with the state in the plan's.  Sources are added after the E update, samples
-// are taken after the sources, as src/prismo/core/simulation.py:147-164 orders
-// them.
+// side), and calls begin and end with the state in the plan's.  Sources are added
+// after the E update, samples are taken after the sources, as
+// src/prismo/core/simulation.py:147-164 orders them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

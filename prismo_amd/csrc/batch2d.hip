@@ -155,8 +155,9 @@ struct BatchIo {
 
 // S = 8: up to eight steps; S = 1: one step, whose tiles have a halo of one cell
 // (62 columns by 30 rows written of 64 by 32, not 48 by 16) and whose E-side
-// memory is updated in place, as no halo cell's E is used.  par: field set read,
-// pe: E-side memory set read.  Calls of one step (32 designs of 532 x 332 cells):
+// memory is updated in place: its neighbour may have written a halo cell's value
+// before the tile reads it, but that goes into the halo cell's E alone, which a
+// single step does not use.  par: field set read, pe: E-side memory set read.  Calls of one step (32 designs of 532 x 332 cells):
 // with S = 8 46 us FP32, 131 FP64; with S = 1 33 and 82 (one step per launch and
 // no halo: 42 and 84).
 template <typename T, int CK, int R, int S>
